@@ -38,12 +38,16 @@ namespace {
 
 constexpr double kMinPolarizability = 1e-9;   // core/pgm_constants.h:9
 constexpr int kNHist = 5;                     // 4 predictor entries + the slot this step writes
-// Spreading bricks: the larger edge halves the tiles' halo (17^3 vs 13^3 points flushed per 12^3 vs 8^3 owned,
-// 2.8 vs 4.3 atomic additions per grid point at order 6) but makes fewer workgroups; it is used when the engine's
-// grids still give kMinBricks of them (4 per CU), the smaller one otherwise.  Measured: the 64-snapshot batch
-// (~2,400 bricks of 12) 2,184 -> 2,293 snapshot-gradients/s; the 96k box (216 bricks of 12, 729 of 8) keeps 8,
-// its spread being 30% slower with 12.
-constexpr int kBrickSmall = 8, kBrickLarge = 12, kMinBricks = 1024;
+// Bricks of the spread and the gather (chooseBrick): a larger edge means less halo (at order 6, 19^3 points per 14^3
+// owned are 2.5 atomic additions per grid point, 13^3 per 8^3 are 4.3) but fewer workgroups, and a partial brick at the
+// end of a dimension is paid in full.
+constexpr int kBrickSmall = 8, kBrickLarge = 14, kMinBricks = 512;
+constexpr size_t kBrickLds = 80*1024;         // LDS of a spread's tile: two workgroups per CU
+constexpr size_t kPlaneLds = 150*1024;        // dynamic LDS an x-plane block may take (160 KiB less its static arrays)
+// The PME solves run beside the pair passes only from this size on, unless the autotuner or the caller says so: below
+// it a solve is a chain of launches of a few us each, and the two streams' waits for each other cost more than the
+// overlap gains (1,536 atoms 700 us per step beside, 590 in line; 24,000 atoms 712 and 725; 98,000 1,335 and 1,545).
+constexpr int kOverlapAtoms = 16384;
 constexpr int kChunkAtoms = 2048;             // rows per first-stage block of the per-system sums
 
 void hipCheck(hipError_t e, const char* what) {
@@ -1092,13 +1096,14 @@ public:
         const bool f32 = sizeof(T) == sizeof(float);
         launchFieldOperands<T>(st_, n, orderD_.as<int>(), fqD_.as<double>(), fdD_.as<double>(), rgT<T>(),
                                posDD_.as<double4>(), f32 ? posT<T>() : nullptr, permD_.as<double>(), permTD_.as<T4>());
-        for (DevBuf* b : {&edD_, &erD_, &bD_, &tdD_})
+        for (DevBuf* b : {&edD_, &bD_, &tdD_})
             b->reserve(3*sizeof(double)*n);
+        erD_.reserve(recBytes());
         nbD_.reserve(n*sizeof(int));
         pairSetup<T>(setupLanes(), fused_, nullptr);
         pmeSolve<T>(permTD_.as<T4>(), true, posT<T>(), 0, false, erD_.as<double>(), nullptr, nullptr, nullptr);
         const double cself = 4.0*s_.beta*s_.beta*s_.beta/(3.0*kSqrtPi);
-        launchCombineB(st_, n, edD_.as<double>(), erD_.as<double>(), permD_.as<double>(), cself, bD_.as<double>());
+        launchCombineB(st_, n, edD_.as<double>(), recField(erD_), permD_.as<double>(), cself, bD_.as<double>());
         tmpD_.reserve(3*sizeof(double)*n);
         launchUnsort3(st_, n, rankD_.as<int>(), bD_.as<double>(), tmpD_.as<double>());
         HIPCHK(hipMemcpyAsync(out, tmpD_.p, 3*sizeof(double)*n, hipMemcpyDeviceToHost, st_));
@@ -1277,11 +1282,15 @@ public:
             for (int o = 0; o < 2; o++)
                 overlapMs_[o] = mixed ? timeProduct<float>(o == 1, reps) : timeProduct<double>(o == 1, reps);
             pmeOverlap_ = overlapMs_[1] <= overlapMs_[0];
+            overlapChosen_ = true;
         });
         return best;
     }
     bool pmeOverlap() const { return pmeOverlap_; }
-    void setPmeOverlap(bool on) { pmeOverlap_ = on; }
+    void setPmeOverlap(bool on) {
+        pmeOverlap_ = on;
+        overlapChosen_ = true;
+    }
     const double* overlapTimes() const { return overlapMs_; }
     bool fieldOtf() const { return fieldOtf_; }
     void setFieldOtf(bool on) {
@@ -1441,6 +1450,7 @@ private:
     // the device's PME stream, shared by its engines (acquirePmeStream)
     hipStream_t st2_ = nullptr, pmeSt_ = nullptr;
     bool pmeOverlap_ = true;              // PME on st2_ beside the pair passes (the autotuner measures it)
+    bool overlapChosen_ = false;          // ... as the caller or the autotuner chose, else only from kOverlapAtoms on
     double overlapMs_[2] = {0.0, 0.0};    // the autotuner's CG product: PME after, beside the field pass
     hipEvent_t evFork_ = nullptr, evJoin_ = nullptr;
     int n_ = 0, nGlobal_ = 0, covN_ = -1, covBuiltN_ = -1;   // covBuiltN_: the atom count of the covalent CSR
@@ -1569,7 +1579,7 @@ private:
     DevBuf qSD_, rgSD_, alphaSD_, posDD_, posFD_;
     DevBuf permD_, permTD_, edD_, erD_, bD_, xD_, rD_, zD_, pD_, apD_, tdD_, trD_, pTD_, dD_, dTD_, etotD_;
     DevBuf fpairD_, frecD_, fcovD_, forcesOutD_, tmpD_;
-    DevBuf brickOfD_, pslotD_, brickCountD_, brickStartD_, pmeAtomD_, baseD_, splD_;
+    DevBuf brickOfD_, pslotD_, brickCountD_, brickStartD_, pmeAtomD_;
     DevBuf fqD_, fdD_;   // the charges and dipoles of a field evaluation (caller's order)
     DevBuf gridD_, gridFixedD_, cplxD_, inflD_, twD_, bmodD_;
     const long long* fixedClean_ = nullptr;   // gridFixedD_ as last left all zero, over fixedCleanWords_ words
@@ -1577,6 +1587,7 @@ private:
     DevBuf cgPartD_, partD_, resD_, cgD_, doneD_, histD_, maxBitsD_;
     DevBuf perAtomD_, chunkSumD_;
     DevBuf fftGroupsD_;     // the merged transform launches' group table
+    DevBuf blockGroupD_[4];   // and the group of every block of the z, y, x and fused z+y launches
     FftLaunch fftL_{};
     // systems tables (batch)
     DevBuf sysOfD_, boxTabD_, boxTabFD_, pmeTabD_, brickSysD_, groupBoxD_, chunkStartD_, sysChunkD_;
@@ -1793,29 +1804,70 @@ private:
             uploadBoxTables();
     }
 
+    // Whether the PME solves run as x-plane passes (kPlaneSpread, kFftXConv, kPlaneGather): three launches a solve in
+    // place of seven, no fixed-point grid and no potentials in memory, but only as many workgroups as x-planes.  With
+    // 512 planes or more (a batch) the chip is full: the 64-snapshot batch 17.6 -> 16.8 ms.  With fewer, as long as a
+    // plane's atoms do not outweigh the launches saved: in mixed precision 1,536 atoms on 32^3 (288 atom rows per
+    // plane) 712 -> 600 us, 24,000 on 70^3 (2,057) 730 -> 685, 96,000 on 72^3 (8,000) 2,020 -> 2,600; in FP64 30,000
+    // on 75 x 80 x 72 (2,400) 1,370 -> 1,398.
+    bool planePath() const {
+        size_t lds = 0;
+        long long planes = 0;
+        for (const Sys& y : sys_) {
+            FftGroup f{};
+            for (int a = 0; a < 3; a++)
+                f.g.K[a] = y.grid[a];
+            f.g.K3h = y.grid[2]/2+1;
+            f.ngrid = 1;
+            int b[4];
+            size_t l[5];
+            s_.precision == PGM_MIXED ? fftGroupShape<float>(f, false, b, l) : fftGroupShape<double>(f, false, b, l);
+            lds = std::max({lds, l[3], l[4]});
+            planes += y.grid[0];
+        }
+        if (lds > kPlaneLds)
+            return false;
+        const long long most = s_.precision == PGM_MIXED ? 2200 : 1500;   // atom rows per plane
+        return planes >= kManyPlanes || (long long) n_*s_.order <= most*planes;
+    }
+    static constexpr int kManyPlanes = 512;
+    // The brick edge with the fewest tile points (each a global addition in the spread and a load in the gather) that
+    // still makes kMinBricks workgroups, keeps a tile within kBrickLds and wraps into every grid once; the small one
+    // where none does.  72^3: 9, 112^3: 14 (spread 45 -> 37 us, gather 27 -> 19 us a solve), 216^3: 14.
+    int chooseBrick() const {
+        int best = kBrickSmall;
+        double bestPoints = 0;
+        for (int e = kBrickSmall; e <= kBrickLarge; e++) {
+            double bricks = 0, points = 0;
+            const double edge = e+s_.order-1;
+            bool ok = edge*edge*edge*sizeof(long long)*(s_.precision == PGM_MIXED ? 1 : 2) <= (double) kBrickLds;
+            for (const Sys& y : sys_) {
+                double nb = 1;
+                for (int a = 0; a < 3; a++) {
+                    nb *= (y.grid[a]+e-1)/e;
+                    ok = ok && y.grid[a] >= e;
+                }
+                bricks += nb;
+                points += nb*edge*edge*edge;
+            }
+            if (e == kBrickSmall || (ok && bricks >= kMinBricks && points < bestPoints)) {
+                best = e;
+                bestPoints = points;
+            }
+        }
+        return best;
+    }
+
     // Grid shapes -> transform groups; offsets of every system's grids, bricks and cells; the batch tables.
     void buildLayout() {
         groups_.clear();
-        long long largeBricks = 0;
-        bool gridsFit = true;   // the spread wraps a tile row into the grid once: every dimension >= the brick
-        for (const Sys& y : sys_) {
-            largeBricks += (long long) ((y.grid[0]+kBrickLarge-1)/kBrickLarge)*((y.grid[1]+kBrickLarge-1)/kBrickLarge)*
-                           ((y.grid[2]+kBrickLarge-1)/kBrickLarge);
-            for (int a = 0; a < 3; a++)
-                gridsFit = gridsFit && y.grid[a] >= kBrickLarge;
-        }
-        const long long tileEdge = kBrickLarge+s_.order-1;
-        const long long tileLarge = tileEdge*tileEdge*tileEdge;
-        // the spread's LDS tile holds 8 bytes per point and grid word (one word in FP32, two in FP64: 77 KiB at
-        // order 6, within the 160 KiB of LDS a gfx950 workgroup may take); higher orders keep the small brick
-        const bool largeFits = tileLarge*(long long) sizeof(double) <= 64*1024;
-        brick_ = (largeFits && gridsFit && largeBricks >= kMinBricks) ? kBrickLarge : kBrickSmall;
+        const bool plane = planePath();
+        brick_ = plane ? kBrickSmall : chooseBrick();
         for (size_t s = 0; s < sys_.size(); s++) {
             Sys& y = sys_[s];
             PmeGrid g{};
             for (int a = 0; a < 3; a++) {
                 g.K[a] = y.grid[a];
-                g.plan[a] = makePlan(g.K[a]);
                 g.nb[a] = (g.K[a]+brick_-1)/brick_;
             }
             g.K3h = g.K[2]/2+1;
@@ -1866,7 +1918,13 @@ private:
         }
         // the merged transform launches: every group's share of each stage
         std::vector<FftGroup> fg;
+        std::vector<unsigned short> blockGroup[4];
+        if (groups_.size() > 65535)
+            throw std::invalid_argument("pgm_hip: more than 65535 PME grid shapes");
         fftL_ = FftLaunch{};
+        // (the wide radices pay where a launch fills the chip: 216^3 1,660 -> 1,500 us per evaluation, 112^3 and 72^3 5% slower)
+        const bool wide = realTotal_ >= 4000000;
+        fftL_.wide = wide ? 1 : 0;
         int boxOff = 0;
         for (Group& G : groups_) {
             FftGroup f{};
@@ -1878,26 +1936,36 @@ private:
             f.partOff = G.partOff;
             f.boxOff = boxOff;
             int b[4];
-            size_t l[4];
+            size_t l[5];
             if (mixed)
-                fftGroupShape<float>(f, b, l);
+                fftGroupShape<float>(f, wide, b, l);
             else
-                fftGroupShape<double>(f, b, l);
+                fftGroupShape<double>(f, wide, b, l);
             for (int k = 0; k < 4; k++) {
                 f.blk0[k] = fftL_.blocks[k];
                 fftL_.blocks[k] += b[k];
-                fftL_.lds[k] = std::max(fftL_.lds[k], l[k]);
+                blockGroup[k].insert(blockGroup[k].end(), b[k], (unsigned short) fg.size());
             }
+            for (int k = 0; k < 5; k++)
+                fftL_.lds[k] = std::max(fftL_.lds[k], l[k]);
             if (b[2] != G.blocksPerGrid*f.ngrid)
                 throw std::logic_error("pgm_hip: transform block counts disagree");
             boxOff += f.ngrid;
             fg.push_back(f);
         }
         // z and y fused when the x-planes alone give enough blocks (many small grids) and a plane fits the LDS
-        fftL_.zyFused = (fftL_.blocks[3] >= 512 && fftL_.lds[3] <= 48*1024) ? 1 : 0;
+        fftL_.plane = plane ? 1 : 0;
+        fftL_.zyFused = (plane || (fftL_.blocks[3] >= 512 && fftL_.lds[3] <= 48*1024)) ? 1 : 0;
+        // (few planes: as many wavefronts per plane as a workgroup holds; many: several workgroups per CU)
+        fftL_.planeThreads = plane && fftL_.blocks[3] < kManyPlanes ? 1024 : 256;
         upload(fftGroupsD_, fg.data(), fg.size()*sizeof(FftGroup));
         fftL_.groups = fftGroupsD_.as<FftGroup>();
         fftL_.ngroups = (int) fg.size();
+        if (fg.size() > 1)
+            for (int k = 0; k < 4; k++) {
+                upload(blockGroupD_[k], blockGroup[k].data(), blockGroup[k].size()*sizeof(unsigned short));
+                fftL_.blockGroup[k] = blockGroupD_[k].as<unsigned short>();
+            }
         brickTotal_ = 0;
         for (Sys& y : sys_) {
             y.brickOff = brickTotal_;
@@ -1906,8 +1974,9 @@ private:
         // device arrays of the layout
         const size_t tsz = mixed ? sizeof(float) : sizeof(double), t2 = 2*tsz;
         gridD_.reserve((size_t) realTotal_*tsz);
-        gridFixedD_.reserve((size_t) realTotal_*sizeof(long long)*(s_.precision == PGM_MIXED ? 1 : 2));
-        cplxD_.reserve((size_t) cplxTotal_*t2);
+        if (!plane)   // the x-plane spread accumulates in LDS
+            gridFixedD_.reserve((size_t) realTotal_*sizeof(long long)*(s_.precision == PGM_MIXED ? 1 : 2));
+        cplxD_.reserve((size_t) cplxTotal_*t2*(plane ? 2 : 1));   // (two solves at once)
         inflD_.reserve((size_t) cplxTotal_*tsz);
         twD_.reserve((size_t) twTotal_*t2);
         std::vector<double> bm;
@@ -2016,9 +2085,13 @@ private:
         p.table = batch_ ? pmeTabD_.as<PmeSys>() : nullptr;
         p.sysOf = batch_ ? sysOfD_.as<int>() : nullptr;
         p.brickSys = batch_ ? brickSysD_.as<int>() : nullptr;
+        p.groupSys = batch_ ? recSysD_.as<int>() : nullptr;
         p.nbrick = brickTotal_;
         p.order = s_.order;
         p.brick = brick_;
+        // (every lane evaluates its atom's splines, so few lanes per atom where a brick's atoms fill the workgroup:
+        // 96,000 atoms on 512 bricks 2,010 us an evaluation at 2, 2,070 at 4; 30,000 on 900 1,396 and 1,370)
+        p.atomLanes = n_ >= 64LL*brickTotal_ ? 2 : 4;
         p.fixedStride = (size_t) realTotal_;
         return p;
     }
@@ -2283,7 +2356,7 @@ private:
     // PME beside the pair passes unless PME phases are being timed (their brackets are on the engine stream).
     bool overlapPme() const {
         constexpr unsigned pmeMask = (1u << kPhSpread) | (1u << kPhFft) | (1u << kPhGather);
-        return pmeOverlap_ && !(timing_ && (phaseMask_ & pmeMask));
+        return pmeOverlap_ && (overlapChosen_ || n_ >= kOverlapAtoms) && !(timing_ && (phaseMask_ & pmeMask));
     }
     // The PME stream of one evaluation, back to the engine stream when the scope ends (also on an error).
     struct PmeStreamScope {
@@ -2306,11 +2379,60 @@ private:
     }
 
     template<class T>
+    void convolve(T* grid, int energyMode, bool strain, const int* skip, long long* fixed, int stages, int nsolve) {
+        typedef typename Vec2<T>::type T2;
+        const BoxT<double> one = makeBox<double>(sys_[0].H, sys_[0].recip);
+        launchPmeConvolve<T>(pmeSt_, fftL_, grid, cplxD_.as<T2>(), inflD_.as<T>(), twD_.as<T2>(), one,
+                             batch_ ? groupBoxD_.as<BoxT<double>>() : nullptr, s_.beta, energyMode, strain ? 1 : 0,
+                             partD_.as<double>(), skip, fixed, (size_t) realTotal_, stages, nsolve,
+                             (size_t) cplxTotal_);
+    }
+    // The x-plane passes (fftL_.plane): the densities of the solves spread and transformed in z and y.
+    template<class T>
+    void planeSpread(PlaneSolves<T>& solves, const int* skip, int it) {
+        typedef typename Vec2<T>::type T2;
+        solves.cplxStride = (size_t) cplxTotal_;
+        tb(kPhSpread, it);
+        launchPlaneSpread<T>(pmeSt_, fftL_, pmeSel(), brickStartD_.as<int>(), pmeAtomD_.as<PmeAtom<T>>(),
+                             posT<T>(), solves, cplxD_.as<T2>(), twD_.as<T2>(), skip);
+        te();
+    }
+    // ... and whole solves: spread, convolution, the fields gathered.
+    template<class T>
+    void planeSolve(PlaneSolves<T> solves, const int* skip, int it = -1) {
+        typedef typename Vec2<T>::type T2;
+        planeSpread<T>(solves, skip, it);
+        tb(kPhFft, it);
+        convolve<T>(nullptr, 0, false, skip, nullptr, 0, solves.n);
+        te();
+        tb(kPhGather, it);
+        launchPlaneGather<T>(pmeSt_, fftL_, pmeSel(), brickStartD_.as<int>(), pmeAtomD_.as<PmeAtom<T>>(),
+                             solves, cplxD_.as<T2>(), twD_.as<T2>(), skip);
+        te();
+    }
+    // A solve's field as its readers take it, and the bytes it needs.
+    RecField recField(const DevBuf& b) const { return RecField{b.as<double>(), fftL_.plane ? s_.order : 1}; }
+    size_t recBytes() const { return 3*sizeof(double)*n_*(size_t) (fftL_.plane ? s_.order : 1); }
+
+    template<class T>
     void pmeGrids(const typename Vec4<T>::type* dip, bool withQ, const typename Vec4<T>::type* posq, int energyMode,
                   bool strain, T* grid, const int* skip, double* res, int it,
                   const typename Vec4<T>::type* dipDot = nullptr, const typename Vec4<T>::type* disp = nullptr) {
-        typedef typename Vec2<T>::type T2;
         const PmeSel ps = pmeSel();
+        if (fftL_.plane && !dipDot) {   // spread into the x-planes, the potentials to grid
+            PlaneSolves<T> one{};
+            one.n = 1;
+            one.dip[0] = dip;
+            one.withQ[0] = withQ ? 1 : 0;
+            planeSpread<T>(one, skip, it);
+            tb(kPhFft, it);
+            convolve<T>(grid, energyMode, strain, skip, nullptr, kFftInverse, 1);
+            if (energyMode)
+                launchRangeSums(pmeSt_, partD_.as<double>(), 10, recStartD_.as<int>(), nRecRanges_,
+                                recSysD_.as<int>(), kResCount, res+kResRec);
+            te();
+            return;
+        }
         // the charge/dipole grids through the fixed-point accumulator (order-independent), a tangent density
         // (dipDot) straight into grid
         long long* fixed = dipDot ? nullptr : gridFixedD_.as<long long>();
@@ -2325,14 +2447,11 @@ private:
         }
         else
             launchZero<T>(pmeSt_, grid, (size_t) realTotal_, skip);
-        launchSpread<T>(pmeSt_, ps, brickStartD_.as<int>(), pmeAtomD_.as<int>(), baseD_.as<int>(), splD_.as<T>(), dip,
+        launchSpread<T>(pmeSt_, ps, brickStartD_.as<int>(), pmeAtomD_.as<PmeAtom<T>>(), dip,
                         posq, withQ ? 1 : 0, grid, fixed, skip, dipDot, disp);
         te();
         tb(kPhFft, it);
-        const BoxT<double> one = makeBox<double>(sys_[0].H, sys_[0].recip);
-        launchPmeConvolve<T>(pmeSt_, fftL_, grid, cplxD_.as<T2>(), inflD_.as<T>(), twD_.as<T2>(), one,
-                             batch_ ? groupBoxD_.as<BoxT<double>>() : nullptr, s_.beta, energyMode, strain ? 1 : 0,
-                             partD_.as<double>(), skip, fixed, (size_t) realTotal_);
+        convolve<T>(grid, energyMode, strain, skip, fixed, kFftForward | kFftInverse, 1);
         if (fixed) {   // enqueued: the spread's words are read and zeroed before anything else uses the grid
             fixedClean_ = fixed;
             fixedCleanWords_ = fixedWords;
@@ -2346,9 +2465,18 @@ private:
     template<class T>
     void pmeSolve(const typename Vec4<T>::type* dip, bool withQ, const typename Vec4<T>::type* posq, int energyMode,
                   bool strain, double* field, double* force, const int* skip, double* res, int it = -1) {
+        if (fftL_.plane && !force) {
+            PlaneSolves<T> one{};
+            one.n = 1;
+            one.dip[0] = dip;
+            one.withQ[0] = withQ ? 1 : 0;
+            one.out[0] = field;
+            planeSolve<T>(one, skip, it);
+            return;
+        }
         pmeGrids<T>(dip, withQ, posq, energyMode, strain, gridD_.as<T>(), skip, res, it);
         tb(kPhGather, it);
-        launchGather<T>(pmeSt_, pmeSel(), n_, pmeAtomD_.as<int>(), baseD_.as<int>(), splD_.as<T>(), gridD_.as<T>(), dip,
+        launchGather<T>(pmeSt_, pmeSel(), brickStartD_.as<int>(), pmeAtomD_.as<PmeAtom<T>>(), gridD_.as<T>(), dip,
                         posq, force ? 1 : 0, field, force, skip);
         te();
     }
@@ -2387,7 +2515,7 @@ private:
                                  doneD_.as<int>(), rgT<T>());
         };
         tb(kPhCg);
-        launchCgInit<T>(st_, n, alphaSD_.as<double>(), b, x, tdD_.as<double>(), trD_.as<double>(), cself, s_.tol,
+        launchCgInit<T>(st_, n, alphaSD_.as<double>(), b, x, tdD_.as<double>(), recField(trD_), cself, s_.tol,
                         s_.max_iter, rD_.as<double>(), zD_.as<double>(), pD_.as<double>(), pTD_.as<T4>(),
                         cgPartD_.as<double>(), cgD_.as<CgState>(), doneD_.as<int>(), pc, rgT<T>());
         precond(0, true);
@@ -2440,7 +2568,7 @@ private:
         const int* skip = doneD_.as<int>()+it;
         matvec<T>(posT, pTD_.as<T4>(), skip, it);
         tb(kPhCg, it);
-        launchCgAp(st_, n, it, alphaSD_.as<double>(), pD_.as<double>(), tdD_.as<double>(), trD_.as<double>(), cself,
+        launchCgAp(st_, n, it, alphaSD_.as<double>(), pD_.as<double>(), tdD_.as<double>(), recField(trD_), cself,
                    apD_.as<double>(), cgPartD_.as<double>(), doneD_.as<int>());
         launchCgUpdate(st_, n, it, alphaSD_.as<double>(), pD_.as<double>(), apD_.as<double>(), x, rD_.as<double>(),
                        zD_.as<double>(), cgPartD_.as<double>(), doneD_.as<int>(), pc);
@@ -2560,9 +2688,7 @@ private:
         pslotD_.reserve(n*sizeof(int));
         brickCountD_.reserve((brickTotal_+1)*sizeof(int));
         brickStartD_.reserve((brickTotal_+1)*sizeof(int));
-        pmeAtomD_.reserve(n*sizeof(int));
-        baseD_.reserve(3*n*sizeof(int));
-        splD_.reserve((size_t) n*9*s_.order*sizeof(T));
+        pmeAtomD_.reserve(n*sizeof(PmeAtom<T>));
         resD_.reserve(sys_.size()*kResCount*sizeof(double));
         maxBitsD_.reserve(2*sizeof(unsigned));
         tb(kPhPrep);
@@ -2600,7 +2726,7 @@ private:
         launchScan(st_, brickCountD_.as<int>(), brickStartD_.as<int>(), brickTotal_,
                    scanScratch(brickScanD_, brickTotal_));
         launchPmePlace<T>(st_, n, posDD_.as<double4>(), ps, brickOfD_.as<int>(), pslotD_.as<int>(),
-                          brickStartD_.as<int>(), pmeAtomD_.as<int>(), baseD_.as<int>(), splD_.as<T>());
+                          brickStartD_.as<int>(), pmeAtomD_.as<PmeAtom<T>>());
         te();
     }
 
@@ -2614,9 +2740,11 @@ private:
         const BoxSel<T> bt = boxSel<T>();
         const double cself = 4.0*s_.beta*s_.beta*s_.beta/(3.0*kSqrtPi);
         // per-atom buffers
-        for (DevBuf* b : {&permD_, &edD_, &erD_, &bD_, &xD_, &rD_, &zD_, &pD_, &apD_, &tdD_, &trD_, &dD_, &etotD_,
-                          &fpairD_, &frecD_, &fcovD_})
+        for (DevBuf* b : {&permD_, &edD_, &bD_, &xD_, &rD_, &zD_, &pD_, &apD_, &tdD_, &dD_, &etotD_, &fpairD_,
+                          &frecD_, &fcovD_})
             b->reserve(v3);
+        for (DevBuf* b : {&erD_, &trD_})
+            b->reserve(recBytes());
         for (DevBuf* b : {&permTD_, &pTD_, &dTD_})
             b->reserve(n*sizeof(T4));
         perAtomD_.reserve((size_t) n*11*sizeof(double));
@@ -2659,11 +2787,17 @@ private:
             te();
             preReady_ = true;
         }
-        pmeSolve<T>(permTD_.as<T4>(), true, pos, 0, false, erD_.as<double>(), nullptr, nullptr, nullptr);
-        if (dual)   // the guess's reciprocal field (its direct field rides on the setup pass)
-            pmeSolve<T>(pTD_.as<T4>(), false, pos, 0, false, trD_.as<double>(), nullptr, nullptr, nullptr);
+        // (the guess's reciprocal field too: its direct field rides on the setup pass)
+        if (dual && fftL_.plane)
+            planeSolve<T>(PlaneSolves<T>{2, {permTD_.as<T4>(), pTD_.as<T4>()}, {1, 0},
+                                         {erD_.as<double>(), trD_.as<double>()}, 0}, nullptr);
+        else {
+            pmeSolve<T>(permTD_.as<T4>(), true, pos, 0, false, erD_.as<double>(), nullptr, nullptr, nullptr);
+            if (dual)
+                pmeSolve<T>(pTD_.as<T4>(), false, pos, 0, false, trD_.as<double>(), nullptr, nullptr, nullptr);
+        }
         join();
-        launchCombineB(st_, n, edD_.as<double>(), erD_.as<double>(), permD_.as<double>(), cself, bD_.as<double>());
+        launchCombineB(st_, n, edD_.as<double>(), recField(erD_), permD_.as<double>(), cself, bD_.as<double>());
         // induced dipoles
         int pushSlot = -1;
         if (induce) {
@@ -2860,7 +2994,7 @@ private:
             if (ddT)
                 pmeGrids<T>(dTD_.as<T4>(), true, pos, 0, false, gridTD_.as<T>(), nullptr, nullptr, -1, ddT,
                             gTD_.as<T4>());
-            launchGatherTangent<T>(pmeSt_, pmeSel(), n, pmeAtomD_.as<int>(), baseD_.as<int>(), splD_.as<T>(),
+            launchGatherTangent<T>(pmeSt_, pmeSel(), n, brickStartD_.as<int>(), pmeAtomD_.as<PmeAtom<T>>(),
                                    gridD_.as<T>(), ddT ? gridTD_.as<T>() : nullptr, ddT ? gTD_.as<T4>() : nullptr,
                                    pmeOutD_.as<double>());
             join();

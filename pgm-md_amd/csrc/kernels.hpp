@@ -223,23 +223,30 @@ void launchPairTangent(hipStream_t st, int n, const typename Vec4<T>::type* pos,
 
 // a / d for 0 <= a < 2^20 and 1 <= d < 2^12 by one multiply: floor(a * ceil(2^32 / d) / 2^32) is exact there
 // (the rounding of the reciprocal contributes a * (ceil - 2^32/d) / 2^32 < a * d / 2^32 < 1/d).  Replaces the
-// ~20-instruction integer divisions of the FFT index arithmetic.
+// ~20-instruction integer divisions of the FFT index arithmetic.  magic 0: d = 1.
 struct FastDiv {
-    unsigned long long magic;
+    unsigned magic;
     __host__ __device__ __forceinline__ int div(int a) const {
-        return (int) (((unsigned long long) (unsigned) a*magic) >> 32);
+        return magic ? (int) (((unsigned long long) (unsigned) a*magic) >> 32) : a;
     }
 };
-inline FastDiv fastDiv(int d) { return FastDiv{((1ull << 32)+(unsigned long long) d-1)/(unsigned long long) d}; }
+inline FastDiv fastDiv(int d) {
+    return FastDiv{d == 1 ? 0u : (unsigned) (((1ull << 32)+(unsigned long long) d-1)/(unsigned long long) d)};
+}
 
-// Stages of a mixed-radix FFT of length K; for each stage the divisions by m = K/R and by Ns = R_0...R_{s-1}.
+// Stages of a mixed-radix FFT; for each the divisions by m = K/R and by Ns = R_0...R_{s-1}.
 struct FftPlan {
-    int K;
+    struct Stage {
+        int radix;
+        FastDiv byM, byNs;
+    };
     int nstage;
-    int radix[10];
-    FastDiv byM[10], byNs[10];
+    int pad;
+    Stage stage[10];
 };
-FftPlan makePlan(int K);
+constexpr int kPlanInts = sizeof(FftPlan)/sizeof(int);
+// wide: radices 2..10 (the fewest stages), else 2, 3, 4, 5, 7.  Throws for a length with other prime factors.
+FftPlan makePlan(int K, bool wide = false);
 
 struct PmeGrid {
     int K[3];
@@ -248,7 +255,6 @@ struct PmeGrid {
     int brick;     // edge of the spreading bricks in grid points
     int nb[3];     // bricks per dimension
     int nbrick;
-    FftPlan plan[3];
 };
 
 // One system's PME grid in a batch: its grid, box, the offset of its real grid and its first global brick.
@@ -266,24 +272,36 @@ struct PmeSel {
     const PmeSys* table;    // batch: per system; nullptr: a single system
     const int* sysOf;       // batch: system of every (sorted) atom index
     const int* brickSys;    // batch: system of every global brick
+    const int* groupSys;    // batch: system of every stacked grid, group after group
     int nbrick;             // bricks of all systems
     int order;
     int brick;
+    FastDiv byTile;         // (the gather's) division by its tile's edge
+    int atomLanes;          // lanes per atom of the spread and the gather over bricks: 2 (full bricks) or 8
     size_t fixedStride;     // FP64 fixed-point grids: the second words' offset (the stacked real grids' size)
 };
 
-// Binning of the sorted atoms into spreading bricks and their spline weights, in brick order.
+// An atom of the PME passes, in brick order: its base grid point, its (sorted) index and its fractions of a grid
+// cell, from which a pass evaluates the spline weights it needs (bsplines).  32 or 48 bytes in place of a table of 9 P
+// weights per atom (216 or 432 bytes at order 6), whose lines were what the spread and the gather waited for.
+template<class T>
+struct __align__(16) PmeAtom {
+    int base[3];
+    int s;
+    T fr[4];   // (the last unused)
+};
+// Binning of the sorted atoms into spreading bricks, and their records in brick order.
 template<class T>
 void launchPmeBin(hipStream_t st, int n, const double4* posD, PmeSel ps, int* brickOf, int* slot, int* brickCount);
 template<class T>
 void launchPmePlace(hipStream_t st, int n, const double4* posD, PmeSel ps, const int* brickOf, const int* slot,
-                    const int* brickStart, int* pmeAtom, int* base, T* spl);
+                    const int* brickStart, PmeAtom<T>* atoms);
 // Spread charges (withQ) and dipoles of the sorted atoms onto the fixed-point grids fixed (GridFixed<T>::words
 // words per point, the second words of all points after the first words of all points; zeroed by the caller;
 // order-independent) or, with dipDot, the change of that density for displacements disp and dipole changes dipDot
 // onto the real grids grid (zeroed by the caller).
 template<class T>
-void launchSpread(hipStream_t st, PmeSel ps, const int* brickStart, const int* pmeAtom, const int* base, const T* spl,
+void launchSpread(hipStream_t st, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms,
                   const typename Vec4<T>::type* dip, const typename Vec4<T>::type* posq, int withQ, T* grid,
                   long long* fixed, const int* skip, const typename Vec4<T>::type* dipDot = nullptr,
                   const typename Vec4<T>::type* disp = nullptr);
@@ -313,6 +331,29 @@ __device__ __forceinline__ void toFixed(T v, long long& hi, long long& lo) {
     else
         lo = 0;
 }
+// toFixed for |v| < fixedLimit<T>() without the 64-bit conversions (about ten FP64 instructions each): adding
+// 1.5 2^k puts the last place of the sum at the fixed-point unit, so the sum's bits less the constant's are the
+// value rounded to nearest even, the same integer as toFixed gives.  FP32: k = 20 (unit 2^-32); FP64: k = 28 for
+// the first word (2^-24), the exact remainder with k = -4 for the second (2^-56).
+template<class T>
+__host__ __device__ constexpr T fixedLimit() {
+    return sizeof(T) == sizeof(float) ? T(1 << 18) : T(1 << 26);
+}
+template<class T>
+__device__ __forceinline__ void toFixedFast(T v, long long& hi, long long& lo) {
+    if constexpr (GridFixed<T>::words == 2) {
+        constexpr double m1 = 402653184.0, m2 = 0.09375;
+        const double d = v+m1;
+        hi = __double_as_longlong(d)-__double_as_longlong(m1);
+        const double e = (v-(d-m1))+m2;
+        lo = __double_as_longlong(e)-__double_as_longlong(m2);
+    }
+    else {
+        constexpr double m = 1572864.0;
+        hi = __double_as_longlong((double) v+m)-__double_as_longlong(m);
+        lo = 0;
+    }
+}
 // The value of a point whose words are at p[0] and (FP64) p[stride].
 template<class T>
 __device__ __forceinline__ T fromFixed(const long long* p, size_t stride) {
@@ -332,7 +373,7 @@ __device__ __forceinline__ T takeFixed(long long* p, size_t stride) {
 }
 
 // One grid shape's share of a merged transform launch: every shape of a batch goes through each stage (z, y,
-// x + convolution, y, z) in one launch; a block finds its shape by its block index.
+// x + convolution, y, z) in one launch.
 struct FftGroup {
     PmeGrid g;
     int ngrid;                   // stacked grids of this shape
@@ -342,17 +383,25 @@ struct FftGroup {
     int boxOff;                  // its first system's box in the batch box table
     int pz, zy, zx;              // lines per block of the z, y and x stages
     int blk0[4];                 // its first block in the z, y, x and fused z+y launches
+    FastDiv byK2, byKh, byZy, byZx;
+    FftPlan plan[3];             // the transforms along x, y and z
 };
 struct FftLaunch {
     const FftGroup* groups;      // device table
     int ngroups;
+    const unsigned short* blockGroup[4];   // the group of every block of the four launches (nullptr: one group)
     int blocks[4];               // z, y, x and fused z+y launch sizes
-    size_t lds[4];               // dynamic LDS of those stages (the largest shape's)
+    size_t lds[5];               // dynamic LDS of those stages and the x-plane spread (the largest shape's)
+    int wide;                    // the plans' radices (makePlan)
     int zyFused;                 // z and y in one pass per x-plane (many small grids), else apart
+    int plane;                   // spread and gather in the x-plane passes too (kPlaneSpread, kPlaneGather)
+    int planeThreads;            // threads per block of the x-plane passes
 };
 // The shape of group g's stages (lines per block) and its blocks per stage, as the transforms use them.
 template<class T>
-void fftGroupShape(FftGroup& G, int blocks[4], size_t lds[4]);
+void fftGroupShape(FftGroup& G, bool wide, int blocks[4], size_t lds[5]);
+// The z and y transforms a convolution includes beside its x pass.
+enum { kFftForward = 1, kFftInverse = 2 };
 // Forward transforms, influence function (energy and strain partials when asked), inverse transforms of all
 // grids of all groups; real: the stacked real grids, cplx/influence/tw: the stacked complex arrays.  boxes: per
 // stacked grid (nullptr: box for all).  partials: [.][10] (energy, strain 0..8) per x block, the blocks of a
@@ -363,19 +412,41 @@ template<class T>
 void launchPmeConvolve(hipStream_t st, const FftLaunch& L, T* real, typename Vec2<T>::type* cplx, const T* influence,
                        const typename Vec2<T>::type* tw, BoxT<double> box, const BoxT<double>* boxes, double beta,
                        int energy, int strain, double* partials, const int* skip, long long* fixed,
-                       size_t fixedStride);
+                       size_t fixedStride, int stages = kFftForward | kFftInverse, int nsolve = 1,
+                       size_t cplxStride = 0);
+// The solves an x-plane launch runs at once: dipoles (and charges), and where each solve's field goes: P shares per
+// sorted atom, one per x-plane it reaches, out[(s P + j) 3 + c] (summed by the readers, RecField).  cplxStride:
+// elements between the solves' complex grids.
+template<class T>
+struct PlaneSolves {
+    int n;
+    const typename Vec4<T>::type* dip[2];
+    int withQ[2];
+    double* out[2];
+    size_t cplxStride;
+};
+// The density of the solves spread into the x-planes and transformed in z and y into cplx; their potentials transformed
+// back and gathered (launchPmeConvolve with stages = 0 in between).
+template<class T>
+void launchPlaneSpread(hipStream_t st, const FftLaunch& L, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms,
+                       const typename Vec4<T>::type* posq, const PlaneSolves<T>& solves,
+                       typename Vec2<T>::type* cplx, const typename Vec2<T>::type* tw, const int* skip);
+template<class T>
+void launchPlaneGather(hipStream_t st, const FftLaunch& L, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms,
+                       const PlaneSolves<T>& solves, typename Vec2<T>::type* cplx,
+                       const typename Vec2<T>::type* tw, const int* skip);
 // Blocks of the x pass per grid (the rows of its energy partials) when ngrid grids of shape g are stacked.
 template<class T>
 int convolveBlocksPerGrid(PmeGrid g, int ngrid);
 // Field -grad phi (sorted order) and, when final, the reciprocal forces.
 template<class T>
-void launchGather(hipStream_t st, PmeSel ps, int n, const int* pmeAtom, const int* base, const T* spl, const T* phi,
+void launchGather(hipStream_t st, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms, const T* phi,
                   const typename Vec4<T>::type* dip, const typename Vec4<T>::type* posq, int final_, double* field,
                   double* force, const int* skip);
 // Potential and field of the convolved grid phi at the atoms and, with phiDot, their tangents for atoms displaced
 // by disp: out (sorted order) phi[n], E[3n] at offsets 0 and n, phi'[n], E'[3n] at offsets 5n and 6n.
 template<class T>
-void launchGatherTangent(hipStream_t st, PmeSel ps, int n, const int* pmeAtom, const int* base, const T* spl,
+void launchGatherTangent(hipStream_t st, PmeSel ps, int n, const int* brickStart, const PmeAtom<T>* atoms,
                          const T* phi, const T* phiDot, const typename Vec4<T>::type* disp, double* out);
 template<class T>
 void launchInfluence(hipStream_t st, PmeGrid g, const double* bmod, BoxT<double> box, double beta, double volume,
@@ -406,10 +477,24 @@ struct GuessCoef {
     double c[4];
 };
 
+// The reciprocal field of a solve: parts 3-vectors per sorted atom to be summed (the x-plane gather writes one per
+// plane an atom reaches, kGather the sum).
+struct RecField {
+    const double* p;
+    int parts;
+};
+__device__ __forceinline__ double recField(const RecField& f, int s, int c) {
+    const double* v = f.p+(size_t) s*f.parts*3+c;
+    double sum = v[0];
+    for (int j = 1; j < f.parts; j++)
+        sum += v[3*j];
+    return sum;
+}
+
 void launchGuess(hipStream_t st, int n, const int* order, const int* gidx, const double* hist, size_t slotStride,
                  GuessCoef gc, const double* alpha, const double* b, double* x);
 // b = field_dir + field_rec + cself * perm.
-void launchCombineB(hipStream_t st, int n, const double* ed, const double* er, const double* perm, double cself,
+void launchCombineB(hipStream_t st, int n, const double* ed, RecField er, const double* perm, double cself,
                     double* b);
 template<class T>
 void launchToVec4(hipStream_t st, int n, const double* v, typename Vec4<T>::type* out, const T* rgw = nullptr);
@@ -423,10 +508,10 @@ struct Precond {
 };
 template<class T>
 void launchCgInit(hipStream_t st, int n, const double* alpha, const double* b, const double* x, const double* td,
-                  const double* tr, double cself, double tol, int maxIter, double* r, double* z, double* p,
+                  RecField tr, double cself, double tol, int maxIter, double* r, double* z, double* p,
                   typename Vec4<T>::type* pT, double* partials, CgState* cg, int* done, Precond pc,
                   const T* rgw = nullptr);
-void launchCgAp(hipStream_t st, int n, int it, const double* alpha, const double* p, const double* td, const double* tr,
+void launchCgAp(hipStream_t st, int n, int it, const double* alpha, const double* p, const double* td, RecField tr,
                 double cself, double* ap, double* partials, const int* done);
 void launchCgUpdate(hipStream_t st, int n, int it, const double* alpha, const double* p, const double* ap, double* x,
                     double* r, double* z, double* partials, const int* done, Precond pc);

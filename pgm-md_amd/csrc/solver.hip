@@ -54,10 +54,10 @@ __global__ void kGuess(int n, const int* order, const int* gidx, const double* h
     x[k] = (a > 0 ? v : 0.0);
 }
 
-__global__ void kCombineB(int n, const double* ed, const double* er, const double* perm, double cself, double* b) {
+__global__ void kCombineB(int n, const double* ed, RecField er, const double* perm, double cself, double* b) {
     const int k = blockIdx.x*blockDim.x+threadIdx.x;
     if (k < 3*n)
-        b[k] = ed[k]+er[k]+cself*perm[k];
+        b[k] = ed[k]+recField(er, k/3, k%3)+cself*perm[k];
 }
 
 // The pair vector type of a 3-vector per atom, w = rgw[s] (the radius parameter, read by the FP32 field pass
@@ -79,7 +79,7 @@ __global__ void kToVec4(int n, const double* v, typename Vec4<T>::type* out, con
 // alpha/(1 - alpha cj) r and the partials of r.z; with the short-range preconditioner kPrecond<true> does that.
 template<class T>
 __global__ void __launch_bounds__(kCgBlock) kCgInit(int n, const double* alpha, const double* b, const double* x,
-                                                    const double* td, const double* tr, double cself, double* r,
+                                                    const double* td, RecField tr, double cself, double* r,
                                                     double* z, double* p, typename Vec4<T>::type* pT,
                                                     double* partials, Precond pc, const T* rgw) {
     __shared__ double smem[40];
@@ -91,7 +91,7 @@ __global__ void __launch_bounds__(kCgBlock) kCgInit(int n, const double* alpha, 
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const int k = 3*s+c;
-            const double ax = (a > 0 ? x[k]/a-(td[k]+tr[k]+cself*x[k]) : 0.0);
+            const double ax = (a > 0 ? x[k]/a-(td[k]+recField(tr, s, c)+cself*x[k]) : 0.0);
             const double rv = (a > 0 ? b[k]-ax : 0.0);
             const double zv = f*rv;
             r[k] = rv;
@@ -139,15 +139,16 @@ __global__ void __launch_bounds__(kCgBlock) kCgInitCheck(int n, int nb, double t
 }
 
 __global__ void __launch_bounds__(kCgBlock) kCgAp(int n, const double* alpha, const double* p, const double* td,
-                                                  const double* tr, double cself, double* ap, double* partials,
+                                                  RecField tr, double cself, double* ap, double* partials,
                                                   const int* skip) {
     __shared__ double smem[40];
     if (*skip)
         return;
     double pap = 0;
     for (int k = blockIdx.x*blockDim.x+threadIdx.x; k < 3*n; k += gridDim.x*blockDim.x) {
-        const double a = alpha[k/3];
-        const double v = (a > 0 ? p[k]/a-(td[k]+tr[k]+cself*p[k]) : 0.0);
+        const int s = k/3;
+        const double a = alpha[s];
+        const double v = (a > 0 ? p[k]/a-(td[k]+recField(tr, s, k-3*s)+cself*p[k]) : 0.0);
         ap[k] = v;
         pap += p[k]*v;
     }
@@ -545,7 +546,7 @@ void launchGuess(hipStream_t st, int n, const int* order, const int* gidx, const
     kGuess<<<nblk(3LL*n, 256), 256, 0, st>>>(n, order, gidx, hist, slotStride, gc, alpha, b, x);
 }
 
-void launchCombineB(hipStream_t st, int n, const double* ed, const double* er, const double* perm, double cself,
+void launchCombineB(hipStream_t st, int n, const double* ed, RecField er, const double* perm, double cself,
                     double* b) {
     kCombineB<<<nblk(3LL*n, 256), 256, 0, st>>>(n, ed, er, perm, cself, b);
 }
@@ -557,14 +558,14 @@ void launchToVec4(hipStream_t st, int n, const double* v, typename Vec4<T>::type
 
 template<class T>
 void launchCgInit(hipStream_t st, int n, const double* alpha, const double* b, const double* x, const double* td,
-                  const double* tr, double cself, double tol, int maxIter, double* r, double* z, double* p,
+                  RecField tr, double cself, double tol, int maxIter, double* r, double* z, double* p,
                   typename Vec4<T>::type* pT, double* partials, CgState* cg, int* done, Precond pc, const T* rgw) {
     const int nb = cgBlocks(n);
     kCgInit<T><<<nb, kCgBlock, 0, st>>>(n, alpha, b, x, td, tr, cself, r, z, p, pT, partials, pc, rgw);
     kCgInitCheck<<<1, kCgBlock, 0, st>>>(n, nb, tol, maxIter, partials, cg, done);
 }
 
-void launchCgAp(hipStream_t st, int n, int it, const double* alpha, const double* p, const double* td, const double* tr,
+void launchCgAp(hipStream_t st, int n, int it, const double* alpha, const double* p, const double* td, RecField tr,
                 double cself, double* ap, double* partials, const int* done) {
     kCgAp<<<cgBlocks(n), kCgBlock, 0, st>>>(n, alpha, p, td, tr, cself, ap, partials, done+it);
 }
@@ -657,7 +658,7 @@ void launchUnsort3(hipStream_t st, int n, const int* rank, const double* v, doub
                                          double4*, Vec4<T>::type*, double*, Vec4<T>::type*);                          \
     template void launchToVec4<T>(hipStream_t, int, const double*, Vec4<T>::type*, const T*);                       \
     template void launchCgInit<T>(hipStream_t, int, const double*, const double*, const double*, const double*,     \
-                                  const double*, double, double, int, double*, double*, double*, Vec4<T>::type*,     \
+                                  RecField, double, double, int, double*, double*, double*, Vec4<T>::type*,         \
                                   double*, CgState*, int*, Precond, const T*);                                       \
     template void launchPrecond<T>(hipStream_t, int, int, bool, const double*, const double*, const double*,         \
                                    const Vec4<T>::type*, BoxSel<T>, const int*, const int*, const Vec2<T>::type*,     \
