@@ -48,7 +48,6 @@ constexpr size_t kPlaneLds = 150*1024;        // dynamic LDS an x-plane block ma
 // it a solve is a chain of launches of a few us each, and the two streams' waits for each other cost more than the
 // overlap gains (1,536 atoms 700 us per step beside, 590 in line; 24,000 atoms 712 and 725; 98,000 1,335 and 1,545).
 constexpr int kOverlapAtoms = 16384;
-constexpr int kChunkAtoms = 2048;             // rows per first-stage block of the per-system sums
 
 void hipCheck(hipError_t e, const char* what) {
     if (e != hipSuccess)
@@ -280,16 +279,6 @@ std::vector<double> bsplineModuli(int K, int p) {
 }
 
 
-// The result slots of one system's evaluation (device, read back once).
-enum {
-    kResPair = 0,      // energy, strain[9] (pair, already halved)
-    kResRec = 10,      // energy, strain[9] (k-space)
-    kResComb = 20,     // |d|^2, polarization, E_rec (x) d [9]
-    kResCov = 31,      // covalent strain [9]
-    kResGvdw = 40,     // GVDW energy
-    kResCount = 41,
-};
-
 }   // namespace
 
 namespace {
@@ -332,8 +321,9 @@ public:
             // pinned words read back by the evaluations (allocated here: a launch makes no allocation that
             // could wait for the GPU)
             listH_.reserve(64);
-            cgH_.reserve(64);
-            scalH_.reserve(64);
+            const size_t cgWords = (size_t) std::min(s_.max_iter, 1 << 20)+2;
+            cgH_.reserve(cgWords*sizeof(double));
+            scalH_.reserve(cgWords*sizeof(double));
             resH_.reserve(kResCount*sizeof(double));   // one system's sums
             scratchPtr_ = scratchAddress();
             st2_ = acquirePmeStream();   // last: released by the destructor, which runs only for a built engine
@@ -758,58 +748,53 @@ public:
             // sufficed (the solve's device flag); a solve that needed more is evaluated again, from the same guess
             // (the history is advanced only by a complete solve), with its convergence checked on the host.
             bool ahead = polarizable_ && s_.polarizable && numRecent_ > 0;
+            FinalOut out{};
+            out.fOut = fDev;
+            out.fixedOut = fixed;
+            out.stride = stride;
+            out.fixedScale = fixedScale;
+            if (fHost || keepForces) {
+                forcesOutD_.reserve(3*sizeof(double)*n_);
+                out.fAssign = forcesOutD_.as<double>();
+            }
+            // the evaluation's positions, for a backward at the same positions (which then skips evaluating)
+            lastPosD_.reserve(3*sizeof(double)*n_);
+            out.posKeep = lastPosD_.as<double>();
             for (;;) {
+                out.guard = ahead;
                 asyncEval_ = asyncCg_ = ahead;
                 asyncPredict_ = predictedIterations();
                 asyncStop_ = -1;
                 pendingPush_ = -1;
                 try {
                     if (mixed)
-                        run<float>(newStep, strainOut != nullptr);
+                        run<float>(newStep, strainOut != nullptr, out);
                     else
-                        run<double>(newStep, strainOut != nullptr);
+                        run<double>(newStep, strainOut != nullptr, out);
                 }
                 catch (...) {
                     asyncEval_ = asyncCg_ = false;
                     throw;
                 }
                 asyncEval_ = asyncCg_ = false;
-                const int* guard = (ahead && asyncStop_ >= 0 && asyncStop_ < s_.max_iter)
-                                       ? doneD_.as<int>()+asyncStop_ : nullptr;
-                // forces out, caller's order
-                tb(kPhFinal);
-                if (fDev || fixed)
-                    launchForcesOut(st_, n_, rankD_.as<int>(), fpairD_.as<double>(), frecD_.as<double>(),
-                                    fcovD_.as<double>(), s_.ke, fDev, fixed, stride, fixedScale, guard);
-                if (fHost || keepForces) {
-                    forcesOutD_.reserve(3*sizeof(double)*n_);
-                    launchZero<double>(st_, forcesOutD_.as<double>(), 3*(size_t) n_, nullptr);
-                    launchForcesOut(st_, n_, rankD_.as<int>(), fpairD_.as<double>(), frecD_.as<double>(),
-                                    fcovD_.as<double>(), s_.ke, forcesOutD_.as<double>(), nullptr, 0, 0.0);
+                if (out.fAssign) {
                     stageH_.reserve(3*sizeof(double)*n_);
                     HIPCHK(hipMemcpyAsync(stageH_.p, forcesOutD_.p, 3*sizeof(double)*n_, hipMemcpyDeviceToHost,
                                           st_));
                 }
-                te();
-                // the evaluation's positions, for a backward at the same positions (which then skips evaluating)
-                lastPosD_.reserve(3*sizeof(double)*n_);
-                HIPCHK(hipMemcpyAsync(lastPosD_.p, posDev_, 3*sizeof(double)*n_, hipMemcpyDeviceToDevice, st_));
                 const size_t resBytes = sys_.size()*kResCount*sizeof(double);
                 resH_.reserve(resBytes);
                 HIPCHK(hipMemcpyAsync(resH_.p, resD_.p, resBytes, hipMemcpyDeviceToHost, st_));
                 waitStream();
                 if (!ahead || asyncStop_ < 0)
                     break;
-                CgState cs;
-                int done;
-                std::memcpy(&cs, cgH_.p, sizeof(CgState));
-                std::memcpy(&done, cgH_.as<char>()+sizeof(CgState), sizeof(int));
-                const bool shortSolve = !done && asyncStop_ < s_.max_iter;
-                noteIterations(shortSolve ? asyncStop_+1 : cs.iterations);
+                const CgEnd end = cgEnd(cgH_.as<double>(), asyncStop_);
+                const bool shortSolve = !end.done && asyncStop_ < s_.max_iter;
+                noteIterations(shortSolve ? asyncStop_+1 : end.iterations);
                 if (!shortSolve) {
                     commitPush(pendingPush_);
-                    iterations_ = lastIterations_ = cs.iterations;
-                    residual_ = cs.err;
+                    iterations_ = lastIterations_ = end.iterations;
+                    residual_ = end.err;
                     break;
                 }
                 ahead = false;
@@ -878,8 +863,12 @@ public:
             pendingPrev_ = pendingChecking_ && prevValid_ && !repeat;
             if (pendingChecking_)
                 startListCheck(pendingPrev_);
-            posPrevD_.reserve(3*sizeof(double)*n_);
-            HIPCHK(hipMemcpyAsync(posPrevD_.p, posDev_, 3*sizeof(double)*n_, hipMemcpyDeviceToDevice, st_));
+            FinalOut out{};
+            out.fixedOut = fixed;
+            out.stride = stride;
+            out.fixedScale = fixedScale;
+            posPrevD_.reserve(3*sizeof(double)*n_);   // kept for the next launch's check, after this one's
+            out.posKeep = posPrevD_.as<double>();
             prevValid_ = !extList_;
             const bool mixed = s_.precision == PGM_MIXED;
             mixed ? prep<float>() : prep<double>();
@@ -889,7 +878,7 @@ public:
             syncCgNext_ = false;
             pendingPush_ = -1;
             try {
-                mixed ? run<float>(newStep, false) : run<double>(newStep, false);
+                mixed ? run<float>(newStep, false, out) : run<double>(newStep, false, out);
             }
             catch (...) {
                 asyncEval_ = asyncCg_ = false;
@@ -899,10 +888,6 @@ public:
             asyncEval_ = asyncCg_ = false;
             if (!cgAhead)
                 asyncStop_ = -1;   // the solve completed on the host: iterations_, residual_ are final
-            tb(kPhFinal);
-            launchForcesOut(st_, n_, rankD_.as<int>(), fpairD_.as<double>(), frecD_.as<double>(), fcovD_.as<double>(),
-                            s_.ke, nullptr, fixed, stride, fixedScale);
-            te();
             const size_t resBytes = sys_.size()*kResCount*sizeof(double);
             resH_.reserve(resBytes);
             HIPCHK(hipMemcpyAsync(resH_.p, resD_.p, resBytes, hipMemcpyDeviceToHost, st_));
@@ -964,13 +949,10 @@ public:
         double err = residual_;
         bool shortSolve = false;
         if (asyncStop_ >= 0 && polarizable_ && s_.polarizable) {
-            CgState cs;
-            int done;
-            std::memcpy(&cs, cgH_.p, sizeof(CgState));
-            std::memcpy(&done, cgH_.as<char>()+sizeof(CgState), sizeof(int));
-            its = cs.iterations;
-            err = cs.err;
-            shortSolve = !done && asyncStop_ < s_.max_iter;
+            const CgEnd end = cgEnd(cgH_.as<double>(), asyncStop_);
+            its = end.iterations;
+            err = end.err;
+            shortSolve = !end.done && asyncStop_ < s_.max_iter;
             noteIterations(shortSolve ? asyncStop_+1 : its);
         }
         if (stale) {
@@ -1101,7 +1083,7 @@ public:
         erD_.reserve(recBytes());
         nbD_.reserve(n*sizeof(int));
         pairSetup<T>(setupLanes(), fused_, nullptr);
-        pmeSolve<T>(permTD_.as<T4>(), true, posT<T>(), 0, false, erD_.as<double>(), nullptr, nullptr, nullptr);
+        pmeSolve<T>(permTD_.as<T4>(), true, posT<T>(), 0, false, erD_.as<double>(), nullptr, CgSkip{});
         const double cself = 4.0*s_.beta*s_.beta*s_.beta/(3.0*kSqrtPi);
         launchCombineB(st_, n, edD_.as<double>(), recField(erD_), permD_.as<double>(), cself, bD_.as<double>());
         tmpD_.reserve(3*sizeof(double)*n);
@@ -1142,7 +1124,7 @@ public:
                 cand = cmpPosD_.as<double>();
             }
             cmpFlagD_.reserve(sizeof(int));
-            launchZero<int>(st_, cmpFlagD_.as<int>(), 1, nullptr);
+            launchZero<int>(st_, cmpFlagD_.as<int>(), 1, CgSkip{});
             launchDiffers(st_, 3LL*n_, cand, lastPosD_.as<double>(), cmpFlagD_.as<int>());
             cmpH_.reserve(64);
             HIPCHK(hipMemcpyAsync(cmpH_.p, cmpFlagD_.p, sizeof(int), hipMemcpyDeviceToHost, st_));
@@ -1578,21 +1560,21 @@ private:
     DevBuf listScanD_, brickScanD_;   // the tile sums of the long scans (list build, PME bricks)
     DevBuf qSD_, rgSD_, alphaSD_, posDD_, posFD_;
     DevBuf permD_, permTD_, edD_, erD_, bD_, xD_, rD_, zD_, pD_, apD_, tdD_, trD_, pTD_, dD_, dTD_, etotD_;
-    DevBuf fpairD_, frecD_, fcovD_, forcesOutD_, tmpD_;
+    DevBuf fpairD_, frecD_, forcesOutD_, tmpD_;
     DevBuf brickOfD_, pslotD_, brickCountD_, brickStartD_, pmeAtomD_;
     DevBuf fqD_, fdD_;   // the charges and dipoles of a field evaluation (caller's order)
     DevBuf gridD_, gridFixedD_, cplxD_, inflD_, twD_, bmodD_;
     const long long* fixedClean_ = nullptr;   // gridFixedD_ as last left all zero, over fixedCleanWords_ words
     size_t fixedCleanWords_ = 0;
-    DevBuf cgPartD_, partD_, resD_, cgD_, doneD_, histD_, maxBitsD_;
+    DevBuf cgPartD_, partD_, resD_, cgD_, histD_, maxBitsD_;
     DevBuf perAtomD_, chunkSumD_;
     DevBuf fftGroupsD_;     // the merged transform launches' group table
     DevBuf blockGroupD_[4];   // and the group of every block of the z, y, x and fused z+y launches
     FftLaunch fftL_{};
     // systems tables (batch)
     DevBuf sysOfD_, boxTabD_, boxTabFD_, pmeTabD_, brickSysD_, groupBoxD_, chunkStartD_, sysChunkD_;
-    DevBuf recStartD_, recSysD_, qBackD_, wED_;
-    int nChunks_ = 0, nRecRanges_ = 0;
+    DevBuf recStartD_, recSysD_, sysRecD_, qBackD_, wED_;   // sysRec: system -> its place among the stacked grids
+    int nChunks_ = 0;
     // parameter gradients
     DevBuf pairOutD_, pmeOutD_, gridTD_, gSD_, gTD_, pdotD_, lamD_, adjBD_, ddotD_, ddotTD_, etotDotD_, gInD_, gradD_;
     int adjIterations_ = 0, lastAdjIterations_ = 0;
@@ -1991,14 +1973,17 @@ private:
                 launchTwiddles<double>(st_, G.g, twD_.as<double2>()+G.twOff);
         }
         upload(bmodD_, bm.data(), bm.size()*sizeof(double));
-        nRecRanges_ = (int) recSys.size();
+        std::vector<int> sysRec(recSys.size());
+        for (size_t r = 0; r < recSys.size(); r++)
+            sysRec[recSys[r]] = (int) r;
+        upload(sysRecD_, sysRec.data(), sysRec.size()*sizeof(int));
         upload(recStartD_, recStart.data(), recStart.size()*sizeof(int));
         upload(recSysD_, recSys.data(), recSys.size()*sizeof(int));
-        // per-system sums of per-atom rows: chunks of at most kChunkAtoms atoms inside one system
+        // per-system sums of per-atom rows: chunks of at most kFinalChunk atoms inside one system
         std::vector<int> chunkStart(1, 0), sysChunk(1, 0);
         for (Sys& y : sys_) {
-            for (int a = y.a0; a < y.a1; a += kChunkAtoms)
-                chunkStart.push_back(std::min(y.a1, a+kChunkAtoms));
+            for (int a = y.a0; a < y.a1; a += kFinalChunk)
+                chunkStart.push_back(std::min(y.a1, a+kFinalChunk));
             sysChunk.push_back((int) chunkStart.size()-1);
         }
         nChunks_ = (int) chunkStart.size()-1;
@@ -2253,7 +2238,7 @@ private:
         rankD_.reserve(n*sizeof(int));
         sortedCellD_.reserve(n*sizeof(int));
         subOfD_.reserve(n*sizeof(int));
-        launchZero<int>(st_, cellCountD_.as<int>(), (size_t) cellTotal_, nullptr);
+        launchZero<int>(st_, cellCountD_.as<int>(), (size_t) cellTotal_, CgSkip{});
         for (const Sys& y : sys_) {
             const int ns = y.a1-y.a0;
             const BoxT<double> bd = makeBox<double>(y.H, y.recip);
@@ -2379,7 +2364,7 @@ private:
     }
 
     template<class T>
-    void convolve(T* grid, int energyMode, bool strain, const int* skip, long long* fixed, int stages, int nsolve) {
+    void convolve(T* grid, int energyMode, bool strain, CgSkip skip, long long* fixed, int stages, int nsolve) {
         typedef typename Vec2<T>::type T2;
         const BoxT<double> one = makeBox<double>(sys_[0].H, sys_[0].recip);
         launchPmeConvolve<T>(pmeSt_, fftL_, grid, cplxD_.as<T2>(), inflD_.as<T>(), twD_.as<T2>(), one,
@@ -2389,7 +2374,7 @@ private:
     }
     // The x-plane passes (fftL_.plane): the densities of the solves spread and transformed in z and y.
     template<class T>
-    void planeSpread(PlaneSolves<T>& solves, const int* skip, int it) {
+    void planeSpread(PlaneSolves<T>& solves, CgSkip skip, int it) {
         typedef typename Vec2<T>::type T2;
         solves.cplxStride = (size_t) cplxTotal_;
         tb(kPhSpread, it);
@@ -2399,7 +2384,7 @@ private:
     }
     // ... and whole solves: spread, convolution, the fields gathered.
     template<class T>
-    void planeSolve(PlaneSolves<T> solves, const int* skip, int it = -1) {
+    void planeSolve(PlaneSolves<T> solves, CgSkip skip, int it = -1) {
         typedef typename Vec2<T>::type T2;
         planeSpread<T>(solves, skip, it);
         tb(kPhFft, it);
@@ -2416,7 +2401,7 @@ private:
 
     template<class T>
     void pmeGrids(const typename Vec4<T>::type* dip, bool withQ, const typename Vec4<T>::type* posq, int energyMode,
-                  bool strain, T* grid, const int* skip, double* res, int it,
+                  bool strain, T* grid, CgSkip skip, int it,
                   const typename Vec4<T>::type* dipDot = nullptr, const typename Vec4<T>::type* disp = nullptr) {
         const PmeSel ps = pmeSel();
         if (fftL_.plane && !dipDot) {   // spread into the x-planes, the potentials to grid
@@ -2427,9 +2412,6 @@ private:
             planeSpread<T>(one, skip, it);
             tb(kPhFft, it);
             convolve<T>(grid, energyMode, strain, skip, nullptr, kFftInverse, 1);
-            if (energyMode)
-                launchRangeSums(pmeSt_, partD_.as<double>(), 10, recStartD_.as<int>(), nRecRanges_,
-                                recSysD_.as<int>(), kResCount, res+kResRec);
             te();
             return;
         }
@@ -2442,7 +2424,7 @@ private:
             // the forward z transform zeroes every word it reads, so the grid is clean for the next spread; it is
             // cleared here only when that is not known (new buffer, a larger layout, a solve cut short)
             if (fixed != fixedClean_ || fixedWords > fixedCleanWords_)
-                launchZero<long long>(pmeSt_, fixed, fixedWords, nullptr);
+                launchZero<long long>(pmeSt_, fixed, fixedWords, CgSkip{});
             fixedClean_ = nullptr;
         }
         else
@@ -2456,15 +2438,12 @@ private:
             fixedClean_ = fixed;
             fixedCleanWords_ = fixedWords;
         }
-        if (energyMode)
-            launchRangeSums(pmeSt_, partD_.as<double>(), 10, recStartD_.as<int>(), nRecRanges_, recSysD_.as<int>(),
-                            kResCount, res+kResRec);
         te();
     }
 
     template<class T>
     void pmeSolve(const typename Vec4<T>::type* dip, bool withQ, const typename Vec4<T>::type* posq, int energyMode,
-                  bool strain, double* field, double* force, const int* skip, double* res, int it = -1) {
+                  bool strain, double* field, double* force, CgSkip skip, int it = -1) {
         if (fftL_.plane && !force) {
             PlaneSolves<T> one{};
             one.n = 1;
@@ -2474,7 +2453,7 @@ private:
             planeSolve<T>(one, skip, it);
             return;
         }
-        pmeGrids<T>(dip, withQ, posq, energyMode, strain, gridD_.as<T>(), skip, res, it);
+        pmeGrids<T>(dip, withQ, posq, energyMode, strain, gridD_.as<T>(), skip, it);
         tb(kPhGather, it);
         launchGather<T>(pmeSt_, pmeSel(), brickStartD_.as<int>(), pmeAtomD_.as<PmeAtom<T>>(), gridD_.as<T>(), dip,
                         posq, force ? 1 : 0, field, force, skip);
@@ -2482,7 +2461,7 @@ private:
     }
 
     template<class T>
-    void matvec(const typename Vec4<T>::type* posT, const typename Vec4<T>::type* dipT, const int* skip,
+    void matvec(const typename Vec4<T>::type* posT, const typename Vec4<T>::type* dipT, CgSkip skip,
                 int it = -1) {
         // the fork is recorded before the pair pass is enqueued (the PME stream waits for nothing later), and the
         // long pair pass is enqueued first, so the host's PME launches do not delay it
@@ -2492,93 +2471,109 @@ private:
                            g12D_.as<typename Vec2<T>::type>(), boxSel<T>(), tdD_.as<double>(), skip, lanes_, fieldOtf_,
                            (T) s_.beta, nextListDirection());
         te();
-        pmeSolve<T>(dipT, false, posT, 0, false, trD_.as<double>(), nullptr, skip, nullptr, it);
+        pmeSolve<T>(dipT, false, posT, 0, false, trD_.as<double>(), nullptr, skip, it);
         join();
     }
 
+    // How a solve ended, from its norm and residuals cg[0..1+stop] (CgSkip): the iterations it took, its last residual,
+    // and whether it converged.
+    struct CgEnd {
+        int iterations;
+        double err;
+        bool done;
+    };
+    CgEnd cgEnd(const double* cg, int stop) const {
+        int it = 0;
+        while (it < stop && cg[1+it]/cg[0] > s_.tol)
+            it++;
+        const double err = cg[1+it]/cg[0];
+        return CgEnd{it, err, !(err > s_.tol)};
+    }
+    CgSkip cgSkip(int it) const { return CgSkip{cgD_.as<double>(), it, s_.tol}; }
+    // The state after `it` iterations into pinned memory, without a wait.
+    void readCg(HostBuf& h, int it) {
+        h.reserve((size_t) (it+2)*sizeof(double));
+        HIPCHK(hipMemcpyAsync(h.p, cgD_.p, (size_t) (it+2)*sizeof(double), hipMemcpyDeviceToHost, st_));
+    }
+
     // Jacobi-preconditioned CG on the polarizable rows of (alpha^-1 - T) x = b from the guess x, whose product
-    // T x is in tdD_ / trD_.  Iterations are enqueued ahead in chunks of the last solve's count, each behind a
-    // device flag, and the host reads the state once per chunk.  Returns the iterations; err: the final residual.
+    // T x is in tdD_ / trD_.  Iterations are enqueued ahead in chunks of the last solve's count, each behind the
+    // residual before it, and the host reads the state once per chunk.  Returns the iterations; err: the final
+    // residual.
     template<class T>
-    int cgSolve(const typename Vec4<T>::type* posT, const double* b, double* x, int& lastIts, double& err) {
+    int cgSolve(const typename Vec4<T>::type* posT, const CgRhs& rhs, double* x, int& lastIts, double& err) {
         typedef typename Vec4<T>::type T4;
         typedef typename Vec2<T>::type T2;
         const int n = n_;
         const double cself = 4.0*s_.beta*s_.beta*s_.beta/(3.0*kSqrtPi);
         const Precond pc{preReady_, (!preReady_ && jacobiSelf_) ? cself : 0.0};
-        const BoxSel<T> bt = boxSel<T>();
-        auto precond = [&](int it, bool init) {
-            if (pc.pre)
-                launchPrecond<T>(st_, n, it, init, alphaSD_.as<double>(), rD_.as<double>(), apD_.as<double>(), posT,
-                                 bt, srCountD_.as<int>(), srJD_.as<int>(), srGD_.as<T2>(), srOverD_.as<int>(),
-                                 zD_.as<double>(), pD_.as<double>(), pTD_.as<T4>(), cgPartD_.as<double>(),
-                                 doneD_.as<int>(), rgT<T>());
-        };
+        cgPartD_.reserve(kPRegions*kCgMaxBlocks*sizeof(double));
+        cgD_.reserve((size_t) (s_.max_iter+2)*sizeof(double));
         tb(kPhCg);
-        launchCgInit<T>(st_, n, alphaSD_.as<double>(), b, x, tdD_.as<double>(), recField(trD_), cself, s_.tol,
-                        s_.max_iter, rD_.as<double>(), zD_.as<double>(), pD_.as<double>(), pTD_.as<T4>(),
-                        cgPartD_.as<double>(), cgD_.as<CgState>(), doneD_.as<int>(), pc, rgT<T>());
-        precond(0, true);
+        launchCgInit<T>(st_, n, alphaSD_.as<double>(), rhs, x, tdD_.as<double>(), recField(trD_), cself,
+                        rD_.as<double>(), pD_.as<double>(), pTD_.as<T4>(), cgPartD_.as<double>(), cgD_.as<double>(),
+                        pc, rgT<T>());
+        if (pc.pre)
+            launchPrecond<T>(st_, n, 0, true, alphaSD_.as<double>(), rD_.as<double>(), apD_.as<double>(), posT,
+                             boxSel<T>(), srCountD_.as<int>(), srJD_.as<int>(), srGD_.as<T2>(), srOverD_.as<int>(),
+                             zD_.as<double>(), pD_.as<double>(), pTD_.as<T4>(), cgPartD_.as<double>(), CgSkip{},
+                             rgT<T>());
         te();
         int it = 0;
         if (asyncCg_) {
-            // enqueued ahead, no host wait: the predicted iterations, then the state and the flag that says
-            // whether they sufficed, read by the launch's completion
+            // enqueued ahead, no host wait: the predicted iterations, then the state that says whether they sufficed,
+            // read by the launch's completion
             const int stop = std::min(s_.max_iter, asyncPredict_);
             for (; it < stop; it++)
                 cgIteration<T>(posT, x, it, pc);
-            cgH_.reserve(64);
-            HIPCHK(hipMemcpyAsync(cgH_.p, cgD_.p, sizeof(CgState), hipMemcpyDeviceToHost, st_));
-            HIPCHK(hipMemcpyAsync(cgH_.as<char>()+sizeof(CgState), doneD_.as<int>()+stop, sizeof(int),
-                                  hipMemcpyDeviceToHost, st_));
+            readCg(cgH_, stop);
             asyncStop_ = stop;
             return -1;
         }
         int chunk = std::max(1, lastIts);
-        scalH_.reserve(64);
+        CgEnd end{};
         while (true) {
             const int stop = std::min(s_.max_iter, it+chunk);
             for (; it < stop; it++)
                 cgIteration<T>(posT, x, it, pc);
-            HIPCHK(hipMemcpyAsync(scalH_.p, cgD_.p, sizeof(CgState), hipMemcpyDeviceToHost, st_));
-            HIPCHK(hipMemcpyAsync(scalH_.as<char>()+sizeof(CgState), doneD_.as<int>()+it, sizeof(int),
-                                  hipMemcpyDeviceToHost, st_));
+            readCg(scalH_, it);
             waitStream();
-            int doneNow;
-            std::memcpy(&doneNow, scalH_.as<char>()+sizeof(CgState), sizeof(int));
-            if (doneNow || it >= s_.max_iter)
+            end = cgEnd(scalH_.as<double>(), it);
+            if (end.done || it >= s_.max_iter)
                 break;
             chunk = 1;
         }
-        CgState cs;
-        std::memcpy(&cs, scalH_.p, sizeof(CgState));
-        lastIts = cs.iterations;
-        err = cs.err;
-        noteIterations(cs.iterations);
-        return cs.iterations;
+        lastIts = end.iterations;
+        err = end.err;
+        noteIterations(end.iterations);
+        return end.iterations;
     }
 
-    // One CG iteration behind the device flag done[it] (every kernel returns at once when it is set).
+    // One CG iteration behind the residual before it (every kernel returns at once when that has converged).
     template<class T>
     void cgIteration(const typename Vec4<T>::type* posT, double* x, int it, const Precond& pc) {
         typedef typename Vec4<T>::type T4;
         typedef typename Vec2<T>::type T2;
         const int n = n_;
         const double cself = 4.0*s_.beta*s_.beta*s_.beta/(3.0*kSqrtPi);
-        const int* skip = doneD_.as<int>()+it;
+        const CgSkip skip = cgSkip(it);
         matvec<T>(posT, pTD_.as<T4>(), skip, it);
         tb(kPhCg, it);
-        launchCgAp(st_, n, it, alphaSD_.as<double>(), pD_.as<double>(), tdD_.as<double>(), recField(trD_), cself,
-                   apD_.as<double>(), cgPartD_.as<double>(), doneD_.as<int>());
-        launchCgUpdate(st_, n, it, alphaSD_.as<double>(), pD_.as<double>(), apD_.as<double>(), x, rD_.as<double>(),
-                       zD_.as<double>(), cgPartD_.as<double>(), doneD_.as<int>(), pc);
-        if (pc.pre)
+        launchCgAp(st_, n, it, alphaSD_.as<double>(), pD_.as<double>(), rD_.as<double>(), tdD_.as<double>(),
+                   recField(trD_), cself, apD_.as<double>(), cgPartD_.as<double>(), cgD_.as<double>(), skip, pc);
+        if (pc.pre) {
+            launchCgUpdate(st_, n, it, alphaSD_.as<double>(), pD_.as<double>(), apD_.as<double>(), x, rD_.as<double>(),
+                           cgPartD_.as<double>(), cgD_.as<double>(), skip);
             launchPrecond<T>(st_, n, it, false, alphaSD_.as<double>(), rD_.as<double>(), apD_.as<double>(), posT,
                              boxSel<T>(), srCountD_.as<int>(), srJD_.as<int>(), srGD_.as<T2>(), srOverD_.as<int>(),
-                             zD_.as<double>(), pD_.as<double>(), pTD_.as<T4>(), cgPartD_.as<double>(),
-                             doneD_.as<int>(), rgT<T>());
-        launchCgDirection<T>(st_, n, it, s_.tol, s_.max_iter, zD_.as<double>(), pD_.as<double>(), pTD_.as<T4>(),
-                             cgPartD_.as<double>(), cgD_.as<CgState>(), doneD_.as<int>(), rgT<T>());
+                             zD_.as<double>(), pD_.as<double>(), pTD_.as<T4>(), cgPartD_.as<double>(), skip,
+                             rgT<T>());
+            launchCgDirection<T>(st_, n, it, zD_.as<double>(), pD_.as<double>(), pTD_.as<T4>(), cgPartD_.as<double>(),
+                                 skip, rgT<T>());
+        }
+        else
+            launchCgStep<T>(st_, n, it, alphaSD_.as<double>(), apD_.as<double>(), x, rD_.as<double>(), pD_.as<double>(),
+                            pTD_.as<T4>(), cgPartD_.as<double>(), cgD_.as<double>(), skip, pc, rgT<T>());
         te();
     }
 
@@ -2599,14 +2594,6 @@ private:
             lo = std::min(lo, recentIts_[k]);
         }
         return std::min(hi+(numRecent_ > 0 && lo < hi ? 1 : 0), std::max(s_.max_iter, 1));
-    }
-
-    // Per-system sums of per-atom rows [n][width] into res[s][slot..slot+width).
-    void systemSums(const double* rows, int width, double* res, int slot) {
-        chunkSumD_.reserve((size_t) std::max(nChunks_, 1)*11*sizeof(double));
-        launchRangeSums(st_, rows, width, chunkStartD_.as<int>(), nChunks_, nullptr, width, chunkSumD_.as<double>());
-        launchRangeSums(st_, chunkSumD_.as<double>(), width, sysChunkD_.as<int>(), (int) sys_.size(), nullptr,
-                        kResCount, res+slot);
     }
 
     template<class T>
@@ -2730,8 +2717,17 @@ private:
         te();
     }
 
+    // Where an evaluation's forces go (FinalArgs); guard: only if the solve enqueued ahead sufficed.
+    struct FinalOut {
+        double *fAssign, *fOut, *posKeep;
+        long long* fixedOut;
+        int stride;
+        double fixedScale;
+        bool guard;
+    };
+
     template<class T>
-    void run(bool newStep, bool wantStrain) {
+    void run(bool newStep, bool wantStrain, const FinalOut& out) {
         typedef typename Vec4<T>::type T4;
         typedef typename Vec2<T>::type T2;
         const int n = n_;
@@ -2740,18 +2736,14 @@ private:
         const BoxSel<T> bt = boxSel<T>();
         const double cself = 4.0*s_.beta*s_.beta*s_.beta/(3.0*kSqrtPi);
         // per-atom buffers
-        for (DevBuf* b : {&permD_, &edD_, &bD_, &xD_, &rD_, &zD_, &pD_, &apD_, &tdD_, &dD_, &etotD_, &fpairD_,
-                          &frecD_, &fcovD_})
+        for (DevBuf* b : {&permD_, &edD_, &bD_, &xD_, &rD_, &zD_, &pD_, &apD_, &tdD_, &dD_, &etotD_, &fpairD_, &frecD_})
             b->reserve(v3);
         for (DevBuf* b : {&erD_, &trD_})
             b->reserve(recBytes());
         for (DevBuf* b : {&permTD_, &pTD_, &dTD_})
             b->reserve(n*sizeof(T4));
-        perAtomD_.reserve((size_t) n*11*sizeof(double));
+        perAtomD_.reserve((size_t) n*(wantStrain ? 10 : 1)*sizeof(double));
         partD_.reserve((size_t) std::max(partTotal_, 1)*10*sizeof(double));
-        cgPartD_.reserve(kPRegions*kCgMaxBlocks*sizeof(double));
-        cgD_.reserve(sizeof(CgState));
-        doneD_.reserve((s_.max_iter+2)*sizeof(int));
         nbD_.reserve(n*sizeof(int));
         T4* pos = posT<T>();
         // the initial guess: from the history when there is one, then its first product rides on the pair setup
@@ -2763,9 +2755,8 @@ private:
             histD_.reserve(kNHist*stride*sizeof(double));
         if (dual) {
             tb(kPhCg);
-            launchGuess(st_, n, orderD_.as<int>(), gidxD_.as<int>(), histD_.as<double>(), stride, gc,
-                        alphaSD_.as<double>(), bD_.as<double>(), xD_.as<double>());
-            launchToVec4<T>(st_, n, xD_.as<double>(), pTD_.as<T4>(), rgT<T>());
+            launchGuess<T>(st_, n, orderD_.as<int>(), gidxD_.as<int>(), histD_.as<double>(), stride, gc,
+                           alphaSD_.as<double>(), CgRhs{}, cself, nullptr, xD_.as<double>(), pTD_.as<T4>(), rgT<T>());
             te();
         }
         // field of the charges and permanent dipoles (and T x0): compaction + pair setup (fused or as two
@@ -2780,7 +2771,7 @@ private:
             srGD_.reserve((size_t) n*kPreCap*sizeof(T2));
             srOverD_.reserve(sizeof(int));
             tb(kPhCg);
-            launchZero<int>(st_, srOverD_.as<int>(), 1, nullptr);
+            launchZero<int>(st_, srOverD_.as<int>(), 1, CgSkip{});
             launchShortList<T>(st_, n, pos, candStartD_.as<int>(), nbD_.as<int>(), pjD_.as<int>(), g12D_.as<T2>(),
                                bt, (T) (preRadius_*preRadius_), srCountD_.as<int>(), srJD_.as<int>(),
                                srGD_.as<T2>(), srOverD_.as<int>());
@@ -2790,26 +2781,29 @@ private:
         // (the guess's reciprocal field too: its direct field rides on the setup pass)
         if (dual && fftL_.plane)
             planeSolve<T>(PlaneSolves<T>{2, {permTD_.as<T4>(), pTD_.as<T4>()}, {1, 0},
-                                         {erD_.as<double>(), trD_.as<double>()}, 0}, nullptr);
+                                         {erD_.as<double>(), trD_.as<double>()}, 0}, CgSkip{});
         else {
-            pmeSolve<T>(permTD_.as<T4>(), true, pos, 0, false, erD_.as<double>(), nullptr, nullptr, nullptr);
+            pmeSolve<T>(permTD_.as<T4>(), true, pos, 0, false, erD_.as<double>(), nullptr, CgSkip{});
             if (dual)
-                pmeSolve<T>(pTD_.as<T4>(), false, pos, 0, false, trD_.as<double>(), nullptr, nullptr, nullptr);
+                pmeSolve<T>(pTD_.as<T4>(), false, pos, 0, false, trD_.as<double>(), nullptr, CgSkip{});
         }
         join();
-        launchCombineB(st_, n, edD_.as<double>(), recField(erD_), permD_.as<double>(), cself, bD_.as<double>());
+        // b = the field of the charges and permanent dipoles: evaluated by the solve's first kernel where it is read
+        // once, stored by the guess where that needs it too
+        const CgRhs field{nullptr, edD_.as<double>(), recField(erD_), permD_.as<double>()};
+        const CgRhs stored{bD_.as<double>(), nullptr, RecField{}, nullptr};
         // induced dipoles
         int pushSlot = -1;
         if (induce) {
             if (!dual) {
                 tb(kPhCg);
-                launchGuess(st_, n, orderD_.as<int>(), gidxD_.as<int>(), histD_.as<double>(), stride, gc,
-                            alphaSD_.as<double>(), bD_.as<double>(), xD_.as<double>());
-                launchToVec4<T>(st_, n, xD_.as<double>(), pTD_.as<T4>(), rgT<T>());
+                launchGuess<T>(st_, n, orderD_.as<int>(), gidxD_.as<int>(), histD_.as<double>(), stride, gc,
+                               alphaSD_.as<double>(), field, cself, bD_.as<double>(), xD_.as<double>(),
+                               pTD_.as<T4>(), rgT<T>());
                 te();
-                matvec<T>(pos, pTD_.as<T4>(), nullptr);
+                matvec<T>(pos, pTD_.as<T4>(), CgSkip{});
             }
-            const int its = cgSolve<T>(pos, bD_.as<double>(), xD_.as<double>(), lastIterations_, residual_);
+            const int its = cgSolve<T>(pos, dual ? field : stored, xD_.as<double>(), lastIterations_, residual_);
             if (its >= 0)   // (else enqueued ahead: known when the launch completes)
                 iterations_ = its;
             const int h = (int) histSlots_.size();
@@ -2824,8 +2818,8 @@ private:
             te();
         }
         else {
-            launchZero<double>(st_, xD_.as<double>(), 3*(size_t) n, nullptr);
-            launchZero<double>(st_, rD_.as<double>(), 3*(size_t) n, nullptr);
+            launchZero<double>(st_, xD_.as<double>(), 3*(size_t) n, CgSkip{});
+            launchZero<double>(st_, rD_.as<double>(), 3*(size_t) n, CgSkip{});
             launchPost<T>(st_, n, 0.0, alphaSD_.as<double>(), rD_.as<double>(), xD_.as<double>(), permD_.as<double>(),
                           orderD_.as<int>(), gidxD_.as<int>(), nullptr, dD_.as<double>(), rgSD_.as<double>(),
                           dTD_.as<T4>());
@@ -2833,7 +2827,6 @@ private:
             residual_ = 0;
         }
         // final stage
-        double* res = resD_.as<double>();
         fork();
         tb(kPhPairFinal);
         const GvdwArgs<T> ga = gvdwArgs<T>();
@@ -2844,21 +2837,46 @@ private:
             launchGvdwSkip<T>(st_, n, orderD_.as<int>(), rankD_.as<int>(), pos, rgT<T>(), skipStartD_.as<int>(),
                               skipPartD_.as<int>(), bt, (T) (s_.cutoff*s_.cutoff), wantStrain, ga,
                               fpairD_.as<double>(), perAtomD_.as<double>());
-        systemSums(perAtomD_.as<double>(), wantStrain ? 10 : 1, res, kResPair);
-        if (ga.gv)
-            systemSums(gvdwAtomD_.as<double>(), 1, res, kResGvdw);
         te();
-        pmeSolve<T>(dTD_.as<T4>(), true, pos, 1, wantStrain, erD_.as<double>(), frecD_.as<double>(), nullptr, res);
+        pmeSolve<T>(dTD_.as<T4>(), true, pos, 1, wantStrain, erD_.as<double>(), frecD_.as<double>(), CgSkip{});
         join();
         tb(kPhFinal);
-        launchFinalCombine(st_, n, dD_.as<double>(), xD_.as<double>(), alphaSD_.as<double>(), edD_.as<double>(),
-                           erD_.as<double>(), cself, etotD_.as<double>(), perAtomD_.as<double>());
-        systemSums(perAtomD_.as<double>(), 11, res, kResComb);
-        launchCovalentForces(st_, n, rankD_.as<int>(), posDev_, covStartD_.as<int>(), covPartnerD_.as<int>(),
-                             covStrengthD_.as<double>(), revStartD_.as<int>(), revEntryD_.as<int>(),
-                             covAtomOfD_.as<int>(), etotD_.as<double>(), bd, fcovD_.as<double>(),
-                             perAtomD_.as<double>());
-        systemSums(perAtomD_.as<double>(), 9, res, kResCov);
+        chunkSumD_.reserve((size_t) std::max(nChunks_, 1)*kFinalWide*sizeof(double));
+        FinalArgs fa{};
+        fa.n = n;
+        fa.rank = rankD_.as<int>();
+        fa.pos = posDev_;
+        fa.covStart = covStartD_.as<int>();
+        fa.covPartner = covPartnerD_.as<int>();
+        fa.covStrength = covStrengthD_.as<double>();
+        fa.revStart = revStartD_.as<int>();
+        fa.revEntry = revEntryD_.as<int>();
+        fa.covAtomOf = covAtomOfD_.as<int>();
+        fa.d = dD_.as<double>();
+        fa.mu = xD_.as<double>();
+        fa.alpha = alphaSD_.as<double>();
+        fa.ed = edD_.as<double>();
+        fa.er = erD_.as<double>();
+        fa.fpair = fpairD_.as<double>();
+        fa.frec = frecD_.as<double>();
+        fa.pairRows = perAtomD_.as<double>();
+        fa.gvdw = ga.gv ? gvdwAtomD_.as<double>() : nullptr;
+        fa.cself = cself;
+        fa.ke = s_.ke;
+        fa.box = bd;
+        fa.fAssign = out.fAssign;
+        fa.fOut = out.fOut;
+        fa.fixedOut = out.fixedOut;
+        fa.stride = out.stride;
+        fa.fixedScale = out.fixedScale;
+        if (out.guard && asyncStop_ >= 0 && asyncStop_ < s_.max_iter)
+            fa.shortOf = cgSkip(asyncStop_);
+        fa.posKeep = out.posKeep;
+        fa.chunkStart = chunkStartD_.as<int>();
+        fa.chunkSums = chunkSumD_.as<double>();
+        launchFinal(st_, fa, nChunks_, wantStrain);
+        launchFinalSums(st_, chunkSumD_.as<double>(), wantStrain, sysChunkD_.as<int>(), (int) sys_.size(),
+                        partD_.as<double>(), recStartD_.as<int>(), sysRecD_.as<int>(), resD_.as<double>(), kResCount);
         te();
         if (asyncEval_)
             pendingPush_ = pushSlot;   // committed when the launch completes valid
@@ -2885,10 +2903,10 @@ private:
         timing_ = false;
         adjointReady_ = false;   // the products overwrite the evaluation's CG buffers
         PmeStreamScope scope(*this, overlap);
-        matvec<T>(posT<T>(), dTD_.as<T4>(), nullptr);   // warm-up
+        matvec<T>(posT<T>(), dTD_.as<T4>(), CgSkip{});   // warm-up
         HIPCHK(hipEventRecord(a, st_));
         for (int r = 0; r < reps; r++)
-            matvec<T>(posT<T>(), dTD_.as<T4>(), nullptr);
+            matvec<T>(posT<T>(), dTD_.as<T4>(), CgSkip{});
         HIPCHK(hipEventRecord(b, st_));
         HIPCHK(hipEventSynchronize(b));
         float ms = 0;
@@ -2935,7 +2953,7 @@ private:
             pairSetup<T>(lanes, fused, pTD_.as<T4>());
             for (int k = 0; k <= iterations_; k++)
                 launchPairField<T>(st_, n, pos, dTD_.as<T4>(), candStartD_.as<int>(), nbD_.as<int>(), pjD_.as<int>(),
-                                   g12D_.as<T2>(), bt, tdD_.as<double>(), nullptr, lanes, otf, (T) s_.beta,
+                                   g12D_.as<T2>(), bt, tdD_.as<double>(), CgSkip{}, lanes, otf, (T) s_.beta,
                                    nextListDirection());
             launchPairFinal<T>(st_, n, pos, dTD_.as<T4>(), rgT<T>(), (T) s_.beta, candStartD_.as<int>(),
                                nbD_.as<int>(), pjD_.as<int>(), g12D_.as<T2>(), g03D_.as<T2>(), bt,
@@ -2990,9 +3008,9 @@ private:
                                  candStartD_.as<int>(), nbD_.as<int>(), pjD_.as<int>(),
                                  g12D_.as<typename Vec2<T>::type>(), g03D_.as<typename Vec2<T>::type>(), bt,
                                  pairOutD_.as<double>());
-            pmeGrids<T>(dTD_.as<T4>(), true, pos, 0, false, gridD_.as<T>(), nullptr, nullptr, -1);
+            pmeGrids<T>(dTD_.as<T4>(), true, pos, 0, false, gridD_.as<T>(), CgSkip{}, -1);
             if (ddT)
-                pmeGrids<T>(dTD_.as<T4>(), true, pos, 0, false, gridTD_.as<T>(), nullptr, nullptr, -1, ddT,
+                pmeGrids<T>(dTD_.as<T4>(), true, pos, 0, false, gridTD_.as<T>(), CgSkip{}, -1, ddT,
                             gTD_.as<T4>());
             launchGatherTangent<T>(pmeSt_, pmeSel(), n, brickStartD_.as<int>(), pmeAtomD_.as<PmeAtom<T>>(),
                                    gridD_.as<T>(), ddT ? gridTD_.as<T>() : nullptr, ddT ? gTD_.as<T4>() : nullptr,
@@ -3013,11 +3031,12 @@ private:
                 tangentPass(ddotTD_.as<T4>());
                 launchAdjointRhs(st_, n, alphaSD_.as<double>(), pairOutD_.as<double>(), pmeOutD_.as<double>(),
                                  pdotD_.as<double>(), cself, adjBD_.as<double>());
-                launchGuess(st_, n, orderD_.as<int>(), gidxD_.as<int>(), nullptr, 0, GuessCoef{},
-                            alphaSD_.as<double>(), adjBD_.as<double>(), lamD_.as<double>());
-                launchToVec4<T>(st_, n, lamD_.as<double>(), pTD_.as<T4>(), rgT<T>());
-                matvec<T>(pos, pTD_.as<T4>(), nullptr);
-                adjIterations_ = cgSolve<T>(pos, adjBD_.as<double>(), lamD_.as<double>(), lastAdjIterations_,
+                const CgRhs rhs{adjBD_.as<double>(), nullptr, RecField{}, nullptr};
+                launchGuess<T>(st_, n, orderD_.as<int>(), gidxD_.as<int>(), nullptr, 0, GuessCoef{},
+                               alphaSD_.as<double>(), rhs, cself, nullptr, lamD_.as<double>(), pTD_.as<T4>(),
+                               rgT<T>());
+                matvec<T>(pos, pTD_.as<T4>(), CgSkip{});
+                adjIterations_ = cgSolve<T>(pos, rhs, lamD_.as<double>(), lastAdjIterations_,
                                             adjResidual_);
                 lambda = lamD_.as<double>();
                 launchDipoleTangent<T>(st_, n, pdotD_.as<double>(), lambda, ddotD_.as<double>(), ddotTD_.as<T4>());

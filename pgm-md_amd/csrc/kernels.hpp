@@ -8,6 +8,24 @@
 
 namespace pgmhip {
 
+// -------------------------------------------------------------------------------------------- CG state
+//
+// The CG's device-resident scalars: cg[0] = mean |alpha b| + 1e-300, cg[1+it] = max |alpha r| before iteration it (it =
+// 0..maxIter; 0 until known).  Iterations are enqueued ahead: every kernel of iteration it returns at once when the
+// solve has converged before it, cg[1+it]/cg[0] <= tol, and a skipped iteration leaves the next one's word zero, which
+// says the same.  The words are maxima of non-negative values, so they are gathered by integer atomics on their bits,
+// in any order (no kernel of its own reduces them and writes a flag).
+struct CgSkip {
+    const double* cg;   // nullptr: never
+    int it;
+    double tol;
+    __device__ __forceinline__ bool operator()() const { return cg && !(cg[1+it]/cg[0] > tol); }
+};
+
+// Partial sums of the CG kernels: regions of kCgMaxBlocks doubles.
+constexpr int kCgMaxBlocks = 1024;
+enum { kPNorm = 0, kPRz0 = 1, kPRz1 = 2, kPpAp = 3, kPBnum = 4, kPMax = 5, kPzAp = 6, kPfAA = 7, kPRegions = 8 };
+
 // -------------------------------------------------------------------------------------------- systems
 
 // The box of an atom.  A batch packs several independent periodic systems into one set of arrays: the atoms
@@ -175,7 +193,7 @@ void launchPairCompactSetup(hipStream_t st, int n, const typename Vec4<T>::type*
 template<class T>
 void launchPairField(hipStream_t st, int n, const typename Vec4<T>::type* pos, const typename Vec4<T>::type* dip,
                      const int* candStart, const int* nb, const int* pj, const typename Vec2<T>::type* g12,
-                     BoxSel<T> box, double* field, const int* skip, int lanes, bool otf = false, T beta = T(0),
+                     BoxSel<T> box, double* field, CgSkip skip, int lanes, bool otf = false, T beta = T(0),
                      bool reverse = false);
 // The CG preconditioner's short-range list: per atom, its compacted pairs within the radius (srJ partner, srG the
 // stored G1, G2; at most kPreCap, counted in srCount); *over set when an atom has more (cleared by the caller).
@@ -303,7 +321,7 @@ void launchPmePlace(hipStream_t st, int n, const double4* posD, PmeSel ps, const
 template<class T>
 void launchSpread(hipStream_t st, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms,
                   const typename Vec4<T>::type* dip, const typename Vec4<T>::type* posq, int withQ, T* grid,
-                  long long* fixed, const int* skip, const typename Vec4<T>::type* dipDot = nullptr,
+                  long long* fixed, CgSkip skip, const typename Vec4<T>::type* dipDot = nullptr,
                   const typename Vec4<T>::type* disp = nullptr);
 // The PME charge and dipole grids in 64-bit fixed point.  FP32: one word per point, 2^32 units per grid unit, the
 // reference's scale (core/cuda/pgm_cuda.cu:52), for |grid values| < 2^31.  FP64: two words per point, the value
@@ -411,7 +429,7 @@ enum { kFftForward = 1, kFftInverse = 2 };
 template<class T>
 void launchPmeConvolve(hipStream_t st, const FftLaunch& L, T* real, typename Vec2<T>::type* cplx, const T* influence,
                        const typename Vec2<T>::type* tw, BoxT<double> box, const BoxT<double>* boxes, double beta,
-                       int energy, int strain, double* partials, const int* skip, long long* fixed,
+                       int energy, int strain, double* partials, CgSkip skip, long long* fixed,
                        size_t fixedStride, int stages = kFftForward | kFftInverse, int nsolve = 1,
                        size_t cplxStride = 0);
 // The solves an x-plane launch runs at once: dipoles (and charges), and where each solve's field goes: P shares per
@@ -430,11 +448,11 @@ struct PlaneSolves {
 template<class T>
 void launchPlaneSpread(hipStream_t st, const FftLaunch& L, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms,
                        const typename Vec4<T>::type* posq, const PlaneSolves<T>& solves,
-                       typename Vec2<T>::type* cplx, const typename Vec2<T>::type* tw, const int* skip);
+                       typename Vec2<T>::type* cplx, const typename Vec2<T>::type* tw, CgSkip skip);
 template<class T>
 void launchPlaneGather(hipStream_t st, const FftLaunch& L, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms,
                        const PlaneSolves<T>& solves, typename Vec2<T>::type* cplx,
-                       const typename Vec2<T>::type* tw, const int* skip);
+                       const typename Vec2<T>::type* tw, CgSkip skip);
 // Blocks of the x pass per grid (the rows of its energy partials) when ngrid grids of shape g are stacked.
 template<class T>
 int convolveBlocksPerGrid(PmeGrid g, int ngrid);
@@ -442,7 +460,7 @@ int convolveBlocksPerGrid(PmeGrid g, int ngrid);
 template<class T>
 void launchGather(hipStream_t st, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms, const T* phi,
                   const typename Vec4<T>::type* dip, const typename Vec4<T>::type* posq, int final_, double* field,
-                  double* force, const int* skip);
+                  double* force, CgSkip skip);
 // Potential and field of the convolved grid phi at the atoms and, with phiDot, their tangents for atoms displaced
 // by disp: out (sorted order) phi[n], E[3n] at offsets 0 and n, phi'[n], E'[3n] at offsets 5n and 6n.
 template<class T>
@@ -454,22 +472,9 @@ void launchInfluence(hipStream_t st, PmeGrid g, const double* bmod, BoxT<double>
 template<class T>
 void launchTwiddles(hipStream_t st, PmeGrid g, typename Vec2<T>::type* tw);
 template<class T>
-void launchZero(hipStream_t st, T* p, size_t count, const int* skip);
+void launchZero(hipStream_t st, T* p, size_t count, CgSkip skip);
 
 // -------------------------------------------------------------------------------------------- solver
-
-// Scalars of the CG recurrence, device-resident.  done[it] (it = 0..maxIter) is set before iteration it
-// runs: every kernel of iteration it returns at once when it is set, so iterations can be enqueued ahead.
-struct CgState {
-    double norm;      // mean |alpha b| + 1e-300
-    double err;       // max |alpha r| / norm
-    int iterations;
-    int pad;
-};
-
-// Partial sums of the CG kernels: regions of kCgMaxBlocks doubles.
-constexpr int kCgMaxBlocks = 256;
-enum { kPNorm = 0, kPRz0 = 1, kPRz1 = 2, kPpAp = 3, kPBnum = 4, kPMax = 5, kPRegions = 6 };
 
 struct GuessCoef {
     int nc;          // 0: x = alpha b
@@ -491,8 +496,6 @@ __device__ __forceinline__ double recField(const RecField& f, int s, int c) {
     return sum;
 }
 
-void launchGuess(hipStream_t st, int n, const int* order, const int* gidx, const double* hist, size_t slotStride,
-                 GuessCoef gc, const double* alpha, const double* b, double* x);
 // b = field_dir + field_rec + cself * perm.
 void launchCombineB(hipStream_t st, int n, const double* ed, RecField er, const double* perm, double cself,
                     double* b);
@@ -506,15 +509,40 @@ struct Precond {
     bool pre;
     double cj;
 };
+// The right-hand side of a solve: b, or, b null, the field of the charges and permanent dipoles, ed + er + cself perm.
+struct CgRhs {
+    const double* b;
+    const double* ed;
+    RecField er;
+    const double* perm;
+};
+__device__ __forceinline__ double rhsOf(const CgRhs& q, double cself, int s, int c) {
+    const int k = 3*s+c;
+    return q.b ? q.b[k] : q.ed[k]+recField(q.er, s, c)+cself*q.perm[k];
+}
+// The initial guess, also as the pair vector type (w = rgw): the predictor over the history, or, gc.nc == 0, alpha b
+// (b then written to bOut when it is not null: a solve without a history needs b before its first product).
 template<class T>
-void launchCgInit(hipStream_t st, int n, const double* alpha, const double* b, const double* x, const double* td,
-                  RecField tr, double cself, double tol, int maxIter, double* r, double* z, double* p,
-                  typename Vec4<T>::type* pT, double* partials, CgState* cg, int* done, Precond pc,
+void launchGuess(hipStream_t st, int n, const int* order, const int* gidx, const double* hist, size_t slotStride,
+                 GuessCoef gc, const double* alpha, CgRhs rhs, double cself, double* bOut, double* x,
+                 typename Vec4<T>::type* xT, const T* rgw = nullptr);
+template<class T>
+void launchCgInit(hipStream_t st, int n, const double* alpha, CgRhs rhs, const double* x, const double* td,
+                  RecField tr, double cself, double* r, double* p,
+                  typename Vec4<T>::type* pT, double* partials, double* cg, Precond pc,
                   const T* rgw = nullptr);
-void launchCgAp(hipStream_t st, int n, int it, const double* alpha, const double* p, const double* td, RecField tr,
-                double cself, double* ap, double* partials, const int* done);
+// An iteration (Jacobi): the product A p with the sums p.Ap, z.Ap and Ap.f Ap (f the preconditioner's diagonal), then
+// everything else in one pass: with step = r.z/p.Ap and z' = z - step f Ap, the Polak-Ribiere numerator z'.(r' - r) is
+// -step (z.Ap - step Ap.f Ap), so the direction's coefficient is known before r' is written.
+void launchCgAp(hipStream_t st, int n, int it, const double* alpha, const double* p, const double* r, const double* td,
+                RecField tr, double cself, double* ap, double* partials, double* cg, CgSkip skip, Precond pc);
+template<class T>
+void launchCgStep(hipStream_t st, int n, int it, const double* alpha, const double* ap, double* x, double* r,
+                  double* p, typename Vec4<T>::type* pT, double* partials, double* cg, CgSkip skip, Precond pc,
+                  const T* rgw = nullptr);
+// ... and with the short-range preconditioner: launchCgAp, launchCgUpdate, launchPrecond, launchCgDirection.
 void launchCgUpdate(hipStream_t st, int n, int it, const double* alpha, const double* p, const double* ap, double* x,
-                    double* r, double* z, double* partials, const int* done, Precond pc);
+                    double* r, double* partials, double* cg, CgSkip skip);
 // z = alpha (r + sum_j T_ij alpha_j r_j) over the short list (partners with alpha_j > 0; M = D when *over), its
 // sums into the CG partials: init (after launchCgInit): p = z, r.z; else (after launchCgUpdate of iteration it):
 // -step z.Ap and the new r.z (core/cuda/pgm_cuda.cu:1526-1588).
@@ -522,34 +550,58 @@ template<class T>
 void launchPrecond(hipStream_t st, int n, int it, bool init, const double* alpha, const double* r, const double* ap,
                    const typename Vec4<T>::type* pos, BoxSel<T> box, const int* srCount, const int* srJ,
                    const typename Vec2<T>::type* srG, const int* over, double* z, double* p,
-                   typename Vec4<T>::type* pT, double* partials, const int* done, const T* rgw = nullptr);
+                   typename Vec4<T>::type* pT, double* partials, CgSkip skip, const T* rgw = nullptr);
 template<class T>
-void launchCgDirection(hipStream_t st, int n, int it, double tol, int maxIter, const double* z, double* p,
-                       typename Vec4<T>::type* pT, double* partials, CgState* cg, int* done, const T* rgw = nullptr);
+void launchCgDirection(hipStream_t st, int n, int it, const double* z, double* p, typename Vec4<T>::type* pT,
+                       double* partials, CgSkip skip, const T* rgw = nullptr);
 // x += peek alpha r; history push (global order, hist may be NULL); total dipoles d = perm + x, also as the pair
 // vector type dT with w = the radius parameter rgS of the (sorted) atom.
 template<class T>
 void launchPost(hipStream_t st, int n, double peek, const double* alpha, const double* r, double* x, const double* perm,
                 const int* order, const int* gidx, double* hist, double* d, const double* rgS,
                 typename Vec4<T>::type* dT);
-// Total field, and per atom perAtom[n][11]: |d|^2, mu^2/(2 alpha), E_rec (x) d (row-major).
-void launchFinalCombine(hipStream_t st, int n, const double* d, const double* mu, const double* alpha,
-                        const double* edir, const double* erec, double cself, double* etot, double* perAtom);
-// Covalent chain rule per atom (caller's order); per atom strain perAtom[n][9].
-void launchCovalentForces(hipStream_t st, int n, const int* rank, const double* pos, const int* covStart,
-                          const int* covPartner, const double* covStrength, const int* revStart, const int* revEntry,
-                          const int* covAtomOf, const double* etot, BoxSel<double> box, double* fcov,
-                          double* perAtom);
-// guard (may be null): the forces are added only where *guard is nonzero (a solve's convergence flag).
-void launchForcesOut(hipStream_t st, int n, const int* rank, const double* fpair, const double* frec,
-                     const double* fcov, double ke, double* fOut, long long* fixedOut, int stride, double fixedScale,
-                     const int* guard = nullptr);
-// Column sums of partials [nblk][width] into out[0..width).
-void launchReducePartials(hipStream_t st, const double* partials, int nblk, int width, double* out);
-// Column sums of row ranges: out[outRow(r)*outStride + c] = sum of rows[k][c], k in [starts[r], starts[r+1]),
-// for r < nr, c < width; outRow(r) = outIndex[r], or r when outIndex is null.  One block per range.
-void launchRangeSums(hipStream_t st, const double* rows, int width, const int* starts, int nr, const int* outIndex,
-                     int outStride, double* out);
+// The end of an evaluation in one pass over chunks of atoms (each inside one system): the total field ed + er + cself d
+// at the atoms and their covalent neighbours, the covalent chain rule, the forces out (caller's order, added; where
+// skip says that a solve enqueued ahead fell short, none), the positions kept, and per chunk the sums of the sorted
+// atoms' rows: with strain all of kFinalWide columns, else the kFinalNarrow first ones, which are the pair energy,
+// |d|^2, mu^2/(2 alpha) and the GVDW energy; then the pair strain, E_rec (x) d and the covalent strain, 9 each.
+constexpr int kFinalNarrow = 4, kFinalWide = 31, kFinalChunk = 256;
+// The result slots of one system's evaluation (device, read back once).
+enum {
+    kResPair = 0,      // energy, strain[9] (pair, already halved)
+    kResRec = 10,      // energy, strain[9] (k-space)
+    kResComb = 20,     // |d|^2, polarization, E_rec (x) d [9]
+    kResCov = 31,      // covalent strain [9]
+    kResGvdw = 40,     // GVDW energy
+    kResCount = 41,
+};
+struct FinalArgs {
+    int n;
+    const int* rank;
+    const double* pos;
+    const int *covStart, *covPartner;
+    const double* covStrength;
+    const int *revStart, *revEntry, *covAtomOf;
+    const double *d, *mu, *alpha, *ed, *er;   // sorted
+    const double *fpair, *frec;               // sorted pair and reciprocal forces
+    const double* pairRows;                   // sorted: [n] energy, or with strain [n][10] energy, strain
+    const double* gvdw;                       // sorted GVDW energies (nullptr: none)
+    double cself, ke;
+    BoxSel<double> box;
+    double* fAssign;                          // forces assigned, 3n (may be null)
+    double* fOut;                             // forces added (each may be null)
+    long long* fixedOut;
+    int stride;
+    double fixedScale;
+    CgSkip shortOf;                           // the forces are added only if this says converged (or is unset)
+    double* posKeep;                          // pos copied here (may be null)
+    const int* chunkStart;
+    double* chunkSums;                        // [chunks][kFinalNarrow or kFinalWide]
+};
+void launchFinal(hipStream_t st, const FinalArgs& a, int nchunks, bool strain);
+// The result slots of every system from the chunks' sums and the x pass's partials (recRows: [.][10] energy, strain).
+void launchFinalSums(hipStream_t st, const double* chunkSums, bool strain, const int* sysChunk, int nsys,
+                     const double* recRows, const int* recStart, const int* sysRec, double* res, int resStride);
 // In the caller's order: out[i] = v[rank[i]] (3-vectors).
 // The operands of a field evaluation of given charges q and dipoles d (caller's order) into the sorted arrays:
 // posD.w and, when set, posT.w = q; dS, dT = d (dT.w = rgw).

@@ -386,11 +386,11 @@ __global__ void __launch_bounds__(kPairBlock) kPairField(int n, const typename V
                                                          const int* __restrict__ candStart,
                                                          const int* __restrict__ nb, const int* __restrict__ pj,
                                                          const typename Vec2<T>::type* __restrict__ g12, BoxSel<T> bs,
-                                                         double* __restrict__ field, const int* skip,
+                                                         double* __restrict__ field, CgSkip skip,
                                                          bool reverse) {
     typedef typename Vec4<T>::type T4;
     typedef typename Vec2<T>::type T2;
-    if (skip && *skip)
+    if (skip())
         return;
     const int gid = xcdBlock(reverse)*blockDim.x+threadIdx.x;
     const int s = gid/L, lane = gid%L;
@@ -453,8 +453,8 @@ __global__ void __launch_bounds__(kPairBlock) kPairFieldOtf(int n, const float4*
                                                             const int* __restrict__ candStart,
                                                             const int* __restrict__ nb, const int* __restrict__ pj,
                                                             BoxSel<float> bs, float beta, double* __restrict__ field,
-                                                            const int* skip, bool reverse) {
-    if (skip && *skip)
+                                                            CgSkip skip, bool reverse) {
+    if (skip())
         return;
     const int gid = xcdBlock(reverse)*blockDim.x+threadIdx.x;
     const int s = gid/L, lane = gid%L;
@@ -998,7 +998,7 @@ void launchPairCompactSetup(hipStream_t st, int n, const typename Vec4<T>::type*
 template<class T>
 void launchPairField(hipStream_t st, int n, const typename Vec4<T>::type* pos, const typename Vec4<T>::type* dip,
                      const int* candStart, const int* nb, const int* pj, const typename Vec2<T>::type* g12,
-                     BoxSel<T> box, double* field, const int* skip, int lanes, bool otf, T beta, bool reverse) {
+                     BoxSel<T> box, double* field, CgSkip skip, int lanes, bool otf, T beta, bool reverse) {
     dispatchLanes(lanes, box.table != nullptr, [&](auto L, auto B) {
         if constexpr (sizeof(T) == sizeof(float)) {
             if (otf) {
@@ -1095,7 +1095,7 @@ void launchShortList(hipStream_t st, int n, const typename Vec4<T>::type* pos, c
                                             const Vec4<T>::type*, const int*, const int*, int*, int*, Vec2<T>::type*, \
                                             Vec2<T>::type*, BoxSel<T>, T, T, T, double*, double*, int);               \
     template void launchPairField<T>(hipStream_t, int, const Vec4<T>::type*, const Vec4<T>::type*, const int*,       \
-                                     const int*, const int*, const Vec2<T>::type*, BoxSel<T>, double*, const int*,    \
+                                     const int*, const int*, const Vec2<T>::type*, BoxSel<T>, double*, CgSkip,        \
                                      int, bool, T, bool);                                                             \
     template void launchPairFinal<T>(hipStream_t, int, const Vec4<T>::type*, const Vec4<T>::type*, const T*, T,      \
                                      const int*, const int*, const int*, const Vec2<T>::type*, const Vec2<T>::type*,  \

@@ -516,7 +516,7 @@ __global__ void __launch_bounds__(kBlock) kSpread(PmeSel ps, const int* __restri
                                                   const typename Vec4<T>::type* __restrict__ dip,
                                                   const typename Vec4<T>::type* __restrict__ posq, int withQ,
                                                   T* __restrict__ gridAll, long long* __restrict__ fixedAll,
-                                                  const int* skip,
+                                                  CgSkip skip,
                                                   const typename Vec4<T>::type* __restrict__ dipDot,
                                                   const typename Vec4<T>::type* __restrict__ disp) {
     typedef typename Vec4<T>::type T4;
@@ -526,7 +526,7 @@ __global__ void __launch_bounds__(kBlock) kSpread(PmeSel ps, const int* __restri
     extern __shared__ __align__(16) unsigned char smemRaw[];
     double* tile = reinterpret_cast<double*>(smemRaw);
     unsigned long long* tileI = reinterpret_cast<unsigned long long*>(smemRaw);   // W words per point, apart
-    if (skip && *skip)
+    if (skip())
         return;
     const int bid = blockIdx.x;
     const PmeSys* se = sysEntry<BATCH>(ps, BATCH ? ps.brickSys[bid] : 0);
@@ -661,11 +661,11 @@ template<class T, bool INVERSE, bool WIDE>
 __global__ void __launch_bounds__(kBlock) kFftZ(const FftGroup* __restrict__ groups,
                                                 const unsigned short* __restrict__ blockGroup,
                                                 T* __restrict__ realAll, typename Vec2<T>::type* __restrict__ cplxAll,
-                                                const typename Vec2<T>::type* __restrict__ twAll, const int* skip,
+                                                const typename Vec2<T>::type* __restrict__ twAll, CgSkip skip,
                                                 long long* __restrict__ fixedAll, size_t fixedStride) {
     typedef typename Vec2<T>::type T2;
     extern __shared__ __align__(16) unsigned char smemRaw[];
-    if (skip && *skip)
+    if (skip())
         return;
     const FftGroup& grp = groupOf(groups, blockGroup);
     const PmeGrid& g = grp.g;
@@ -774,10 +774,10 @@ template<class T, bool INVERSE, bool WIDE>
 __global__ void __launch_bounds__(kBlock) kFftY(const FftGroup* __restrict__ groups,
                                                 const unsigned short* __restrict__ blockGroup,
                                                 typename Vec2<T>::type* __restrict__ cplxAll,
-                                                const typename Vec2<T>::type* __restrict__ twAll, const int* skip) {
+                                                const typename Vec2<T>::type* __restrict__ twAll, CgSkip skip) {
     typedef typename Vec2<T>::type T2;
     extern __shared__ __align__(16) unsigned char smemRaw[];
-    if (skip && *skip)
+    if (skip())
         return;
     const FftGroup& grp = groupOf(groups, blockGroup);
     const PmeGrid& g = grp.g;
@@ -915,11 +915,11 @@ __global__ void __launch_bounds__(kPlaneThreads) kFftZY(const FftGroup* __restri
                                                         T* __restrict__ realAll,
                                                         typename Vec2<T>::type* __restrict__ cplxAll,
                                                         const typename Vec2<T>::type* __restrict__ twAll,
-                                                        const int* skip, long long* __restrict__ fixedAll,
+                                                        CgSkip skip, long long* __restrict__ fixedAll,
                                                         size_t fixedStride) {
     typedef typename Vec2<T>::type T2;
     extern __shared__ __align__(16) unsigned char smemRaw[];
-    if (skip && *skip)
+    if (skip())
         return;
     const FftGroup& grp = groupOf(groups, blockGroup);
     const PmeGrid& g = grp.g;
@@ -971,12 +971,11 @@ __global__ void __launch_bounds__(kPlaneThreads) kFftZY(const FftGroup* __restri
 // global atomics on it, no clearing.  Inverse (kPlaneGather): the plane's potential is gathered from LDS as it
 // leaves the z transform, each atom's share of the field from this plane written to its own place (out, P per atom,
 // summed by the reader): no grid of potentials in memory, no gather of 36 unaligned rows per atom.  A solve is three
-// launches (with kFftXConv) instead of seven.
+// launches (with kFftXConv) instead of seven.  Measured at 64 snapshots (2,735 planes, 207,831 atoms): spread + z + y
+// 128 -> 91 us, y + z + gather 90 -> 77 us per pass.  Bound by LDS latency and barriers: few wavefronts per plane.
 //
 // The atoms that reach plane x have x base points x..x+P-1 (mod K0): a run of slabs of bricks, contiguous in brick
-// order, and a second run where the range wraps.  Time per pass at 64 snapshots (2,900 planes, 207,831 atoms): spread
-// + z + y 128 -> 90 us, y + z + gather 90 -> 80 us.  Bound by LDS latency and barriers: few wavefronts per plane.
-//  planeAtoms walks the two runs in chunks: the chunk's atoms that
+// order, and a second run where the range wraps.  planeAtoms walks the two runs in chunks: the chunk's atoms that
 // do reach the plane are listed in LDS (with their row j1 = base - x), then work(atom in brick order, j1) runs with
 // every lane busy, one lane per atom and its P rows of P points.
 template<class T, int P, class Work>
@@ -1040,13 +1039,13 @@ __global__ void __launch_bounds__(kPlaneThreads) kPlaneSpread(const FftGroup* __
                                                               PlaneSolves<T> solves,
                                                               typename Vec2<T>::type* __restrict__ cplxAll,
                                                               const typename Vec2<T>::type* __restrict__ twAll,
-                                                              const int* skip) {
+                                                              CgSkip skip) {
     typedef typename Vec4<T>::type T4;
     typedef typename Vec2<T>::type T2;
     constexpr int W = GridFixed<T>::words;
     extern __shared__ __align__(16) unsigned char smemRaw[];
     __shared__ __align__(16) int list[kPlaneList+4];   // and its counter: whole 16 bytes before the dynamic LDS
-    if (skip && *skip)
+    if (skip())
         return;
     const FftGroup& grp = groupOf(groups, blockGroup);
     const PmeGrid& g = grp.g;
@@ -1118,11 +1117,11 @@ __global__ void __launch_bounds__(kPlaneThreads) kPlaneGather(const FftGroup* __
                                                               const PmeAtom<T>* __restrict__ atoms, PlaneSolves<T> solves,
                                                               typename Vec2<T>::type* __restrict__ cplxAll,
                                                               const typename Vec2<T>::type* __restrict__ twAll,
-                                                              const int* skip) {
+                                                              CgSkip skip) {
     typedef typename Vec2<T>::type T2;
     extern __shared__ __align__(16) unsigned char smemRaw[];
     __shared__ __align__(16) int list[kPlaneList+4];   // and its counter: whole 16 bytes before the dynamic LDS
-    if (skip && *skip)
+    if (skip())
         return;
     const FftGroup& grp = groupOf(groups, blockGroup);
     const PmeGrid& g = grp.g;
@@ -1187,11 +1186,11 @@ __global__ void __launch_bounds__(kBlock) kFftXConv(const FftGroup* __restrict__
                                                     const typename Vec2<T>::type* __restrict__ twAll,
                                                     BoxT<double> boxOne, const BoxT<double>* boxes, double beta,
                                                     int energy, int strain, double* __restrict__ partials,
-                                                    const int* skip, size_t cplxStride) {
+                                                    CgSkip skip, size_t cplxStride) {
     typedef typename Vec2<T>::type T2;
     extern __shared__ __align__(16) unsigned char smemRaw[];
     __shared__ double red[kBlock/64][10];
-    if (skip && *skip)
+    if (skip())
         return;
     const FftGroup& grp = groupOf(groups, blockGroup);
     const PmeGrid& g = grp.g;
@@ -1311,12 +1310,12 @@ __global__ void __launch_bounds__(kBlock) kGather(PmeSel ps, int n, const int* _
                                                   const typename Vec4<T>::type* __restrict__ posq,
                                                   const typename Vec4<T>::type* __restrict__ disp,
                                                   double* __restrict__ field, double* __restrict__ force,
-                                                  const int* skip) {
+                                                  CgSkip skip) {
     typedef typename Vec4<T>::type T4;
     constexpr bool POT = MODE >= kGatherPot, HESS = MODE == kGatherForce || MODE == kGatherTan, TAN = MODE == kGatherTan;
     extern __shared__ __align__(16) unsigned char smemRaw[];
     T* tile = reinterpret_cast<T*>(smemRaw);
-    if (skip && *skip)
+    if (skip())
         return;
     const int bid = blockIdx.x;
     const int first = brickStart[bid], count = brickStart[bid+1]-first;
@@ -1480,8 +1479,8 @@ __global__ void kTwiddles(PmeGrid g, typename Vec2<T>::type* tw) {
 }
 
 template<class T>
-__global__ void kZero(T* p, size_t count, const int* skip) {
-    if (skip && *skip)
+__global__ void kZero(T* p, size_t count, CgSkip skip) {
+    if (skip())
         return;
     for (size_t i = (size_t) blockIdx.x*blockDim.x+threadIdx.x; i < count; i += (size_t) gridDim.x*blockDim.x)
         p[i] = T(0);
@@ -1573,7 +1572,7 @@ void dispatchBricks(const PmeSel& ps, Fn fn) {
 template<class T>
 void launchSpread(hipStream_t st, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms,
                   const typename Vec4<T>::type* dip, const typename Vec4<T>::type* posq, int withQ, T* grid,
-                  long long* fixed, const int* skip, const typename Vec4<T>::type* dipDot,
+                  long long* fixed, CgSkip skip, const typename Vec4<T>::type* dipDot,
                   const typename Vec4<T>::type* disp) {
     const int E = ps.brick+ps.order-1;
     const size_t lds = (size_t) E*E*E*sizeof(double)*(dipDot ? 1 : GridFixed<T>::words);
@@ -1621,7 +1620,7 @@ void fftGroupShape(FftGroup& G, bool wide, int blocks[4], size_t lds[5]) {
 template<class T>
 void launchPmeConvolve(hipStream_t st, const FftLaunch& L, T* real, typename Vec2<T>::type* cplx, const T* influence,
                        const typename Vec2<T>::type* tw, BoxT<double> box, const BoxT<double>* boxes, double beta,
-                       int energy, int strain, double* partials, const int* skip, long long* fixed,
+                       int energy, int strain, double* partials, CgSkip skip, long long* fixed,
                        size_t fixedStride, int stages, int nsolve, size_t cplxStride) {
     const FftGroup* G = L.groups;
     auto go = [&](auto W) {
@@ -1656,7 +1655,7 @@ void launchPmeConvolve(hipStream_t st, const FftLaunch& L, T* real, typename Vec
 template<class T>
 void launchPlaneSpread(hipStream_t st, const FftLaunch& L, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms,
                        const typename Vec4<T>::type* posq, const PlaneSolves<T>& solves,
-                       typename Vec2<T>::type* cplx, const typename Vec2<T>::type* tw, const int* skip) {
+                       typename Vec2<T>::type* cplx, const typename Vec2<T>::type* tw, CgSkip skip) {
     dispatchOrder(ps.order, ps.table != nullptr, [&](auto P, auto B) {
         auto go = [&](auto W) {
             kPlaneSpread<T, P(), B(), W()><<<dim3(L.blocks[3], solves.n), L.planeThreads, L.lds[4], st>>>(
@@ -1669,7 +1668,7 @@ void launchPlaneSpread(hipStream_t st, const FftLaunch& L, PmeSel ps, const int*
 template<class T>
 void launchPlaneGather(hipStream_t st, const FftLaunch& L, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms,
                        const PlaneSolves<T>& solves, typename Vec2<T>::type* cplx,
-                       const typename Vec2<T>::type* tw, const int* skip) {
+                       const typename Vec2<T>::type* tw, CgSkip skip) {
     dispatchOrder(ps.order, ps.table != nullptr, [&](auto P, auto B) {
         auto go = [&](auto W) {
             kPlaneGather<T, P(), B(), W()><<<dim3(L.blocks[3], solves.n), L.planeThreads, L.lds[3], st>>>(
@@ -1698,17 +1697,17 @@ void launchGatherTangent(hipStream_t st, PmeSel ps, int n, const int* brickStart
     dispatchBricks(ps, [&](auto P, auto B, auto G) {
         if (phiDot)
             kGather<T, P(), kGatherTan, B(), G()><<<ps.nbrick, kBlock, gatherLds<T>(ps, 2), st>>>(
-                ps, n, brickStart, atoms, phi, phiDot, disp, nullptr, disp, out, nullptr, nullptr);
+                ps, n, brickStart, atoms, phi, phiDot, disp, nullptr, disp, out, nullptr, CgSkip{});
         else
             kGather<T, P(), kGatherPot, B(), G()><<<ps.nbrick, kBlock, gatherLds<T>(ps, 1), st>>>(
-                ps, n, brickStart, atoms, phi, nullptr, nullptr, nullptr, nullptr, out, nullptr, nullptr);
+                ps, n, brickStart, atoms, phi, nullptr, nullptr, nullptr, nullptr, out, nullptr, CgSkip{});
     });
 }
 
 template<class T>
 void launchGather(hipStream_t st, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms, const T* phi,
                   const typename Vec4<T>::type* dip, const typename Vec4<T>::type* posq, int final_, double* field,
-                  double* force, const int* skip) {
+                  double* force, CgSkip skip) {
     ps.byTile = fastDiv(ps.brick+ps.order-1);
     dispatchBricks(ps, [&](auto P, auto B, auto G) {
         if (final_)
@@ -1733,7 +1732,7 @@ void launchTwiddles(hipStream_t st, PmeGrid g, typename Vec2<T>::type* tw) {
 }
 
 template<class T>
-void launchZero(hipStream_t st, T* p, size_t count, const int* skip) {
+void launchZero(hipStream_t st, T* p, size_t count, CgSkip skip) {
     const int blocks = (int) std::min<size_t>(2048, (count+255)/256);
     kZero<T><<<std::max(1, blocks), 256, 0, st>>>(p, count, skip);
 }
@@ -1743,30 +1742,30 @@ void launchZero(hipStream_t st, T* p, size_t count, const int* skip) {
     template void launchPmePlace<T>(hipStream_t, int, const double4*, PmeSel, const int*, const int*, const int*,      \
                                     PmeAtom<T>*);                                                                      \
     template void launchSpread<T>(hipStream_t, PmeSel, const int*, const PmeAtom<T>*,                                  \
-                                  const Vec4<T>::type*, const Vec4<T>::type*, int, T*, long long*, const int*,         \
+                                  const Vec4<T>::type*, const Vec4<T>::type*, int, T*, long long*, CgSkip,             \
                                   const Vec4<T>::type*, const Vec4<T>::type*);                                         \
     template void launchGatherTangent<T>(hipStream_t, PmeSel, int, const int*, const PmeAtom<T>*, const T*,            \
                                          const T*, const Vec4<T>::type*, double*);                                     \
     template void fftGroupShape<T>(FftGroup&, bool, int*, size_t*);                                                       \
     template void launchPmeConvolve<T>(hipStream_t, const FftLaunch&, T*, Vec2<T>::type*, const T*,                    \
                                        const Vec2<T>::type*, BoxT<double>, const BoxT<double>*, double, int, int,     \
-                                       double*, const int*, long long*, size_t, int, int, size_t);                    \
+                                       double*, CgSkip, long long*, size_t, int, int, size_t);                    \
     template void launchPlaneSpread<T>(hipStream_t, const FftLaunch&, PmeSel, const int*, const PmeAtom<T>*,           \
                                        const Vec4<T>::type*, const PlaneSolves<T>&, Vec2<T>::type*,         \
-                                       const Vec2<T>::type*, const int*);                                             \
+                                       const Vec2<T>::type*, CgSkip);                                                 \
     template void launchPlaneGather<T>(hipStream_t, const FftLaunch&, PmeSel, const int*, const PmeAtom<T>*,           \
                                        const PlaneSolves<T>&, Vec2<T>::type*, const Vec2<T>::type*,         \
-                                       const int*);                                                                    \
+                                       CgSkip);                                                                        \
     template void launchGather<T>(hipStream_t, PmeSel, const int*, const PmeAtom<T>*, const T*,                        \
-                                  const Vec4<T>::type*, const Vec4<T>::type*, int, double*, double*, const int*);      \
+                                  const Vec4<T>::type*, const Vec4<T>::type*, int, double*, double*, CgSkip);          \
     template void launchInfluence<T>(hipStream_t, PmeGrid, const double*, BoxT<double>, double, double, T*);           \
     template void launchTwiddles<T>(hipStream_t, PmeGrid, Vec2<T>::type*);                                             \
-    template void launchZero<T>(hipStream_t, T*, size_t, const int*);                                                 \
+    template void launchZero<T>(hipStream_t, T*, size_t, CgSkip);                                                     \
     template int convolveBlocksPerGrid<T>(PmeGrid, int);
 PGM_INSTANTIATE_PME(float)
 PGM_INSTANTIATE_PME(double)
-template void launchZero<int>(hipStream_t, int*, size_t, const int*);
-template void launchZero<unsigned>(hipStream_t, unsigned*, size_t, const int*);
-template void launchZero<long long>(hipStream_t, long long*, size_t, const int*);
+template void launchZero<int>(hipStream_t, int*, size_t, CgSkip);
+template void launchZero<unsigned>(hipStream_t, unsigned*, size_t, CgSkip);
+template void launchZero<long long>(hipStream_t, long long*, size_t, CgSkip);
 
 }   // namespace pgmhip

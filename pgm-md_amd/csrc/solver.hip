@@ -9,9 +9,8 @@
 //               (core/pgm_core.cpp:488-534).
 #include "kernels.hpp"
 
-#include <stdexcept>
-
 #include <algorithm>
+#include <type_traits>
 
 namespace pgmhip {
 
@@ -21,37 +20,108 @@ constexpr int kCgBlock = 256;
 
 inline int nblk(long long threads, int bs) { return (int) ((threads+bs-1)/bs); }
 
-// Sum (or max) of one partials region of nb entries, computed redundantly by every block; valid in all threads.
-template<bool MAX>
-__device__ __forceinline__ double reduceRegion(const double* reg, int nb, double* smem) {
-    double v = 0;
-    for (int k = threadIdx.x; k < nb; k += blockDim.x)
-        v = MAX ? fmax(v, reg[k]) : v+reg[k];
-    v = MAX ? blockMax(v, smem) : blockSum(v, smem);
-    if (threadIdx.x == 0)
-        smem[32] = v;
+// Sums of the partials regions r[0..N) of nb entries each, computed redundantly by every block; valid in all threads.
+// One pass over the regions and one barrier.
+template<int N>
+__device__ __forceinline__ void reduceRegions(const double* partials, const int (&r)[N], int nb, double (*smem)[N],
+                                              double (&out)[N]) {
+    double v[N];
+#pragma unroll
+    for (int q = 0; q < N; q++)
+        v[q] = 0;
+    for (int k = threadIdx.x; k < nb; k += kCgBlock)
+#pragma unroll
+        for (int q = 0; q < N; q++)
+            v[q] += partials[r[q]*kCgMaxBlocks+k];
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        v[q] = groupSum<64>(v[q]);
+        if ((threadIdx.x & 63) == 0)
+            smem[threadIdx.x >> 6][q] = v[q];
+    }
     __syncthreads();
-    const double r = smem[32];
-    __syncthreads();
-    return r;
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        out[q] = 0;
+#pragma unroll
+        for (int w = 0; w < kCgBlock/64; w++)
+            out[q] += smem[w][q];
+    }
 }
 
-__global__ void kGuess(int n, const int* order, const int* gidx, const double* hist, size_t stride, GuessCoef gc,
-                       const double* alpha, const double* b, double* x) {
-    const int k = blockIdx.x*blockDim.x+threadIdx.x;
-    if (k >= 3*n)
-        return;
-    const int s = k/3, c = k-3*s;
-    const double a = alpha[s];
-    if (gc.nc == 0) {
-        x[k] = a*b[k];
-        return;
+// The block's sums of v into its entries of the regions r, and the maximum of mx into word (integer atomics on the
+// bits of a non-negative double).
+template<int N>
+__device__ __forceinline__ void writePartials(double (&v)[N], const int (&r)[N], double* partials, double (*smem)[N+1],
+                                              double mx, double* word) {
+#pragma unroll
+    for (int q = 0; q < N; q++)
+        v[q] = groupSum<64>(v[q]);
+    if (word)
+        mx = groupMax64(mx);
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int q = 0; q < N; q++)
+            smem[threadIdx.x >> 6][q] = v[q];
+        smem[threadIdx.x >> 6][N] = mx;
     }
-    const size_t g = 3*(size_t) gidx[order[s]]+c;
-    double v = 0;
-    for (int h = 0; h < gc.nc; h++)
-        v += gc.c[h]*hist[gc.slot[h]*stride+g];
-    x[k] = (a > 0 ? v : 0.0);
+    __syncthreads();
+    if (threadIdx.x < N) {
+        double t = 0;
+        for (int w = 0; w < kCgBlock/64; w++)
+            t += smem[w][threadIdx.x];
+        partials[r[threadIdx.x]*kCgMaxBlocks+blockIdx.x] = t;
+    }
+    if (threadIdx.x == N && word) {
+        double t = 0;
+        for (int w = 0; w < kCgBlock/64; w++)
+            t = fmax(t, smem[w][N]);
+        atomicMax(reinterpret_cast<unsigned long long*>(word), (unsigned long long) __double_as_longlong(t));
+    }
+}
+
+template<class T>
+__device__ __forceinline__ typename Vec4<T>::type pairVector(const double* v, T w) {
+    typename Vec4<T>::type o;
+    o.x = (T) v[0];
+    o.y = (T) v[1];
+    o.z = (T) v[2];
+    o.w = w;
+    return o;
+}
+
+template<class T>
+__global__ void kGuess(int n, const int* order, const int* gidx, const double* hist, size_t stride, GuessCoef gc,
+                       const double* alpha, CgRhs rhs, double cself, double* bOut, double* x,
+                       typename Vec4<T>::type* xT, const T* rgw) {
+    const int s = blockIdx.x*blockDim.x+threadIdx.x;
+    if (s >= n)
+        return;
+    const double a = alpha[s];
+    double v[3] = {0, 0, 0};
+    if (gc.nc == 0) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const double b = rhsOf(rhs, cself, s, c);
+            if (bOut)
+                bOut[3*s+c] = b;
+            v[c] = a*b;
+        }
+    }
+    else {
+        const double* h = hist+3*(size_t) gidx[order[s]];
+        for (int q = 0; q < gc.nc; q++)
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+                v[c] += gc.c[q]*h[gc.slot[q]*stride+c];
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            v[c] = (a > 0 ? v[c] : 0.0);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+        x[3*s+c] = v[c];
+    xT[s] = pairVector<T>(v, rgw ? rgw[s] : T(0));
 }
 
 __global__ void kCombineB(int n, const double* ed, RecField er, const double* perm, double cself, double* b) {
@@ -65,23 +135,23 @@ __global__ void kCombineB(int n, const double* ed, RecField er, const double* pe
 template<class T>
 __global__ void kToVec4(int n, const double* v, typename Vec4<T>::type* out, const T* rgw) {
     const int s = blockIdx.x*blockDim.x+threadIdx.x;
-    if (s >= n)
-        return;
-    typename Vec4<T>::type o;
-    o.x = (T) v[3*s];
-    o.y = (T) v[3*s+1];
-    o.z = (T) v[3*s+2];
-    o.w = rgw ? rgw[s] : T(0);
-    out[s] = o;
+    if (s < n)
+        out[s] = pairVector<T>(v+3*s, rgw ? rgw[s] : T(0));
 }
 
+// An iteration of the solve is launch-bound on small systems (each launch costs ~6 us of the stream, a kernel of 1,536
+// atoms runs 3-5 us) and a pass over 24-byte rows on large ones, so it takes two kernels: kCgAp with every sum the
+// step needs (p.Ap, z.Ap, Ap.f Ap: beta follows from those, z' = z - step f Ap), and kCgStep, which moves x, r and p at
+// once and evaluates z = f r where it is used.  The residual goes through one atomic maximum, which every later kernel
+// compares for itself.  Against four kernels per iteration, a separate convergence flag and the final stage in ten
+// launches: 1,536 atoms 522 -> 467 us per step, 8,550 557 -> 496, 24,000 685 -> 605, 999,000 10.2 -> 9.95 ms.
 // r = b - A x (polarizable rows); partials of sum |alpha b| and max |alpha r|.  Jacobi (not pc.pre): z = p =
 // alpha/(1 - alpha cj) r and the partials of r.z; with the short-range preconditioner kPrecond<true> does that.
 template<class T>
-__global__ void __launch_bounds__(kCgBlock) kCgInit(int n, const double* alpha, const double* b, const double* x,
+__global__ void __launch_bounds__(kCgBlock) kCgInit(int n, const double* alpha, CgRhs rhs, const double* x,
                                                     const double* td, RecField tr, double cself, double* r,
-                                                    double* z, double* p, typename Vec4<T>::type* pT,
-                                                    double* partials, Precond pc, const T* rgw) {
+                                                    double* p, typename Vec4<T>::type* pT, double* partials,
+                                                    Precond pc, const T* rgw) {
     __shared__ double smem[40];
     double nrm = 0, rz = 0, mx = 0;
     for (int s = blockIdx.x*blockDim.x+threadIdx.x; s < n; s += gridDim.x*blockDim.x) {
@@ -91,27 +161,21 @@ __global__ void __launch_bounds__(kCgBlock) kCgInit(int n, const double* alpha, 
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const int k = 3*s+c;
+            const double b = rhsOf(rhs, cself, s, c);
             const double ax = (a > 0 ? x[k]/a-(td[k]+recField(tr, s, c)+cself*x[k]) : 0.0);
-            const double rv = (a > 0 ? b[k]-ax : 0.0);
+            const double rv = (a > 0 ? b-ax : 0.0);
             const double zv = f*rv;
             r[k] = rv;
-            nrm += fabs(a*b[k]);
+            nrm += fabs(a*b);
             mx = fmax(mx, fabs(a*rv));   // the tolerance is on |alpha r| with every preconditioner
             if (!pc.pre) {
-                z[k] = zv;
                 p[k] = zv;
                 rz += rv*zv;
             }
             pv[c] = zv;
         }
-        if (!pc.pre) {
-            typename Vec4<T>::type o;
-            o.x = (T) pv[0];
-            o.y = (T) pv[1];
-            o.z = (T) pv[2];
-            o.w = rgw ? rgw[s] : T(0);
-            pT[s] = o;
-        }
+        if (!pc.pre)
+            pT[s] = pairVector<T>(pv, rgw ? rgw[s] : T(0));
     }
     nrm = blockSum(nrm, smem);
     rz = blockSum(rz, smem);
@@ -124,76 +188,112 @@ __global__ void __launch_bounds__(kCgBlock) kCgInit(int n, const double* alpha, 
     }
 }
 
-__global__ void __launch_bounds__(kCgBlock) kCgInitCheck(int n, int nb, double tol, int maxIter,
-                                                         const double* partials, CgState* cg, int* done) {
+// The norm and the first residual into cg.
+__global__ void __launch_bounds__(kCgBlock) kCgInitCheck(int n, int nb, const double* partials, double* cg) {
     __shared__ double smem[40];
-    const double nrm = reduceRegion<false>(partials+kPNorm*kCgMaxBlocks, nb, smem)/(3.0*n)+1e-300;
-    const double mx = reduceRegion<true>(partials+kPMax*kCgMaxBlocks, nb, smem);
-    if (threadIdx.x == 0) {
-        const double err = mx/nrm;
-        cg->norm = nrm;
-        cg->err = err;
-        cg->iterations = 0;
-        done[0] = (err > tol && 0 < maxIter) ? 0 : 1;
+    double nrm = 0, mx = 0;
+    for (int k = threadIdx.x; k < nb; k += blockDim.x) {
+        nrm += partials[kPNorm*kCgMaxBlocks+k];
+        mx = fmax(mx, partials[kPMax*kCgMaxBlocks+k]);
     }
-}
-
-__global__ void __launch_bounds__(kCgBlock) kCgAp(int n, const double* alpha, const double* p, const double* td,
-                                                  RecField tr, double cself, double* ap, double* partials,
-                                                  const int* skip) {
-    __shared__ double smem[40];
-    if (*skip)
-        return;
-    double pap = 0;
-    for (int k = blockIdx.x*blockDim.x+threadIdx.x; k < 3*n; k += gridDim.x*blockDim.x) {
-        const int s = k/3;
-        const double a = alpha[s];
-        const double v = (a > 0 ? p[k]/a-(td[k]+recField(tr, s, k-3*s)+cself*p[k]) : 0.0);
-        ap[k] = v;
-        pap += p[k]*v;
-    }
-    pap = blockSum(pap, smem);
-    if (threadIdx.x == 0)
-        partials[kPpAp*kCgMaxBlocks+blockIdx.x] = pap;
-}
-
-// x += step p, r' = r - step Ap; partials of max |alpha r'| and, Jacobi (not pc.pre), with z' = alpha/(1 - alpha
-// cj) r', of z'.(r' - r) and r'.z' (with the short-range preconditioner kPrecond<false> does those).
-__global__ void __launch_bounds__(kCgBlock) kCgUpdate(int n, int it, const double* alpha, const double* p,
-                                                      const double* ap, double* x, double* r, double* z,
-                                                      double* partials, const int* skip, Precond pc) {
-    __shared__ double smem[40];
-    if (*skip)
-        return;
-    const int nb = gridDim.x;
-    const double pap = reduceRegion<false>(partials+kPpAp*kCgMaxBlocks, nb, smem);
-    const double rz = reduceRegion<false>(partials+((it & 1) ? kPRz1 : kPRz0)*kCgMaxBlocks, nb, smem);
-    const double step = rz/fmax(pap, 1e-300);
-    double bnum = 0, rzn = 0, mx = 0;
-    for (int k = blockIdx.x*blockDim.x+threadIdx.x; k < 3*n; k += gridDim.x*blockDim.x) {
-        const double a = alpha[k/3];
-        x[k] += step*p[k];
-        const double rold = r[k];
-        const double rn = rold-step*ap[k];
-        mx = fmax(mx, fabs(a*rn));
-        r[k] = rn;
-        if (!pc.pre) {
-            const double zn = a/(1.0-a*pc.cj)*rn;
-            bnum += zn*(rn-rold);
-            rzn += rn*zn;
-            z[k] = zn;
-        }
-    }
-    bnum = blockSum(bnum, smem);
-    rzn = blockSum(rzn, smem);
+    nrm = blockSum(nrm, smem);
     mx = blockMax(mx, smem);
     if (threadIdx.x == 0) {
-        if (!pc.pre) {
-            partials[kPBnum*kCgMaxBlocks+blockIdx.x] = bnum;
-            partials[((it & 1) ? kPRz0 : kPRz1)*kCgMaxBlocks+blockIdx.x] = rzn;
-        }
-        partials[kPMax*kCgMaxBlocks+blockIdx.x] = mx;
+        cg[0] = nrm/(3.0*n)+1e-300;
+        cg[1] = mx;
     }
+}
+
+// Ap of iteration it and its partial sums; clears the iteration's residual word, also where the solve has converged
+// (the iterations after it are then skipped as well).
+__global__ void __launch_bounds__(kCgBlock) kCgAp(int n, int it, const double* alpha, const double* p, const double* r,
+                                                  const double* td, RecField tr, double cself, double* ap,
+                                                  double* partials, double* cg, CgSkip skip, Precond pc) {
+    __shared__ double smem[kCgBlock/64][4];
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        cg[2+it] = 0.0;
+    if (skip())
+        return;
+    double v[3] = {0, 0, 0};   // p.Ap, z.Ap, Ap.f Ap
+    for (int s = blockIdx.x*blockDim.x+threadIdx.x; s < n; s += gridDim.x*blockDim.x) {
+        const double a = alpha[s], f = a/(1.0-a*pc.cj);
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const int k = 3*s+c;
+            const double pk = p[k];
+            const double q = (a > 0 ? pk/a-(td[k]+recField(tr, s, c)+cself*pk) : 0.0);
+            ap[k] = q;
+            v[0] += pk*q;
+            if (!pc.pre) {
+                v[1] += f*r[k]*q;
+                v[2] += f*q*q;
+            }
+        }
+    }
+    const int reg[3] = {kPpAp, kPzAp, kPfAA};
+    writePartials<3>(v, reg, partials, smem, 0.0, nullptr);
+}
+
+// x += step p, r' = r - step Ap, z' = f r', p' = z' + beta p: the partials of r'.z' and max |alpha r'|.
+template<class T>
+__global__ void __launch_bounds__(kCgBlock) kCgStep(int n, int it, const double* alpha, const double* ap, double* x,
+                                                    double* r, double* p, typename Vec4<T>::type* pT,
+                                                    double* partials, double* cg, CgSkip skip, Precond pc,
+                                                    const T* rgw) {
+    __shared__ double smem[kCgBlock/64][4];
+    __shared__ double smem2[kCgBlock/64][2];
+    if (skip())
+        return;
+    const int reg[4] = {kPpAp, kPzAp, kPfAA, (it & 1) ? kPRz1 : kPRz0};
+    double sum[4];
+    reduceRegions<4>(partials, reg, gridDim.x, smem, sum);
+    const double rz = sum[3], step = rz/fmax(sum[0], 1e-300);
+    const double bc = -step*(sum[1]-step*sum[2])/fmax(rz, 1e-300);
+    double v[1] = {0}, mx = 0;
+    for (int s = blockIdx.x*blockDim.x+threadIdx.x; s < n; s += gridDim.x*blockDim.x) {
+        const double a = alpha[s], f = a/(1.0-a*pc.cj);
+        double d[3];
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const int k = 3*s+c;
+            const double pk = p[k];
+            x[k] += step*pk;
+            const double rn = r[k]-step*ap[k];
+            const double zn = f*rn;
+            r[k] = rn;
+            d[c] = zn+bc*pk;
+            p[k] = d[c];
+            mx = fmax(mx, fabs(a*rn));
+            v[0] += rn*zn;
+        }
+        pT[s] = pairVector<T>(d, rgw ? rgw[s] : T(0));
+    }
+    const int out[1] = {(it & 1) ? kPRz0 : kPRz1};
+    writePartials<1>(v, out, partials, smem2, mx, cg+2+it);
+}
+
+// With the short-range preconditioner: x += step p, r' = r - step Ap and max |alpha r'| (kPrecond<false> does the rest).
+__global__ void __launch_bounds__(kCgBlock) kCgUpdate(int n, int it, const double* alpha, const double* p,
+                                                      const double* ap, double* x, double* r, double* partials,
+                                                      double* cg, CgSkip skip) {
+    __shared__ double smem[kCgBlock/64][2];
+    __shared__ double red[40];
+    if (skip())
+        return;
+    const int reg[2] = {kPpAp, (it & 1) ? kPRz1 : kPRz0};
+    double sum[2];
+    reduceRegions<2>(partials, reg, gridDim.x, smem, sum);
+    const double step = sum[1]/fmax(sum[0], 1e-300);
+    double mx = 0;
+    for (int k = blockIdx.x*blockDim.x+threadIdx.x; k < 3*n; k += gridDim.x*blockDim.x) {
+        x[k] += step*p[k];
+        const double rn = r[k]-step*ap[k];
+        mx = fmax(mx, fabs(alpha[k/3]*rn));
+        r[k] = rn;
+    }
+    mx = blockMax(mx, red);
+    if (threadIdx.x == 0)
+        atomicMax(reinterpret_cast<unsigned long long*>(cg+2+it), (unsigned long long) __double_as_longlong(mx));
 }
 
 // The short-range preconditioner, z_s = alpha_s (r_s + sum_j T_sj alpha_j r_j), T_sj u = -u G1 + (u.x) x G2 over
@@ -207,18 +307,19 @@ __global__ void __launch_bounds__(kCgBlock) kPrecond(int n, int it, const double
                                                      BoxSel<T> bs, const int* srCount, const int* srJ,
                                                      const typename Vec2<T>::type* srG, const int* over, double* z,
                                                      double* p, typename Vec4<T>::type* pT, double* partials,
-                                                     const int* skip, const T* rgw) {
+                                                     CgSkip skip, const T* rgw) {
     typedef typename Vec4<T>::type T4;
     typedef typename Vec2<T>::type T2;
     __shared__ double smem[40];
-    if (!INIT && *skip)
+    __shared__ double red[kCgBlock/64][2];
+    if (!INIT && skip())
         return;
-    const int nb = gridDim.x;
     double step = 0;
     if (!INIT) {
-        const double pap = reduceRegion<false>(partials+kPpAp*kCgMaxBlocks, nb, smem);
-        const double rz = reduceRegion<false>(partials+((it & 1) ? kPRz1 : kPRz0)*kCgMaxBlocks, nb, smem);
-        step = rz/fmax(pap, 1e-300);
+        const int reg[2] = {kPpAp, (it & 1) ? kPRz1 : kPRz0};
+        double sum[2];
+        reduceRegions<2>(partials, reg, gridDim.x, red, sum);
+        step = sum[1]/fmax(sum[0], 1e-300);
     }
     const bool useT = (*over == 0);
     double rz = 0, bnum = 0;
@@ -281,21 +382,16 @@ __global__ void __launch_bounds__(kCgBlock) kPrecond(int n, int it, const double
 }
 
 template<class T>
-__global__ void __launch_bounds__(kCgBlock) kCgDirection(int n, int it, double tol, int maxIter, const double* z,
-                                                         double* p, typename Vec4<T>::type* pT,
-                                                         const double* partials, CgState* cg, int* done,
-                                                         const T* rgw) {
-    __shared__ double smem[40];
-    if (done[it]) {
-        // finished earlier: the flag of the next iteration (enqueued ahead) must say so too
-        if (blockIdx.x == 0 && threadIdx.x == 0)
-            done[it+1] = 1;
+__global__ void __launch_bounds__(kCgBlock) kCgDirection(int n, int it, const double* z, double* p,
+                                                         typename Vec4<T>::type* pT, const double* partials,
+                                                         CgSkip skip, const T* rgw) {
+    __shared__ double smem[kCgBlock/64][2];
+    if (skip())
         return;
-    }
-    const int nb = gridDim.x;
-    const double bnum = reduceRegion<false>(partials+kPBnum*kCgMaxBlocks, nb, smem);
-    const double rzOld = reduceRegion<false>(partials+((it & 1) ? kPRz1 : kPRz0)*kCgMaxBlocks, nb, smem);
-    const double bc = bnum/fmax(rzOld, 1e-300);
+    const int reg[2] = {kPBnum, (it & 1) ? kPRz1 : kPRz0};
+    double sum[2];
+    reduceRegions<2>(partials, reg, gridDim.x, smem, sum);
+    const double bc = sum[0]/fmax(sum[1], 1e-300);
     for (int s = blockIdx.x*blockDim.x+threadIdx.x; s < n; s += gridDim.x*blockDim.x) {
         double v[3];
 #pragma unroll
@@ -304,21 +400,7 @@ __global__ void __launch_bounds__(kCgBlock) kCgDirection(int n, int it, double t
             v[c] = z[k]+bc*p[k];
             p[k] = v[c];
         }
-        typename Vec4<T>::type o;
-        o.x = (T) v[0];
-        o.y = (T) v[1];
-        o.z = (T) v[2];
-        o.w = rgw ? rgw[s] : T(0);
-        pT[s] = o;
-    }
-    if (blockIdx.x == 0) {
-        const double mx = reduceRegion<true>(partials+kPMax*kCgMaxBlocks, nb, smem);
-        if (threadIdx.x == 0) {
-            const double err = mx/cg->norm;
-            cg->err = err;
-            cg->iterations = it+1;
-            done[it+1] = (err > tol && it+1 < maxIter) ? 0 : 1;
-        }
+        pT[s] = pairVector<T>(v, rgw ? rgw[s] : T(0));
     }
 }
 
@@ -351,48 +433,22 @@ __global__ void kPost(int n, double peek, const double* alpha, const double* r, 
     dT[s] = o;
 }
 
-__global__ void __launch_bounds__(kCgBlock) kFinalCombine(int n, const double* d, const double* mu,
-                                                          const double* alpha, const double* edir,
-                                                          const double* erec, double cself, double* etot,
-                                                          double* perAtom) {
-    const int s = blockIdx.x*blockDim.x+threadIdx.x;
-    if (s >= n)
-        return;
-    const double a = alpha[s];
-    double dv[3], er[3], d2 = 0, pol = 0;
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        dv[c] = d[3*s+c];
-        er[c] = erec[3*s+c];
-        etot[3*s+c] = edir[3*s+c]+er[c]+cself*dv[c];
-        d2 += dv[c]*dv[c];
-        if (a > 0)
-            pol += mu[3*s+c]*mu[3*s+c]/(2.0*a);
-    }
-    double* o = perAtom+11*(size_t) s;
-    o[0] = d2;
-    o[1] = pol;
-#pragma unroll
-    for (int p = 0; p < 3; p++)
-#pragma unroll
-        for (int q = 0; q < 3; q++)
-            o[2+3*p+q] = er[p]*dv[q];
-}
-
-// dE/dr_partner = c (g - (g.u) u)/|v|, g = -E_atom: +t on the atom, -t on the partner, strain t (x) v
-// (core/pgm_core.cpp:512-529).  One thread per atom sums the entries it carries and those it is partner of.
-__device__ __forceinline__ void covalentTerm(int m, const int* covAtomOf, const int* covPartner,
-                                             const double* covStrength, const double* pos, const int* rank,
-                                             const double* etot, const BoxT<double>& box, double t[3], double v[3]) {
-    const int i = covAtomOf[m], j = covPartner[m];
-    double x = pos[3*j]-pos[3*i], y = pos[3*j+1]-pos[3*i+1], z = pos[3*j+2]-pos[3*i+2];
+// Adds the chain-rule terms of covalent entry m: dE/dr_partner = c (g - (g.u) u)/|v|, g = -E_atom: t on the atom, -t on
+// the partner, strain t (x) v (core/pgm_core.cpp:512-529).
+__device__ __forceinline__ void covalentTerm(int m, const FinalArgs& a, const BoxT<double>& box, double t[3],
+                                             double v[3]) {
+    const int i = a.covAtomOf[m], j = a.covPartner[m];
+    double x = a.pos[3*j]-a.pos[3*i], y = a.pos[3*j+1]-a.pos[3*i+1], z = a.pos[3*j+2]-a.pos[3*i+2];
     minImage(x, y, z, box);
     const double len = sqrt(x*x+y*y+z*z);
     const double u[3] = {x/len, y/len, z/len};
-    const int si = rank[i];
-    const double g[3] = {-etot[3*si], -etot[3*si+1], -etot[3*si+2]};
+    const int si = a.rank[i];
+    double g[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        g[k] = -(a.ed[3*si+k]+a.er[3*si+k]+a.cself*a.d[3*si+k]);
     const double gu = g[0]*u[0]+g[1]*u[1]+g[2]*u[2];
-    const double c = covStrength[m]/len;
+    const double c = a.covStrength[m]/len;
 #pragma unroll
     for (int k = 0; k < 3; k++)
         t[k] = c*(g[k]-gu*u[k]);
@@ -401,109 +457,133 @@ __device__ __forceinline__ void covalentTerm(int m, const int* covAtomOf, const 
     v[2] = z;
 }
 
-// Per atom i (caller's order): the chain-rule force of the entries it carries (+t) and of those it is the
-// partner of (-t), and the strain of the entries it carries.  Atom and partner share a system.
-template<bool BATCH>
-__global__ void __launch_bounds__(kCgBlock) kCovalent(int n, const int* rank, const double* pos, const int* covStart,
-                                                      const int* covPartner, const double* covStrength,
-                                                      const int* revStart, const int* revEntry,
-                                                      const int* covAtomOf, const double* etot, BoxSel<double> bs,
-                                                      double* fcov, double* perAtom) {
-    const int i = blockIdx.x*blockDim.x+threadIdx.x;
-    if (i >= n)
-        return;
-    const BoxT<double> box = selectBox<BATCH>(bs, i);
-    double S[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    double f[3] = {0, 0, 0}, t[3], v[3];
-    for (int m = covStart[i]; m < covStart[i+1]; m++) {
-        covalentTerm(m, covAtomOf, covPartner, covStrength, pos, rank, etot, box, t, v);
+// Everything after the last field and force passes in one launch (launch-bound up to some 10^4 atoms, then the pass over
+// its ~250 bytes per atom): the entry fields are re-evaluated at a covalent partner instead of stored and read back.
+// One thread per atom i (caller's order; sorted index s): the force with the chain-rule terms of the covalent entries it
+// carries (+t) and of those it is the partner of (-t), and its rows of the sums.
+template<bool STRAIN, bool BATCH>
+__global__ void __launch_bounds__(kFinalChunk) kFinal(FinalArgs a) {
+    constexpr int NW = STRAIN ? kFinalWide : kFinalNarrow;
+    __shared__ double smem[kFinalChunk/64][NW];
+    const int lo = a.chunkStart[blockIdx.x], hi = a.chunkStart[blockIdx.x+1];
+    const int i = lo+(int) threadIdx.x;
+    double acc[NW];
+#pragma unroll
+    for (int q = 0; q < NW; q++)
+        acc[q] = 0;
+    if (i < hi) {
+        const BoxT<double> box = selectBox<BATCH>(a.box, i);
+        const int s = a.rank[i];
+        double dv[3], er[3], f[3], t[3], v[3];
+        const double al = a.alpha[s];
 #pragma unroll
         for (int k = 0; k < 3; k++) {
-            f[k] += t[k];
-#pragma unroll
-            for (int b = 0; b < 3; b++)
-                S[3*k+b] += t[k]*v[b];
+            dv[k] = a.d[3*s+k];
+            er[k] = a.er[3*s+k];
+            f[k] = 0;
+            acc[1] += dv[k]*dv[k];
+            if (al > 0)
+                acc[2] += a.mu[3*s+k]*a.mu[3*s+k]/(2.0*al);
         }
-    }
-    for (int e = revStart[i]; e < revStart[i+1]; e++) {
-        covalentTerm(revEntry[e], covAtomOf, covPartner, covStrength, pos, rank, etot, box, t, v);
+        if (a.gvdw)
+            acc[3] = a.gvdw[s];
+        if (STRAIN) {
+            const double* row = a.pairRows+10*(size_t) s;
+            acc[0] = row[0];
 #pragma unroll
-        for (int k = 0; k < 3; k++)
-            f[k] -= t[k];
-    }
+            for (int q = 0; q < 9; q++) {
+                acc[4+q] = row[1+q];
+                acc[13+q] = er[q/3]*dv[q%3];
+            }
+        }
+        else
+            acc[0] = a.pairRows[s];
+        for (int m = a.covStart[i]; m < a.covStart[i+1]; m++) {
+            covalentTerm(m, a, box, t, v);
 #pragma unroll
-    for (int k = 0; k < 3; k++)
-        fcov[3*i+k] = f[k];
+            for (int k = 0; k < 3; k++) {
+                f[k] += t[k];
+                if (STRAIN)
 #pragma unroll
-    for (int q = 0; q < 9; q++)
-        perAtom[9*(size_t) i+q] = S[q];
-}
-
-__global__ void kForcesOut(int n, const int* rank, const double* fpair, const double* frec, const double* fcov,
-                           double ke, double* fOut, long long* fixedOut, int stride, double fixedScale,
-                           const int* guard) {
-    const int i = blockIdx.x*blockDim.x+threadIdx.x;
-    if (i >= n || (guard && *guard == 0))
-        return;
-    const int s = rank[i];
+                    for (int b = 0; b < 3; b++)
+                        acc[22+3*k+b] += t[k]*v[b];
+            }
+        }
+        for (int e = a.revStart[i]; e < a.revStart[i+1]; e++) {
+            covalentTerm(a.revEntry[e], a, box, t, v);
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-        const double f = ke*(fpair[3*s+k]+frec[3*s+k]+fcov[3*i+k]);
-        if (fOut)
-            fOut[3*i+k] += f;
-        if (fixedOut)
-            atomicAdd(reinterpret_cast<unsigned long long*>(fixedOut+i+(size_t) k*stride),
-                      (unsigned long long) llrint(f*fixedScale));
-    }
-}
-
-__global__ void __launch_bounds__(256) kReducePartials(const double* partials, int nblk, int width, double* out) {
-    __shared__ double smem[40];
-    for (int q = 0; q < width; q++) {
-        double v = 0;
-        for (int b = threadIdx.x; b < nblk; b += blockDim.x)
-            v += partials[(size_t) b*width+q];
-        v = blockSum(v, smem);
-        if (threadIdx.x == 0)
-            out[q] = v;
-    }
-}
-
-// Every column of a range of rows in one pass: per-thread sums of its rows, then one wavefront reduction per
-// column and one barrier (a reduction per column, each with its barriers, made the final phase's sums slow).
-constexpr int kMaxSumWidth = 12;
-
-__global__ void __launch_bounds__(256) kRangeSums(const double* rows, int width, const int* starts,
-                                                  const int* outIndex, int outStride, double* out) {
-    __shared__ double smem[4][kMaxSumWidth];
-    const int r = blockIdx.x;
-    const int lo = starts[r], hi = starts[r+1];
-    const int orow = outIndex ? outIndex[r] : r;
-    double acc[kMaxSumWidth];
+            for (int k = 0; k < 3; k++)
+                f[k] -= t[k];
+        }
+        const bool add = !a.shortOf.cg || a.shortOf();
 #pragma unroll
-    for (int q = 0; q < kMaxSumWidth; q++)
-        acc[q] = 0.0;
-    for (int k = lo+threadIdx.x; k < hi; k += blockDim.x) {
-        const double* row = rows+(size_t) k*width;
-#pragma unroll
-        for (int q = 0; q < kMaxSumWidth; q++)
-            if (q < width)
-                acc[q] += row[q];
+        for (int k = 0; k < 3; k++) {
+            const double w = a.ke*(a.fpair[3*s+k]+a.frec[3*s+k]+f[k]);
+            if (a.fAssign)
+                a.fAssign[3*i+k] = w;
+            if (a.fOut && add)
+                a.fOut[3*i+k] += w;
+            if (a.fixedOut && add)
+                atomicAdd(reinterpret_cast<unsigned long long*>(a.fixedOut+i+(size_t) k*a.stride),
+                          (unsigned long long) llrint(w*a.fixedScale));
+            if (a.posKeep)
+                a.posKeep[3*i+k] = a.pos[3*i+k];
+        }
     }
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
-    for (int q = 0; q < kMaxSumWidth; q++) {
+    for (int q = 0; q < NW; q++) {
         const double v = groupSum<64>(acc[q]);
-        if (lane == 0 && q < width)
+        if (lane == 0)
             smem[w][q] = v;
     }
     __syncthreads();
-    if ((int) threadIdx.x < width) {
-        double v = 0.0;
-        for (int k = 0; k < (int) (blockDim.x >> 6); k++)
+    if (threadIdx.x < NW) {
+        double v = 0;
+        for (int k = 0; k < kFinalChunk/64; k++)
             v += smem[k][threadIdx.x];
-        out[(size_t) orow*outStride+threadIdx.x] = v;
+        a.chunkSums[(size_t) blockIdx.x*NW+threadIdx.x] = v;
     }
+}
+
+// One block per system: the chunks' columns and the x pass's (energy, strain) columns into its result slots.
+constexpr int kSumBlock = 512;
+
+template<bool STRAIN>
+__global__ void __launch_bounds__(kSumBlock) kFinalSums(const double* chunkSums, const int* sysChunk,
+                                                        const double* recRows, const int* recStart,
+                                                        const int* sysRec, double* res, int resStride) {
+    constexpr int NW = STRAIN ? kFinalWide : kFinalNarrow, NR = STRAIN ? 10 : 1;
+    __shared__ double smem[kSumBlock/64][NW+NR];
+    const int y = blockIdx.x, r = sysRec[y];
+    double acc[NW+NR];
+#pragma unroll
+    for (int q = 0; q < NW+NR; q++)
+        acc[q] = 0;
+    for (int k = sysChunk[y]+(int) threadIdx.x; k < sysChunk[y+1]; k += kSumBlock)
+#pragma unroll
+        for (int q = 0; q < NW; q++)
+            acc[q] += chunkSums[(size_t) k*NW+q];
+    for (int k = recStart[r]+(int) threadIdx.x; k < recStart[r+1]; k += kSumBlock)
+#pragma unroll
+        for (int q = 0; q < NR; q++)
+            acc[NW+q] += recRows[(size_t) k*10+q];
+#pragma unroll
+    for (int q = 0; q < NW+NR; q++) {
+        const double v = groupSum<64>(acc[q]);
+        if ((threadIdx.x & 63) == 0)
+            smem[threadIdx.x >> 6][q] = v;
+    }
+    __syncthreads();
+    const int q = threadIdx.x;
+    if (q >= NW+NR)
+        return;
+    double v = 0;
+    for (int w = 0; w < kSumBlock/64; w++)
+        v += smem[w][q];
+    const int slot = q >= NW ? kResRec+q-NW : q == 0 ? kResPair : q < 3 ? kResComb+q-1 : q == 3 ? kResGvdw
+                     : q < 13 ? kResPair+1+q-4 : q < 22 ? kResComb+2+q-13 : kResCov+q-22;
+    res[(size_t) y*resStride+slot] = v;
 }
 
 // The operands of a field evaluation of given charges q and dipoles d (caller's order): the sorted charges into
@@ -539,11 +619,13 @@ __global__ void kUnsort3(int n, const int* rank, const double* v, double* out) {
 
 }   // namespace
 
-int cgBlocks(int n) { return std::max(1, std::min(kCgMaxBlocks, nblk(3LL*n, kCgBlock))); }
+int cgBlocks(int n) { return std::max(1, std::min(kCgMaxBlocks, nblk(n, kCgBlock))); }
 
+template<class T>
 void launchGuess(hipStream_t st, int n, const int* order, const int* gidx, const double* hist, size_t slotStride,
-                 GuessCoef gc, const double* alpha, const double* b, double* x) {
-    kGuess<<<nblk(3LL*n, 256), 256, 0, st>>>(n, order, gidx, hist, slotStride, gc, alpha, b, x);
+                 GuessCoef gc, const double* alpha, CgRhs rhs, double cself, double* bOut, double* x,
+                 typename Vec4<T>::type* xT, const T* rgw) {
+    kGuess<T><<<nblk(n, 256), 256, 0, st>>>(n, order, gidx, hist, slotStride, gc, alpha, rhs, cself, bOut, x, xT, rgw);
 }
 
 void launchCombineB(hipStream_t st, int n, const double* ed, RecField er, const double* perm, double cself,
@@ -557,33 +639,40 @@ void launchToVec4(hipStream_t st, int n, const double* v, typename Vec4<T>::type
 }
 
 template<class T>
-void launchCgInit(hipStream_t st, int n, const double* alpha, const double* b, const double* x, const double* td,
-                  RecField tr, double cself, double tol, int maxIter, double* r, double* z, double* p,
-                  typename Vec4<T>::type* pT, double* partials, CgState* cg, int* done, Precond pc, const T* rgw) {
+void launchCgInit(hipStream_t st, int n, const double* alpha, CgRhs rhs, const double* x, const double* td,
+                  RecField tr, double cself, double* r, double* p,
+                  typename Vec4<T>::type* pT, double* partials, double* cg, Precond pc, const T* rgw) {
     const int nb = cgBlocks(n);
-    kCgInit<T><<<nb, kCgBlock, 0, st>>>(n, alpha, b, x, td, tr, cself, r, z, p, pT, partials, pc, rgw);
-    kCgInitCheck<<<1, kCgBlock, 0, st>>>(n, nb, tol, maxIter, partials, cg, done);
+    kCgInit<T><<<nb, kCgBlock, 0, st>>>(n, alpha, rhs, x, td, tr, cself, r, p, pT, partials, pc, rgw);
+    kCgInitCheck<<<1, kCgBlock, 0, st>>>(n, nb, partials, cg);
 }
 
-void launchCgAp(hipStream_t st, int n, int it, const double* alpha, const double* p, const double* td, RecField tr,
-                double cself, double* ap, double* partials, const int* done) {
-    kCgAp<<<cgBlocks(n), kCgBlock, 0, st>>>(n, alpha, p, td, tr, cself, ap, partials, done+it);
+void launchCgAp(hipStream_t st, int n, int it, const double* alpha, const double* p, const double* r, const double* td,
+                RecField tr, double cself, double* ap, double* partials, double* cg, CgSkip skip, Precond pc) {
+    kCgAp<<<cgBlocks(n), kCgBlock, 0, st>>>(n, it, alpha, p, r, td, tr, cself, ap, partials, cg, skip, pc);
+}
+
+template<class T>
+void launchCgStep(hipStream_t st, int n, int it, const double* alpha, const double* ap, double* x, double* r,
+                  double* p, typename Vec4<T>::type* pT, double* partials, double* cg, CgSkip skip, Precond pc,
+                  const T* rgw) {
+    kCgStep<T><<<cgBlocks(n), kCgBlock, 0, st>>>(n, it, alpha, ap, x, r, p, pT, partials, cg, skip, pc, rgw);
 }
 
 void launchCgUpdate(hipStream_t st, int n, int it, const double* alpha, const double* p, const double* ap, double* x,
-                    double* r, double* z, double* partials, const int* done, Precond pc) {
-    kCgUpdate<<<cgBlocks(n), kCgBlock, 0, st>>>(n, it, alpha, p, ap, x, r, z, partials, done+it, pc);
+                    double* r, double* partials, double* cg, CgSkip skip) {
+    kCgUpdate<<<cgBlocks(n), kCgBlock, 0, st>>>(n, it, alpha, p, ap, x, r, partials, cg, skip);
 }
 
 template<class T>
 void launchPrecond(hipStream_t st, int n, int it, bool init, const double* alpha, const double* r, const double* ap,
                    const typename Vec4<T>::type* pos, BoxSel<T> box, const int* srCount, const int* srJ,
                    const typename Vec2<T>::type* srG, const int* over, double* z, double* p,
-                   typename Vec4<T>::type* pT, double* partials, const int* done, const T* rgw) {
+                   typename Vec4<T>::type* pT, double* partials, CgSkip skip, const T* rgw) {
     const int nb = cgBlocks(n);
     auto go = [&](auto I, auto B) {
         kPrecond<T, I(), B()><<<nb, kCgBlock, 0, st>>>(n, it, alpha, r, ap, pos, box, srCount, srJ, srG, over, z, p,
-                                                       pT, partials, done+it, rgw);
+                                                       pT, partials, skip, rgw);
     };
     const bool b = box.table != nullptr;
     if (init)
@@ -593,9 +682,9 @@ void launchPrecond(hipStream_t st, int n, int it, bool init, const double* alpha
 }
 
 template<class T>
-void launchCgDirection(hipStream_t st, int n, int it, double tol, int maxIter, const double* z, double* p,
-                       typename Vec4<T>::type* pT, double* partials, CgState* cg, int* done, const T* rgw) {
-    kCgDirection<T><<<cgBlocks(n), kCgBlock, 0, st>>>(n, it, tol, maxIter, z, p, pT, partials, cg, done, rgw);
+void launchCgDirection(hipStream_t st, int n, int it, const double* z, double* p, typename Vec4<T>::type* pT,
+                       double* partials, CgSkip skip, const T* rgw) {
+    kCgDirection<T><<<cgBlocks(n), kCgBlock, 0, st>>>(n, it, z, p, pT, partials, skip, rgw);
 }
 
 template<class T>
@@ -605,42 +694,21 @@ void launchPost(hipStream_t st, int n, double peek, const double* alpha, const d
     kPost<T><<<nblk(n, 256), 256, 0, st>>>(n, peek, alpha, r, x, perm, order, gidx, hist, d, rgS, dT);
 }
 
-void launchFinalCombine(hipStream_t st, int n, const double* d, const double* mu, const double* alpha,
-                        const double* edir, const double* erec, double cself, double* etot, double* perAtom) {
-    kFinalCombine<<<nblk(n, kCgBlock), kCgBlock, 0, st>>>(n, d, mu, alpha, edir, erec, cself, etot, perAtom);
-}
-
-void launchCovalentForces(hipStream_t st, int n, const int* rank, const double* pos, const int* covStart,
-                          const int* covPartner, const double* covStrength, const int* revStart, const int* revEntry,
-                          const int* covAtomOf, const double* etot, BoxSel<double> box, double* fcov,
-                          double* perAtom) {
-    if (box.table)
-        kCovalent<true><<<nblk(n, kCgBlock), kCgBlock, 0, st>>>(n, rank, pos, covStart, covPartner, covStrength,
-                                                                revStart, revEntry, covAtomOf, etot, box, fcov,
-                                                                perAtom);
+void launchFinal(hipStream_t st, const FinalArgs& a, int nchunks, bool strain) {
+    auto go = [&](auto S, auto B) { kFinal<S(), B()><<<nchunks, kFinalChunk, 0, st>>>(a); };
+    const bool b = a.box.table != nullptr;
+    if (strain)
+        b ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
     else
-        kCovalent<false><<<nblk(n, kCgBlock), kCgBlock, 0, st>>>(n, rank, pos, covStart, covPartner, covStrength,
-                                                                 revStart, revEntry, covAtomOf, etot, box, fcov,
-                                                                 perAtom);
+        b ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
 }
 
-void launchForcesOut(hipStream_t st, int n, const int* rank, const double* fpair, const double* frec,
-                     const double* fcov, double ke, double* fOut, long long* fixedOut, int stride, double fixedScale,
-                     const int* guard) {
-    kForcesOut<<<nblk(n, 256), 256, 0, st>>>(n, rank, fpair, frec, fcov, ke, fOut, fixedOut, stride, fixedScale,
-                                             guard);
-}
-
-void launchReducePartials(hipStream_t st, const double* partials, int nblk_, int width, double* out) {
-    kReducePartials<<<1, 256, 0, st>>>(partials, nblk_, width, out);
-}
-
-void launchRangeSums(hipStream_t st, const double* rows, int width, const int* starts, int nr, const int* outIndex,
-                     int outStride, double* out) {
-    if (width < 1 || width > kMaxSumWidth)
-        throw std::logic_error("pgm_hip: range sums of more than 12 columns");
-    if (nr > 0)
-        kRangeSums<<<nr, 256, 0, st>>>(rows, width, starts, outIndex, outStride, out);
+void launchFinalSums(hipStream_t st, const double* chunkSums, bool strain, const int* sysChunk, int nsys,
+                     const double* recRows, const int* recStart, const int* sysRec, double* res, int resStride) {
+    if (strain)
+        kFinalSums<true><<<nsys, kSumBlock, 0, st>>>(chunkSums, sysChunk, recRows, recStart, sysRec, res, resStride);
+    else
+        kFinalSums<false><<<nsys, kSumBlock, 0, st>>>(chunkSums, sysChunk, recRows, recStart, sysRec, res, resStride);
 }
 
 template<class T>
@@ -656,15 +724,19 @@ void launchUnsort3(hipStream_t st, int n, const int* rank, const double* v, doub
 #define PGM_INSTANTIATE_SOLVER(T)                                                                                     \
     template void launchFieldOperands<T>(hipStream_t, int, const int*, const double*, const double*, const T*,      \
                                          double4*, Vec4<T>::type*, double*, Vec4<T>::type*);                          \
+    template void launchGuess<T>(hipStream_t, int, const int*, const int*, const double*, size_t, GuessCoef,         \
+                                 const double*, CgRhs, double, double*, double*, Vec4<T>::type*, const T*);          \
     template void launchToVec4<T>(hipStream_t, int, const double*, Vec4<T>::type*, const T*);                       \
-    template void launchCgInit<T>(hipStream_t, int, const double*, const double*, const double*, const double*,     \
-                                  RecField, double, double, int, double*, double*, double*, Vec4<T>::type*,         \
-                                  double*, CgState*, int*, Precond, const T*);                                       \
+    template void launchCgInit<T>(hipStream_t, int, const double*, CgRhs, const double*, const double*, RecField,    \
+                                  double, double*, double*, Vec4<T>::type*, double*, double*, Precond,               \
+                                  const T*);                                                                \
+    template void launchCgStep<T>(hipStream_t, int, int, const double*, const double*, double*, double*, double*,    \
+                                  Vec4<T>::type*, double*, double*, CgSkip, Precond, const T*);             \
     template void launchPrecond<T>(hipStream_t, int, int, bool, const double*, const double*, const double*,         \
                                    const Vec4<T>::type*, BoxSel<T>, const int*, const int*, const Vec2<T>::type*,     \
-                                   const int*, double*, double*, Vec4<T>::type*, double*, const int*, const T*);     \
-    template void launchCgDirection<T>(hipStream_t, int, int, double, int, const double*, double*, Vec4<T>::type*,  \
-                                       double*, CgState*, int*, const T*);                                           \
+                                   const int*, double*, double*, Vec4<T>::type*, double*, CgSkip, const T*);         \
+    template void launchCgDirection<T>(hipStream_t, int, int, const double*, double*, Vec4<T>::type*, double*,       \
+                                       CgSkip, const T*);                                                             \
     template void launchPost<T>(hipStream_t, int, double, const double*, const double*, double*, const double*,     \
                                 const int*, const int*, double*, double*, const double*, Vec4<T>::type*);
 PGM_INSTANTIATE_SOLVER(float)
