@@ -64,8 +64,6 @@ struct PairPrec<double> {
     static constexpr double kDampCut = 6.0;
 };
 
-__device__ __forceinline__ float erfcT(float x) { return erfcf(x); }
-__device__ __forceinline__ double erfcT(double x) { return erfc(x); }
 __device__ __forceinline__ float erfT(float x) { return erff(x); }
 __device__ __forceinline__ double erfT(double x) { return erf(x); }
 __device__ __forceinline__ float expT(float x) { return __expf(x); }
@@ -119,41 +117,87 @@ __device__ __forceinline__ void erfSeries(T a, T s, T* B) {
     }
 }
 
-// B_n of erf(a r)/r by the closed-form upward recursion (s >= 1), or by the series below.
-template<class T, int NMAX>
-__device__ __forceinline__ void erfKernels(T a, T r, T ir2, T* B) {
-    const T x = a*r, s = x*x;
-    if (s < T(1)) {
-        erfSeries<T, NMAX>(a, s, B);
-        return;
-    }
-    const T g = T(kTwoOverSqrtPi)*a*expT(-s);
-    B[0] = erfT(x)/r;
-    T scale = T(1);
-    const T twoA2 = T(2)*a*a;
+// FP64 building blocks of the pair kernels, without library calls, divisions or square roots (one of the library's erfc,
+// exp, sqrt or divide is 20 to 100 instructions with range branches, and a pair needs seven of them).
+// 1/sqrt(v), v > 0: v_rsq_f64 and one third-order step, within 1 ulp.
+__device__ __forceinline__ double rsqD(double v) {
+    const double y = __builtin_amdgcn_rsq(v), e = fma(-v*y, y, 1.0);
+    return fma(y*e, fma(0.375, e, 0.5), y);
+}
+// 1/v: v_rcp_f64 and one third-order step.
+__device__ __forceinline__ double rcpD(double v) {
+    const double y = __builtin_amdgcn_rcp(v), e = fma(-v, y, 1.0);
+    return fma(y, fma(e, e, e), y);
+}
+// exp(-(s + lo)), s >= 0, |lo| << 1: 2^n e^r, |r| <= ln 2 / 2, the Taylor terms to r^2 exact and a degree-8 polynomial
+// (interpolation at Chebyshev nodes, 3.4e-17) for the rest.
+__device__ __forceinline__ double expNegD(double s, double lo) {
+    const double k = rint(s*-1.44269504088896339);
+    const double r = fma(k, -2.31904681384629956e-17, fma(k, -6.93147180559945286e-01, -s)-lo);
+    double p = 2.51003765231722297e-08;
+    p = fma(p, r, 2.76137965905202207e-07);
+    p = fma(p, r, 2.75572684786510166e-06);
+    p = fma(p, r, 2.48015364068864706e-05);
+    p = fma(p, r, 1.98412698630417918e-04);
+    p = fma(p, r, 1.38888889058726541e-03);
+    p = fma(p, r, 8.33333333333006500e-03);
+    p = fma(p, r, 4.16666666666513641e-02);
+    p = fma(p, r, 1.66666666666666685e-01);
+    p = fma(p, r, 0.5);
+    p = fma(p, r, 1.0);
+    p = fma(p, r, 1.0);
+    return __builtin_amdgcn_ldexp(p, (int) k);
+}
+// exp(x^2) erfc(x) for x >= 0: P(u)/(x + K), u = (x - K)/(x + K), K = 2.5, the Chebyshev expansion of
+// (x + K) exp(x^2) erfc(x) in u to degree 24 (remainder 1e-16 at most; the mapping of Shepherd and Laframboise, Math.
+// Comp. 36, 249, 1981), 4.5e-16 evaluated in FP64.
+__device__ __forceinline__ double erfcxD(double x) {
+    const double t = rcpD(x+2.5), u = (x-2.5)*t;
+    double p = -1.13943375763050212e-09;
+    p = fma(p, u, -3.46738851456642846e-11);
+    p = fma(p, u, 1.13616654610778355e-08);
+    p = fma(p, u, 6.46203952133591332e-09);
+    p = fma(p, u, -5.36892735908146752e-08);
+    p = fma(p, u, -7.41995606534354225e-08);
+    p = fma(p, u, 1.39210995565696456e-07);
+    p = fma(p, u, 4.54263266929759196e-07);
+    p = fma(p, u, -6.74541909340868799e-09);
+    p = fma(p, u, -1.96813742087781588e-06);
+    p = fma(p, u, -2.33199485288660954e-06);
+    p = fma(p, u, 6.75738056042995359e-06);
+    p = fma(p, u, 1.82443088002155857e-05);
+    p = fma(p, u, -1.95333384577758414e-05);
+    p = fma(p, u, -1.12604824560452857e-04);
+    p = fma(p, u, 5.83080587353616042e-05);
+    p = fma(p, u, 7.02693723353389125e-04);
+    p = fma(p, u, -4.39208300105815538e-04);
+    p = fma(p, u, -4.81878552320537737e-03);
+    p = fma(p, u, 8.39304430476217091e-03);
+    p = fma(p, u, 2.83615501319947304e-02);
+    p = fma(p, u, -1.71251145246119035e-01);
+    p = fma(p, u, 4.53914116648096055e-01);
+    p = fma(p, u, -8.04651849439148137e-01);
+    p = fma(p, u, 1.05403182030571796e+00);
+    return p*t;
+}
+
+// B_n of erfc(c r)/r (SIGN = 1) or erf(c r)/r (-1) by the upward recursion, from s = (c r)^2 with its rounding error lo,
+// 1/r and 1/r^2: for erfc all terms are positive (core/pgm_math.h:63-71), for erf s >= 1.
+template<int SIGN, int NMAX>
+__device__ __forceinline__ void gaussKernelsD(double c, double s, double lo, double r, double rinv, double ir2,
+                                              double* B) {
+    const double e = expNegD(s, lo), erfcV = erfcxD(c*r)*e;
+    const double g = kTwoOverSqrtPi*c*e, twoC2 = 2.0*c*c;
+    B[0] = (SIGN > 0 ? erfcV : 1.0-erfcV)*rinv;
+    double scale = SIGN;
 #pragma unroll
     for (int k = 1; k < NMAX; k++) {
-        B[k] = (T(2*k-1)*B[k-1]-scale*g)*ir2;
-        scale *= twoA2;
+        B[k] = fma(double(2*k-1), B[k-1], scale*g)*ir2;
+        scale *= twoC2;
     }
 }
 
-// B_n of erfc(a r)/r: all terms positive (core/pgm_math.h:63-71).
-template<class T, int NMAX>
-__device__ __forceinline__ void erfcKernels(T a, T r, T ir2, T* B) {
-    const T x = a*r;
-    const T g = T(kTwoOverSqrtPi)*a*expT(-x*x);
-    B[0] = erfcT(x)/r;
-    T scale = T(1);
-    const T twoA2 = T(2)*a*a;
-#pragma unroll
-    for (int k = 1; k < NMAX; k++) {
-        B[k] = (T(2*k-1)*B[k-1]+scale*g)*ir2;
-        scale *= twoA2;
-    }
-}
-
-// FP32 forms of erfKernels / erfcKernels: 1/r from v_rsq, erfc(x) from erfcxFast(x) and the exp(-x^2) of the
+// B_n of erf(a r)/r and erfc(a r)/r in FP32: 1/r from v_rsq, erfc(x) from erfcxFast(x) and the exp(-x^2) of the
 // Gaussian term, no divisions.
 template<int NMAX>
 __device__ __forceinline__ void erfKernelsF(float a, float r, float rinv, float* B) {
@@ -191,7 +235,7 @@ __device__ __forceinline__ void erfcKernelsF(float a, float r, float rinv, float
     }
 }
 
-// G_n for FP32 from r^2 and rg_i + rg_j (a = (rg_i + rg_j)^-1/2): the branches of pairKernels below.
+// G_n for FP32 from r^2 and rg_i + rg_j (a = (rg_i + rg_j)^-1/2): the branches of pairKernelsD below.
 template<int NMAX>
 __device__ __forceinline__ void pairKernelsF(float rgSum, float beta, float r2, float* G) {
     const float a = __builtin_amdgcn_rsqf(rgSum);
@@ -244,24 +288,37 @@ __device__ __forceinline__ void g03FromG12(float G1, float G2, float r2, float r
     G3 = (5.0f*G2+tb*tb*hb-ta*ta*ha)*(rinv*rinv);
 }
 
-// G_n = B_n[erf(a r)/r] - B_n[erf(beta r)/r] for n in [N0, NMAX): the series difference for a r < 1, the erfc
-// form Bc(beta) - Bc(a) beyond (core/pgm_math.h:78-92), the Bc(a) part dropped beyond a r > kDampCut.
-template<class T, int NMAX>
-__device__ __forceinline__ void pairKernels(T a, T beta, T r, T* G) {
-    const T ir2 = T(1)/(r*r);
-    T B[NMAX];
-    if (a*r < T(1)) {
-        erfSeries<T, NMAX>(a, (a*r)*(a*r), G);
-        erfKernels<T, NMAX>(beta, r, ir2, B);
+// G_n = B_n[erf(a r)/r] - B_n[erf(beta r)/r] for n < NMAX in FP64, a = rgSum^-1/2: the series difference for a r < 1,
+// the erfc form Bc(beta) - Bc(a) beyond (core/pgm_math.h:78-92), the Bc(a) part dropped beyond a r > kDampCut.  The
+// exponents (c r)^2 carry their rounding error along, so that exp(-(c r)^2) is good to an ulp at every distance.
+// Against the library's functions the setup pass over 88 million pairs takes 1,403 us instead of
+// 1,552 (bound by its 32-byte stores then).
+template<int NMAX>
+__device__ __forceinline__ void pairKernelsD(double rgSum, double beta, double r2In, double* G) {
+    const double r2 = fmax(r2In, 1e-280);   // coincident atoms: r = 0 in the series
+    const double a = rsqD(rgSum), rinv = rsqD(r2), r = r2*rinv;
+    double ir2 = rinv*rinv;
+    ir2 = fma(ir2, fma(-r2, ir2, 1.0), ir2);
+    const double b2 = beta*beta, b2Lo = fma(beta, beta, -b2);
+    const double sb = b2*r2, sbLo = fma(b2, r2, -sb)+b2Lo*r2;
+    double B[NMAX];
+    if (a*r < 1.0) {
+        erfSeries<double, NMAX>(a, (a*r)*(a*r), G);
+        if (sb < 1.0)
+            erfSeries<double, NMAX>(beta, sb, B);
+        else
+            gaussKernelsD<-1, NMAX>(beta, sb, sbLo, r, rinv, ir2, B);
     }
     else {
-        erfcKernels<T, NMAX>(beta, r, ir2, G);
-        if (a*r < PairPrec<T>::kDampCut)
-            erfcKernels<T, NMAX>(a, r, ir2, B);
+        gaussKernelsD<1, NMAX>(beta, sb, sbLo, r, rinv, ir2, G);
+        if (a*r < PairPrec<double>::kDampCut) {
+            const double a2 = a*a, sa = r2*a2;
+            gaussKernelsD<1, NMAX>(a, sa, fma(-sa, rgSum, r2)*a2, r, rinv, ir2, B);
+        }
         else {
 #pragma unroll
             for (int k = 0; k < NMAX; k++)
-                B[k] = T(0);
+                B[k] = 0;
         }
     }
 #pragma unroll

@@ -37,7 +37,7 @@ __global__ void kEvalPair(int n, int precision, const double* rgSum, const doubl
     }
     else {
         double G[4];
-        pairKernels<double, 4>(rsqrt(rgSum[i]), beta, sqrt(r2[i]), G);
+        pairKernelsD<4>(rgSum[i], beta, r2[i], G);
         for (int k = 0; k < 4; k++)
             o[k] = G[k];
         o[4] = G[0];

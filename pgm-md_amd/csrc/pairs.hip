@@ -86,7 +86,7 @@ __device__ __forceinline__ void setupTerm(const typename Vec4<T>::type& pi, T rg
     if constexpr (sizeof(T) == sizeof(float))
         pairKernelsF<4>(rgi+rgj, beta, x*x+y*y+z*z, G);
     else
-        pairKernels<T, 4>(rsqrtT(rgi+rgj), beta, sqrt(x*x+y*y+z*z), G);
+        pairKernelsD<4>(rgi+rgj, beta, x*x+y*y+z*z, G);
     const T c = pjv.w*G[1]+(d.x*x+d.y*y+d.z*z)*G[2];
     e[0] += (double) (c*x-d.x*G[1]);
     e[1] += (double) (c*y-d.y*G[1]);
@@ -112,7 +112,7 @@ __device__ __forceinline__ void setupTermX(T x, T y, T z, T qj, T rgSum, const t
     if constexpr (sizeof(T) == sizeof(float))
         pairKernelsF<4>(rgSum, beta, x*x+y*y+z*z, G);
     else
-        pairKernels<T, 4>(rsqrtT(rgSum), beta, sqrt(x*x+y*y+z*z), G);
+        pairKernelsD<4>(rgSum, beta, x*x+y*y+z*z, G);
     const T c = qj*G[1]+(d.x*x+d.y*y+d.z*z)*G[2];
     e[0] += (double) (c*x-d.x*G[1]);
     e[1] += (double) (c*y-d.y*G[1]);
