@@ -94,27 +94,53 @@ __device__ __forceinline__ float erfcxFast(float x) {
 // of x^2 in the exponent dominates near x = 4.5).
 __device__ __forceinline__ float erfcFast(float x) { return erfcxFast(x)*__expf(-x*x); }
 
+// A polynomial in FP64, C::at(k) its coefficients from the highest degree down.  Each comes from scalar registers, tied
+// to the accumulator so that it is set right before its step: left to itself the compiler keeps the coefficients in
+// vector registers through the pair loops and copies each into the accumulator first (the passes at 200 registers, two
+// wavefronts per SIMD, two vector instructions per step).
+template<int N, class C>
+__device__ __forceinline__ double hornerD(double x) {
+    double p = C::at(0);
+#pragma unroll
+    for (int k = 1; k < N; k++) {
+        double c = C::at(k);
+        asm("" : "+s"(c) : "v"(p));
+        p = fma(p, x, c);
+    }
+    return p;
+}
+
+// 1/(m! (2m+2k+1)) and its sign in the series below.
+constexpr double erfSeriesCoef(int m, int k) {
+    double f = (m & 1) ? -1.0 : 1.0;
+    for (int i = 2; i <= m; i++)
+        f /= i;
+    return f/(2*m+2*k+1);
+}
+
+template<int K>
+struct ErfSeriesD {
+    __device__ static constexpr double at(int k) { return erfSeriesCoef(PairPrec<double>::kSeries-1-k, K); }
+};
+
 // B_n of erf(a r)/r, n < NMAX, by the series in s = (a r)^2 (valid for s < 1; no cancellation at short
 // range): B_n = (2a/sqrt(pi)) (2a^2)^n sum_m (-s)^m / (m! (2m+2n+1)) (core/pgm_math.h:31-49, docs/spec.md Sec. 4).
-template<class T, int NMAX>
-__device__ __forceinline__ void erfSeries(T a, T s, T* B) {
+template<class T, int NMAX, int K = 0>
+__device__ __forceinline__ void erfSeries(T a, T s, T* B, T scale = T(1)) {
     constexpr int NS = PairPrec<T>::kSeries;
-    T term[NS];
-    term[0] = T(1);
+    if constexpr (K == 0)
+        scale = T(kTwoOverSqrtPi)*a;
+    if constexpr (sizeof(T) == sizeof(double))
+        B[K] = scale*hornerD<NS, ErfSeriesD<K>>(s);
+    else {
+        T acc = T(erfSeriesCoef(NS-1, K));
 #pragma unroll
-    for (int m = 1; m < NS; m++)
-        term[m] = -term[m-1]*s*(T(1)/T(m));
-    T scale = T(kTwoOverSqrtPi)*a;
-    const T twoA2 = T(2)*a*a;
-#pragma unroll
-    for (int k = 0; k < NMAX; k++) {
-        T acc = T(0);
-#pragma unroll
-        for (int m = NS-1; m >= 0; m--)
-            acc += term[m]*(T(1)/T(2*m+2*k+1));
-        B[k] = scale*acc;
-        scale *= twoA2;
+        for (int m = NS-2; m >= 0; m--)
+            acc = fma(acc, s, T(erfSeriesCoef(m, K)));
+        B[K] = scale*acc;
     }
+    if constexpr (K+1 < NMAX)
+        erfSeries<T, NMAX, K+1>(a, s, B, scale*(T(2)*a*a));
 }
 
 // FP64 building blocks of the pair kernels, without library calls, divisions or square roots (one of the library's erfc,
@@ -129,56 +155,49 @@ __device__ __forceinline__ double rcpD(double v) {
     const double y = __builtin_amdgcn_rcp(v), e = fma(-v, y, 1.0);
     return fma(y, fma(e, e, e), y);
 }
+struct ExpD {
+    __device__ static constexpr double at(int k) {
+        constexpr double c[12] = {
+            2.51003765231722297e-08, 2.76137965905202207e-07, 2.75572684786510166e-06, 2.48015364068864706e-05,
+            1.98412698630417918e-04, 1.38888889058726541e-03, 8.33333333333006500e-03, 4.16666666666513641e-02,
+            1.66666666666666685e-01, 0.5, 1.0, 1.0,
+        };
+        return c[k];
+    }
+};
 // exp(-(s + lo)), s >= 0, |lo| << 1: 2^n e^r, |r| <= ln 2 / 2, the Taylor terms to r^2 exact and a degree-8 polynomial
 // (interpolation at Chebyshev nodes, 3.4e-17) for the rest.
 __device__ __forceinline__ double expNegD(double s, double lo) {
     const double k = rint(s*-1.44269504088896339);
     const double r = fma(k, -2.31904681384629956e-17, fma(k, -6.93147180559945286e-01, -s)-lo);
-    double p = 2.51003765231722297e-08;
-    p = fma(p, r, 2.76137965905202207e-07);
-    p = fma(p, r, 2.75572684786510166e-06);
-    p = fma(p, r, 2.48015364068864706e-05);
-    p = fma(p, r, 1.98412698630417918e-04);
-    p = fma(p, r, 1.38888889058726541e-03);
-    p = fma(p, r, 8.33333333333006500e-03);
-    p = fma(p, r, 4.16666666666513641e-02);
-    p = fma(p, r, 1.66666666666666685e-01);
-    p = fma(p, r, 0.5);
-    p = fma(p, r, 1.0);
-    p = fma(p, r, 1.0);
+    const double p = hornerD<12, ExpD>(r);
     return __builtin_amdgcn_ldexp(p, (int) k);
 }
+// v^-1/2 and exp(-s) in the pair type.
+__device__ __forceinline__ float rsqT(float v) { return __frsqrt_rn(v); }
+__device__ __forceinline__ double rsqT(double v) { return rsqD(v); }
+__device__ __forceinline__ float expNegT(float s) { return __expf(-s); }
+__device__ __forceinline__ double expNegT(double s) { return expNegD(s, 0.0); }
+struct ErfcxD {
+    __device__ static constexpr double at(int k) {
+        constexpr double c[25] = {
+            -1.13943375763050212e-09, -3.46738851456642846e-11, 1.13616654610778355e-08, 6.46203952133591332e-09,
+            -5.36892735908146752e-08, -7.41995606534354225e-08, 1.39210995565696456e-07, 4.54263266929759196e-07,
+            -6.74541909340868799e-09, -1.96813742087781588e-06, -2.33199485288660954e-06, 6.75738056042995359e-06,
+            1.82443088002155857e-05, -1.95333384577758414e-05, -1.12604824560452857e-04, 5.83080587353616042e-05,
+            7.02693723353389125e-04, -4.39208300105815538e-04, -4.81878552320537737e-03, 8.39304430476217091e-03,
+            2.83615501319947304e-02, -1.71251145246119035e-01, 4.53914116648096055e-01, -8.04651849439148137e-01,
+            1.05403182030571796e+00,
+        };
+        return c[k];
+    }
+};
 // exp(x^2) erfc(x) for x >= 0: P(u)/(x + K), u = (x - K)/(x + K), K = 2.5, the Chebyshev expansion of
 // (x + K) exp(x^2) erfc(x) in u to degree 24 (remainder 1e-16 at most; the mapping of Shepherd and Laframboise, Math.
 // Comp. 36, 249, 1981), 4.5e-16 evaluated in FP64.
 __device__ __forceinline__ double erfcxD(double x) {
     const double t = rcpD(x+2.5), u = (x-2.5)*t;
-    double p = -1.13943375763050212e-09;
-    p = fma(p, u, -3.46738851456642846e-11);
-    p = fma(p, u, 1.13616654610778355e-08);
-    p = fma(p, u, 6.46203952133591332e-09);
-    p = fma(p, u, -5.36892735908146752e-08);
-    p = fma(p, u, -7.41995606534354225e-08);
-    p = fma(p, u, 1.39210995565696456e-07);
-    p = fma(p, u, 4.54263266929759196e-07);
-    p = fma(p, u, -6.74541909340868799e-09);
-    p = fma(p, u, -1.96813742087781588e-06);
-    p = fma(p, u, -2.33199485288660954e-06);
-    p = fma(p, u, 6.75738056042995359e-06);
-    p = fma(p, u, 1.82443088002155857e-05);
-    p = fma(p, u, -1.95333384577758414e-05);
-    p = fma(p, u, -1.12604824560452857e-04);
-    p = fma(p, u, 5.83080587353616042e-05);
-    p = fma(p, u, 7.02693723353389125e-04);
-    p = fma(p, u, -4.39208300105815538e-04);
-    p = fma(p, u, -4.81878552320537737e-03);
-    p = fma(p, u, 8.39304430476217091e-03);
-    p = fma(p, u, 2.83615501319947304e-02);
-    p = fma(p, u, -1.71251145246119035e-01);
-    p = fma(p, u, 4.53914116648096055e-01);
-    p = fma(p, u, -8.04651849439148137e-01);
-    p = fma(p, u, 1.05403182030571796e+00);
-    return p*t;
+    return hornerD<25, ErfcxD>(u)*t;
 }
 
 // B_n of erfc(c r)/r (SIGN = 1) or erf(c r)/r (-1) by the upward recursion, from s = (c r)^2 with its rounding error lo,
@@ -261,38 +280,11 @@ __device__ __forceinline__ void pairKernelsF(float rgSum, float beta, float r2, 
         G[k] -= B[k];
 }
 
-// G0 and G3 of a pair from its G1, G2 (FP32), by the recurrence of the erfc forms
-// Bc_{n+1}[c] = ((2n+1) Bc_n[c] + (2c^2)^n h_c)/r^2, h_c = (2c/sqrt(pi)) exp(-c^2 r^2), applied to
-// G_n = Bc_n[beta] - Bc_n[a]: G0 = r^2 G1 + h_a - h_beta, G3 = (5 G2 + (2 beta^2)^2 h_beta - (2a^2)^2 h_a)/r^2,
-// with h_a = 0 beyond the damping cut as in pairKernelsF.  Close pairs (a r < 1, the series branch, where the
-// upward recurrence would cancel) get all four kernels again from pairKernelsF.
-__device__ __forceinline__ void g03FromG12(float G1, float G2, float r2, float rgSum, float beta, float& G0,
-                                           float& G3);
-
-__device__ __forceinline__ void g03FromG12(float G1, float G2, float r2, float rgSum, float beta, float& G0,
-                                           float& G3) {
-    const float a = __builtin_amdgcn_rsqf(rgSum);
-    const float rinv = __builtin_amdgcn_rsqf(r2);
-    const float r = r2*rinv;
-    if (a*r < 1.0f) {
-        float G[4];
-        pairKernelsF<4>(rgSum, beta, r2, G);
-        G0 = G[0];
-        G3 = G[3];
-        return;
-    }
-    const float ha = a*r < PairPrec<float>::kDampCut ? float(kTwoOverSqrtPi)*a*__expf(-a*a*r2) : 0.0f;
-    const float hb = float(kTwoOverSqrtPi)*beta*__expf(-beta*beta*r2);
-    const float ta = 2.0f*a*a, tb = 2.0f*beta*beta;
-    G0 = r2*G1+ha-hb;
-    G3 = (5.0f*G2+tb*tb*hb-ta*ta*ha)*(rinv*rinv);
-}
-
 // G_n = B_n[erf(a r)/r] - B_n[erf(beta r)/r] for n < NMAX in FP64, a = rgSum^-1/2: the series difference for a r < 1,
 // the erfc form Bc(beta) - Bc(a) beyond (core/pgm_math.h:78-92), the Bc(a) part dropped beyond a r > kDampCut.  The
 // exponents (c r)^2 carry their rounding error along, so that exp(-(c r)^2) is good to an ulp at every distance.
-// Against the library's functions the setup pass over 88 million pairs takes 1,403 us instead of
-// 1,552 (bound by its 32-byte stores then).
+// Against the library's functions the setup pass over 88 million pairs took 1,403 us instead of 1,552, when it also
+// stored 32 bytes of kernels per pair.
 template<int NMAX>
 __device__ __forceinline__ void pairKernelsD(double rgSum, double beta, double r2In, double* G) {
     const double r2 = fmax(r2In, 1e-280);   // coincident atoms: r = 0 in the series

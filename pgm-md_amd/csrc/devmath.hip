@@ -17,8 +17,8 @@ __global__ void kEvalErfc(int n, const float* x, float* y) {
         y[i] = erfcFast(x[i]);
 }
 
-// out[i][0..3] = G0..G3 of the pair kernels; out[i][4..5] = G0, G3 as the FP32 final and tangent passes rebuild
-// them from G1, G2 (FP64: G0, G3 again).
+// out[i][0..3] = G0..G3 of the pair kernels; out[i][4..5] = G0, G3 as the final and tangent passes evaluate them (the
+// same code).
 __global__ void kEvalPair(int n, int precision, const double* rgSum, const double* r2, double beta, double* out) {
     const int i = blockIdx.x*blockDim.x+threadIdx.x;
     if (i >= n)
@@ -28,12 +28,10 @@ __global__ void kEvalPair(int n, int precision, const double* rgSum, const doubl
         float G[4];
         const float rs = (float) rgSum[i], q2 = (float) r2[i], b = (float) beta;
         pairKernelsF<4>(rs, b, q2, G);
-        float G0, G3;
-        g03FromG12(G[1], G[2], q2, rs, b, G0, G3);
         for (int k = 0; k < 4; k++)
             o[k] = G[k];
-        o[4] = G0;
-        o[5] = G3;
+        o[4] = G[0];
+        o[5] = G[3];
     }
     else {
         double G[4];

@@ -1082,7 +1082,7 @@ public:
             b->reserve(3*sizeof(double)*n);
         erD_.reserve(recBytes());
         nbD_.reserve(n*sizeof(int));
-        pairSetup<T>(setupLanes(), fused_, nullptr);
+        pairSetup<T>(setupLanes(), fused_, fieldOtf_, nullptr);
         pmeSolve<T>(permTD_.as<T4>(), true, posT<T>(), 0, false, erD_.as<double>(), nullptr, CgSkip{});
         const double cself = 4.0*s_.beta*s_.beta*s_.beta/(3.0*kSqrtPi);
         launchCombineB(st_, n, edD_.as<double>(), recField(erD_), permD_.as<double>(), cself, bD_.as<double>());
@@ -1278,6 +1278,8 @@ public:
     void setFieldOtf(bool on) {
         if (on && s_.precision != PGM_MIXED)
             throw std::invalid_argument("pgm_hip: the on-the-fly field pass is an FP32 (PGM_MIXED) variant");
+        if (on != fieldOtf_)
+            adjointReady_ = false;   // the state may lack the stored kernels: a backward evaluates again
         fieldOtf_ = on;
     }
     int lanes() const { return lanes_; }
@@ -2286,7 +2288,7 @@ private:
         candD_.reserve(cap*sizeof(int));
         pjD_.reserve(cap*sizeof(int));
         g12D_.reserve(cap*g2);
-        if (s_.precision == PGM_DOUBLE)   // the FP32 path rebuilds G0, G3 from G1, G2
+        if (s_.precision == PGM_DOUBLE)
             g03D_.reserve(cap*g2);
         for (const Sys& y : sys_) {
             const BoxT<double> bd = makeBox<double>(y.H, y.recip);
@@ -2614,20 +2616,20 @@ private:
     }
 
     // The candidates within rc, their kernels and the field of (q, perm) (and of dual): one fused pass or
-    // compaction + setup.
+    // compaction + setup.  The kernels are stored unless the field pass evaluates its own (otf).
     template<class T>
-    void pairSetup(int lanes, bool fused, const typename Vec4<T>::type* dual) {
+    void pairSetup(int lanes, bool fused, bool otf, const typename Vec4<T>::type* dual) {
         typedef typename Vec4<T>::type T4;
         typedef typename Vec2<T>::type T2;
         const BoxSel<T> bt = boxSel<T>();
         const T rc2 = (T) (s_.cutoff*s_.cutoff);
+        T2* g12 = otf ? nullptr : g12D_.as<T2>();
         listReverse_ = true;   // the setup writes the list forward: the next pass reads it from the end
         if (fused) {
             tb(kPhPairSetup);
             launchPairCompactSetup<T>(st_, n_, posT<T>(), rgT<T>(), permTD_.as<T4>(), dual, candStartD_.as<int>(),
-                                      candD_.as<int>(), nbD_.as<int>(), pjD_.as<int>(), g12D_.as<T2>(),
-                                      g03D_.as<T2>(), bt, rc2, (T) s_.beta, (T) rgMax_, edD_.as<double>(),
-                                      tdD_.as<double>(), lanes);
+                                      candD_.as<int>(), nbD_.as<int>(), pjD_.as<int>(), g12, g03D_.as<T2>(), bt, rc2,
+                                      (T) s_.beta, (T) rgMax_, edD_.as<double>(), tdD_.as<double>(), lanes);
             te();
             return;
         }
@@ -2637,7 +2639,7 @@ private:
         te();
         tb(kPhPairSetup);
         launchPairSetup<T>(st_, n_, posT<T>(), rgT<T>(), permTD_.as<T4>(), dual, candStartD_.as<int>(),
-                           nbD_.as<int>(), pjD_.as<int>(), g12D_.as<T2>(), g03D_.as<T2>(), bt, (T) s_.beta,
+                           nbD_.as<int>(), pjD_.as<int>(), g12, g03D_.as<T2>(), bt, (T) s_.beta,
                            edD_.as<double>(), tdD_.as<double>(), lanes);
         te();
     }
@@ -2763,17 +2765,17 @@ private:
         // passes, the autotuner's choice) + PME
         PmeStreamScope pmeScope(*this, overlapPme());
         fork();
-        pairSetup<T>(setupLanes(), fused_, dual ? pTD_.as<T4>() : nullptr);
+        pairSetup<T>(setupLanes(), fused_, fieldOtf_, dual ? pTD_.as<T4>() : nullptr);
         preReady_ = false;
-        if (induce && preRadius_ > 0) {   // the preconditioner's short list, from the stored kernels
+        if (induce && preRadius_ > 0) {   // the preconditioner's short list
             srCountD_.reserve(n*sizeof(int));
             srJD_.reserve((size_t) n*kPreCap*sizeof(int));
             srGD_.reserve((size_t) n*kPreCap*sizeof(T2));
             srOverD_.reserve(sizeof(int));
             tb(kPhCg);
             launchZero<int>(st_, srOverD_.as<int>(), 1, CgSkip{});
-            launchShortList<T>(st_, n, pos, candStartD_.as<int>(), nbD_.as<int>(), pjD_.as<int>(), g12D_.as<T2>(),
-                               bt, (T) (preRadius_*preRadius_), srCountD_.as<int>(), srJD_.as<int>(),
+            launchShortList<T>(st_, n, pos, candStartD_.as<int>(), nbD_.as<int>(), pjD_.as<int>(), rgT<T>(),
+                               (T) s_.beta, bt, (T) (preRadius_*preRadius_), srCountD_.as<int>(), srJD_.as<int>(),
                                srGD_.as<T2>(), srOverD_.as<int>());
             te();
             preReady_ = true;
@@ -2831,8 +2833,8 @@ private:
         tb(kPhPairFinal);
         const GvdwArgs<T> ga = gvdwArgs<T>();
         launchPairFinal<T>(st_, n, pos, dTD_.as<T4>(), rgT<T>(), (T) s_.beta, candStartD_.as<int>(), nbD_.as<int>(),
-                           pjD_.as<int>(), g12D_.as<T2>(), g03D_.as<T2>(), bt, fpairD_.as<double>(),
-                           edD_.as<double>(), perAtomD_.as<double>(), wantStrain, ga, lanes_, nextListDirection());
+                           pjD_.as<int>(), g12D_.as<T2>(), g03D_.as<T2>(), bt, fpairD_.as<double>(), edD_.as<double>(),
+                           perAtomD_.as<double>(), wantStrain, ga, lanes_, nextListDirection());
         if (ga.gv && nSkip_ > 0)
             launchGvdwSkip<T>(st_, n, orderD_.as<int>(), rankD_.as<int>(), pos, rgT<T>(), skipStartD_.as<int>(),
                               skipPartD_.as<int>(), bt, (T) (s_.cutoff*s_.cutoff), wantStrain, ga,
@@ -2924,10 +2926,10 @@ private:
         const bool wasTiming = timing_;
         timing_ = false;
         adjointReady_ = false;   // the timed passes overwrite the evaluation's pair-pass outputs
-        pairSetup<T>(lanes, fused, pTD_.as<T4>());   // warm-up
+        pairSetup<T>(lanes, fused, fieldOtf_, pTD_.as<T4>());   // warm-up
         HIPCHK(hipEventRecord(a, st_));
         for (int r = 0; r < reps; r++)
-            pairSetup<T>(lanes, fused, pTD_.as<T4>());
+            pairSetup<T>(lanes, fused, fieldOtf_, pTD_.as<T4>());
         HIPCHK(hipEventRecord(b, st_));
         HIPCHK(hipEventSynchronize(b));
         float ms = 0;
@@ -2950,7 +2952,7 @@ private:
         timing_ = false;
         adjointReady_ = false;   // the timed passes overwrite the evaluation's pair-pass outputs
         auto once = [&] {
-            pairSetup<T>(lanes, fused, pTD_.as<T4>());
+            pairSetup<T>(lanes, fused, otf, pTD_.as<T4>());
             for (int k = 0; k <= iterations_; k++)
                 launchPairField<T>(st_, n, pos, dTD_.as<T4>(), candStartD_.as<int>(), nbD_.as<int>(), pjD_.as<int>(),
                                    g12D_.as<T2>(), bt, tdD_.as<double>(), CgSkip{}, lanes, otf, (T) s_.beta,

@@ -170,9 +170,9 @@ constexpr int kPairLaneChoices[3] = {16, 32, 64};
 template<class T>
 void launchPairCompact(hipStream_t st, int n, const typename Vec4<T>::type* pos, const int* candStart,
                        const int* cand, int* nb, int* pj, BoxSel<T> box, T rc2, int lanes);
-// Per evaluation, over the compacted pairs: the kernels (g12: G1, G2; g03: G0, G3, stored by the FP64 path only),
-// the direct field of the charges and dipoles dip and, when dual is given, of the dipoles dual alone (the first
-// CG product).
+// Per evaluation, over the compacted pairs: the kernels (g12: G1, G2, null in FP32: not stored; g03: G0,
+// G3, FP64 only), the direct field of
+// the charges and dipoles dip and, when dual is given, of the dipoles dual alone (the first CG product).
 template<class T>
 void launchPairSetup(hipStream_t st, int n, const typename Vec4<T>::type* pos, const T* rg,
                      const typename Vec4<T>::type* dip, const typename Vec4<T>::type* dual, const int* candStart,
@@ -195,11 +195,11 @@ void launchPairField(hipStream_t st, int n, const typename Vec4<T>::type* pos, c
                      const int* candStart, const int* nb, const int* pj, const typename Vec2<T>::type* g12,
                      BoxSel<T> box, double* field, CgSkip skip, int lanes, bool otf = false, T beta = T(0),
                      bool reverse = false);
-// The CG preconditioner's short-range list: per atom, its compacted pairs within the radius (srJ partner, srG the
-// stored G1, G2; at most kPreCap, counted in srCount); *over set when an atom has more (cleared by the caller).
+// The CG preconditioner's short-range list: per atom, its compacted pairs within the radius (srJ partner, srG its
+// G1, G2; at most kPreCap, counted in srCount); *over set when an atom has more (cleared by the caller).
 template<class T>
 void launchShortList(hipStream_t st, int n, const typename Vec4<T>::type* pos, const int* candStart, const int* nb,
-                     const int* pj, const typename Vec2<T>::type* g12, BoxSel<T> box, T rpre2, int* srCount, int* srJ,
+                     const int* pj, const T* rg, T beta, BoxSel<T> box, T rpre2, int* srCount, int* srJ,
                      typename Vec2<T>::type* srG, int* over);
 // The GVDW pair term of the final pass (core/gvdw_kernel.h, combination rule; gv == nullptr: none).
 template<class T>
@@ -211,8 +211,8 @@ struct GvdwArgs {
     double* energy;                     // per sorted atom: half of its pairs' GVDW energy [kJ/mol]
 };
 
-// Energy, forces, field and (strain set) strain of the pairs at the total dipoles from the stored kernels (FP32:
-// G0, G3 rebuilt from G1, G2 with the radii rg and beta); per atom (sorted order) perAtom[n][10] = energy, strain
+// Energy, forces, field and (strain set) strain of the pairs at the total dipoles (w: the radius parameters), from
+// the stored kernels in FP64; per atom (sorted order) perAtom[n][10] = energy, strain
 // 0..8 with strain, else perAtom[n] = energy (each pair's half).
 template<class T>
 void launchPairFinal(hipStream_t st, int n, const typename Vec4<T>::type* pos, const typename Vec4<T>::type* dip,

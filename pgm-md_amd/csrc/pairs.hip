@@ -1,11 +1,11 @@
 // Real-space pGM pair passes over the full neighbour lists, one group of L = 16 lanes per atom, no atomics:
 //   setup  once per evaluation: compacts the candidates within the cutoff (a cheap pass), then evaluates G0..G3
-//          over the compacted pairs with every lane busy, stores (j, G1, G2) and (G0, G3) per pair, and returns
+//          over the compacted pairs with every lane busy, stores (j, G1, G2) and in FP64 (G0, G3) per pair, and returns
 //          the field of the charges and permanent dipoles and, dual, the first CG product T x0 (reference
 //          pairSetup / pairSetupDual, core/cuda/pgm_cuda.cu:168-219, 1110-1185);
 //   field  the dipole part of a CG matrix-vector product from the stored G1, G2 (fieldPass,
 //          core/cuda/pgm_cuda.cu:322-352);
-//   final  energy, forces, field and strain at the total dipoles from the stored G0..G3 (finalPass,
+//   final  energy, forces, field and strain at the total dipoles from G0..G3, stored or evaluated again (finalPass,
 //          core/cuda/pgm_cuda.cu:354-438; core/pgm_core.cpp:422-440).
 // The field and final passes stream the list: every lane first issues the loads of U entries (index and
 // kernels, then the partners' positions and dipoles), then computes, so U independent gathers are in flight.
@@ -22,10 +22,27 @@ namespace {
 constexpr int kPairLanes = 16;
 constexpr int kPairBlock = 256;
 
-// FP64 stores all four kernels per pair; FP32 stores G1, G2 only and rebuilds G0, G3 where they are needed
-// (g03FromG12): the setup pass writes 8 bytes per pair instead of 16, the final pass reads 12 instead of 20.
+// At most 6 of the 8 wavefronts a SIMD holds, whatever the registers would allow: the PME kernels of the other stream
+// need the rest.  A pass whose every block fits beside its like leaves them no room until it drains.  The field pass
+// alone takes 83 us at 7 wavefronts per SIMD and 86 at 6 (98,000 atoms), its product with a PME solve beside it 197 us
+// and 165 (in line: 187); per evaluation at 999,000 atoms 9.86 ms at 7, 8.62 at 6, 8.78 at 5, 9.07 at 4.
+#define PGM_PAIR_BOUNDS __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(1, 6)))
+
+// FP64 stores all four kernels per pair: reading their 32 bytes takes the final pass less than evaluating them (770 us
+// and 1,206 over 88 million pairs; storing G0 and G3 too takes the setup from 980 to 1,300).  FP32 stores G1, G2 for the field
+// passes alone, and nothing where those evaluate their own: the final pass evaluates G0..G3 as fast as it reads 8 bytes
+// and rebuilds the rest (98,000 atoms 1,225 -> 1,140 us per step, 999,000 9.95 -> 9.2 ms).
 template<class T>
-constexpr bool kStoreG03 = sizeof(T) == sizeof(double);
+constexpr bool kStoreAll = sizeof(T) == sizeof(double);
+
+// G0..G3 (n < NMAX) of a pair from rg_i + rg_j and r^2.
+template<class T, int NMAX>
+__device__ __forceinline__ void pairG(T rgSum, T beta, T r2, T* G) {
+    if constexpr (sizeof(T) == sizeof(float))
+        pairKernelsF<NMAX>(rgSum, beta, r2, G);
+    else
+        pairKernelsD<NMAX>(rgSum, beta, r2, G);
+}
 
 // The separate setup pass writes the stored kernels (FP64: 32 bytes per pair, 2.8 GB per evaluation at 96k atoms)
 // with non-temporal stores: no pass reads them again soon enough to find them in a cache, and the data written
@@ -36,9 +53,11 @@ __device__ __forceinline__ void streamStore(V* p, const V& v) {
     __builtin_nontemporal_store(v.y, &p->y);
 }
 
-// Compaction: every atom's candidates within rc, in place in its segment (pj), and the count (nb).
-template<class T, int L, bool BATCH>
-__global__ void __launch_bounds__(kPairBlock) kCompact(int n, const typename Vec4<T>::type* __restrict__ pos,
+// Compaction: every atom's candidates within rc, in place in its segment (pj), and the count (nb).  Bound by the latency
+// of index and position: U steps' loads are in flight at once (48 million candidates
+// 130 -> 107 us in FP32, 140 million 447 -> 427 in FP64).
+template<class T, int L, int U, bool BATCH>
+__global__ void PGM_PAIR_BOUNDS kCompact(int n, const typename Vec4<T>::type* __restrict__ pos,
                                                        const int* __restrict__ candStart,
                                                        const int* __restrict__ cand, int* __restrict__ nb,
                                                        int* __restrict__ pj, BoxSel<T> bs, T rc2) {
@@ -54,65 +73,40 @@ __global__ void __launch_bounds__(kPairBlock) kCompact(int n, const typename Vec
     const T4 pi = pos[s];
     const int start = candStart[s], cnt = candStart[s+1]-start;
     int kept = 0;
-    for (int base = 0; base < cnt; base += L) {
-        const int k = base+lane;
-        bool in = false;
-        int j = 0;
-        if (k < cnt) {
-            j = cand[start+k];   // the raw entry: a caller's list carries the image in it
-            const T4 pjv = pos[entryAtom(j, bs.ext)];
-            T x = pi.x-pjv.x, y = pi.y-pjv.y, z = pi.z-pjv.z;
-            pairImage(x, y, z, box, j, bs.ext);
-            in = x*x+y*y+z*z < rc2;
+    for (int base = 0; base < cnt; base += U*L) {
+        int j[U];   // the raw entries: a caller's list carries the image in them
+        T4 pjv[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = base+u*L+lane;
+            j[u] = cand[start+(k < cnt ? k : 0)];
         }
-        const unsigned long long m = (__ballot(in) >> shift) & gmask;
-        if (in)
-            pj[start+kept+__popcll(m & below)] = j;
-        kept += __popcll(m);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            pjv[u] = pos[entryAtom(j[u], bs.ext)];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            T x = pi.x-pjv[u].x, y = pi.y-pjv[u].y, z = pi.z-pjv[u].z;
+            pairImage(x, y, z, box, j[u], bs.ext);
+            const bool in = base+u*L+lane < cnt && x*x+y*y+z*z < rc2;
+            const unsigned long long m = (__ballot(in) >> shift) & gmask;
+            if (in)
+                pj[start+kept+__popcll(m & below)] = j[u];
+            kept += __popcll(m);
+        }
     }
     if (lane == 0)
         nb[s] = kept;
 }
 
-// The kernels G0..G3 of one compacted pair, the field of (q, dip) at i and, DUAL, of dual at i.
-template<class T, bool DUAL>
-__device__ __forceinline__ void setupTerm(const typename Vec4<T>::type& pi, T rgi, const typename Vec4<T>::type& pjv,
-                                          T rgj, const typename Vec4<T>::type& d, const typename Vec4<T>::type& u,
-                                          const BoxT<T>& box, int v, int ext, T beta, typename Vec2<T>::type& ga,
-                                          typename Vec2<T>::type& gb, double* e, double* f) {
-    T x = pi.x-pjv.x, y = pi.y-pjv.y, z = pi.z-pjv.z;
-    pairImage(x, y, z, box, v, ext);
-    T G[4];
-    if constexpr (sizeof(T) == sizeof(float))
-        pairKernelsF<4>(rgi+rgj, beta, x*x+y*y+z*z, G);
-    else
-        pairKernelsD<4>(rgi+rgj, beta, x*x+y*y+z*z, G);
-    const T c = pjv.w*G[1]+(d.x*x+d.y*y+d.z*z)*G[2];
-    e[0] += (double) (c*x-d.x*G[1]);
-    e[1] += (double) (c*y-d.y*G[1]);
-    e[2] += (double) (c*z-d.z*G[1]);
-    if (DUAL) {
-        const T c2 = (u.x*x+u.y*y+u.z*z)*G[2];
-        f[0] += (double) (c2*x-u.x*G[1]);
-        f[1] += (double) (c2*y-u.y*G[1]);
-        f[2] += (double) (c2*z-u.z*G[1]);
-    }
-    ga.x = G[1];
-    ga.y = G[2];
-    gb.x = G[0];
-    gb.y = G[3];
-}
-
-// setupTerm from the displacement x = r_i - r_j (the pair's image) and the partner's charge.
+// The kernels G1, G2 (FP64: and G0, G3) of one compacted pair, the field of (q, dip) at i and, DUAL, of dual at i, from the displacement
+// x = r_i - r_j (the pair's image) and the partner's charge.
 template<class T, bool DUAL>
 __device__ __forceinline__ void setupTermX(T x, T y, T z, T qj, T rgSum, const typename Vec4<T>::type& d,
                                            const typename Vec4<T>::type& u, T beta, typename Vec2<T>::type& ga,
                                            typename Vec2<T>::type& gb, double* e, double* f) {
     T G[4];
-    if constexpr (sizeof(T) == sizeof(float))
-        pairKernelsF<4>(rgSum, beta, x*x+y*y+z*z, G);
-    else
-        pairKernelsD<4>(rgSum, beta, x*x+y*y+z*z, G);
+    pairG<T, kStoreAll<T> ? 4 : 3>(rgSum, beta, x*x+y*y+z*z, G);
     const T c = qj*G[1]+(d.x*x+d.y*y+d.z*z)*G[2];
     e[0] += (double) (c*x-d.x*G[1]);
     e[1] += (double) (c*y-d.y*G[1]);
@@ -125,8 +119,21 @@ __device__ __forceinline__ void setupTermX(T x, T y, T z, T qj, T rgSum, const t
     }
     ga.x = G[1];
     ga.y = G[2];
-    gb.x = G[0];
-    gb.y = G[3];
+    if (kStoreAll<T>) {
+        gb.x = G[0];
+        gb.y = G[3];
+    }
+}
+
+// setupTermX from the positions.
+template<class T, bool DUAL>
+__device__ __forceinline__ void setupTerm(const typename Vec4<T>::type& pi, T rgi, const typename Vec4<T>::type& pjv,
+                                          T rgj, const typename Vec4<T>::type& d, const typename Vec4<T>::type& u,
+                                          const BoxT<T>& box, int v, int ext, T beta, typename Vec2<T>::type& ga,
+                                          typename Vec2<T>::type& gb, double* e, double* f) {
+    T x = pi.x-pjv.x, y = pi.y-pjv.y, z = pi.z-pjv.z;
+    pairImage(x, y, z, box, v, ext);
+    setupTermX<T, DUAL>(x, y, z, pjv.w, rgi+rgj, d, u, beta, ga, gb, e, f);
 }
 
 // LDS written by some lanes of a wavefront and read by others: no reordering across this point, and the
@@ -140,7 +147,7 @@ __device__ __forceinline__ void waveSync() {
 // Compaction and setup in one pass.  Each group of L lanes tests L candidates per step (one per lane) and
 // ballot-compacts those within rc, with their minimum-image displacement and charge, into its LDS buffer of 2L
 // entries; whenever a group of the wavefront has L entries buffered, every group evaluates up to L of its own
-// (kernels, fields) and writes (j, G1, G2) as contiguous entries of its atom's segment.  No compacted index list
+// (kernels, fields) and writes (j, G1, G2) as contiguous entries of its atom's segment (g12 null: j alone).  No compacted index list
 // goes through HBM, the partner positions are gathered once, and the transcendental part runs with every lane
 // busy.
 //
@@ -152,7 +159,7 @@ __device__ __forceinline__ void waveSync() {
 // instead of in a few rows spread over it.  A stash that is full leaves further ones in the stream (the order
 // is a matter of speed only; every entry is evaluated by the same code whatever its place).
 template<class T, int L, bool DUAL, bool BATCH>
-__global__ void __launch_bounds__(kPairBlock) kCompactSetup(int n, const typename Vec4<T>::type* __restrict__ pos,
+__global__ void PGM_PAIR_BOUNDS kCompactSetup(int n, const typename Vec4<T>::type* __restrict__ pos,
                                                             const T* __restrict__ rg,
                                                             const typename Vec4<T>::type* __restrict__ dip,
                                                             const typename Vec4<T>::type* __restrict__ dual,
@@ -192,8 +199,9 @@ __global__ void __launch_bounds__(kPairBlock) kCompactSetup(int n, const typenam
         T2 ga, gb;
         setupTermX<T, DUAL>(xq.x, xq.y, xq.z, xq.w, rgi+d.w, d, u, beta, ga, gb, e, f);
         pj[out] = v;
-        g12[out] = ga;
-        if (kStoreG03<T>)
+        if (g12)
+            g12[out] = ga;
+        if (kStoreAll<T>)
             g03[out] = gb;
     };
     // software pipeline: the candidate index two chunks ahead and the position one chunk ahead are in flight
@@ -294,7 +302,7 @@ __global__ void __launch_bounds__(kPairBlock) kCompactSetup(int n, const typenam
 
 // Kernels and fields over the compacted pairs: every lane busy, U entries in flight per lane.
 template<class T, int L, int U, bool DUAL, bool BATCH>
-__global__ void __launch_bounds__(kPairBlock) kPairSetup(int n, const typename Vec4<T>::type* __restrict__ pos,
+__global__ void PGM_PAIR_BOUNDS kPairSetup(int n, const typename Vec4<T>::type* __restrict__ pos,
                                                          const T* __restrict__ rg,
                                                          const typename Vec4<T>::type* __restrict__ dip,
                                                          const typename Vec4<T>::type* __restrict__ dual,
@@ -334,8 +342,9 @@ __global__ void __launch_bounds__(kPairBlock) kPairSetup(int n, const typename V
         for (int q = 0; q < U; q++) {
             T2 ga, gb;
             setupTerm<T, DUAL>(pi, rgi, pjv[q], d[q].w, d[q], u[q], box, v[q], bs.ext, beta, ga, gb, e, f);
-            streamStore(g12+start+k+q*L, ga);
-            if (kStoreG03<T>)
+            if (g12)
+                streamStore(g12+start+k+q*L, ga);
+            if (kStoreAll<T>)
                 streamStore(g03+start+k+q*L, gb);
         }
     }
@@ -345,8 +354,9 @@ __global__ void __launch_bounds__(kPairBlock) kPairSetup(int n, const typename V
         const T4 u = DUAL ? dual[j] : pos[j];
         const T4 dj = dip[j];
         setupTerm<T, DUAL>(pi, rgi, pos[j], dj.w, dj, u, box, v, bs.ext, beta, ga, gb, e, f);
-        streamStore(g12+start+k, ga);
-        if (kStoreG03<T>)
+        if (g12)
+            streamStore(g12+start+k, ga);
+        if (kStoreAll<T>)
             streamStore(g03+start+k, gb);
     }
 #pragma unroll
@@ -381,7 +391,7 @@ __device__ __forceinline__ void fieldTerm(const typename Vec4<T>::type& pi, cons
 }
 
 template<class T, int L, int U, bool BATCH>
-__global__ void __launch_bounds__(kPairBlock) kPairField(int n, const typename Vec4<T>::type* __restrict__ pos,
+__global__ void PGM_PAIR_BOUNDS kPairField(int n, const typename Vec4<T>::type* __restrict__ pos,
                                                          const typename Vec4<T>::type* __restrict__ dip,
                                                          const int* __restrict__ candStart,
                                                          const int* __restrict__ nb, const int* __restrict__ pj,
@@ -448,7 +458,7 @@ __device__ __forceinline__ float4 loadRecord(__amdgpu_buffer_rsrc_t r, int offse
 // index, position and dipole (w = its radius parameter rg_j; rg_i rides in the atom's own dipole w), G1 and G2
 // from r^2 and rg_i + rg_j (pairKernelsF, as the setup pass evaluates them).
 template<int L, int U, bool BATCH>
-__global__ void __launch_bounds__(kPairBlock) kPairFieldOtf(int n, const float4* __restrict__ pos,
+__global__ void PGM_PAIR_BOUNDS kPairFieldOtf(int n, const float4* __restrict__ pos,
                                                             const float4* __restrict__ dip,
                                                             const int* __restrict__ candStart,
                                                             const int* __restrict__ nb, const int* __restrict__ pj,
@@ -558,15 +568,10 @@ __device__ __forceinline__ void finalTerm(const typename Vec4<T>::type& pi, cons
     if (GVDW)
         gvdwTerm<T, STRAIN>(x, y, z, x*x+y*y+z*z, gvi, gvj, rgSum, gva.rvdw2, gva.slater != 0, gva.invKe, 1.0, eg,
                             acc, f);
-    const T G1 = ga.x, G2 = ga.y;
-    T G0, G3;
-    if constexpr (kStoreG03<T>) {
-        G0 = gb.x;
-        G3 = gb.y;
-        (void) beta;
-    }
-    else
-        g03FromG12(G1, G2, x*x+y*y+z*z, rgSum, beta, G0, G3);
+    T G[4] = {gb.x, ga.x, ga.y, gb.y};
+    if (!kStoreAll<T>)
+        pairG<T, 4>(rgSum, beta, x*x+y*y+z*z, G);
+    const T G0 = G[0], G1 = G[1], G2 = G[2], G3 = G[3];
     const T qi = pi.w, qj = pjv.w;
     const T dix = di.x*x+di.y*y+di.z*z, djx = dj.x*x+dj.y*y+dj.z*z, didj = di.x*dj.x+di.y*dj.y+di.z*dj.z;
     const T qd = qi*djx-qj*dix;
@@ -598,7 +603,7 @@ __device__ __forceinline__ void finalTerm(const typename Vec4<T>::type& pi, cons
 // perAtom: [n][10] (energy, strain row-major) with STRAIN, else [n] (energy), each half of the atom's pair sums;
 // GVDW: the GVDW energy per atom into gva.energy.
 template<class T, int L, int U, bool STRAIN, bool GVDW, bool BATCH>
-__global__ void __launch_bounds__(kPairBlock) kPairFinal(int n, const typename Vec4<T>::type* __restrict__ pos,
+__global__ void PGM_PAIR_BOUNDS kPairFinal(int n, const typename Vec4<T>::type* __restrict__ pos,
                                                          const typename Vec4<T>::type* __restrict__ dip,
                                                          const T* __restrict__ rg, T beta,
                                                          const int* __restrict__ candStart,
@@ -622,7 +627,7 @@ __global__ void __launch_bounds__(kPairBlock) kPairFinal(int n, const typename V
         const BoxT<T> box = selectBox<BATCH>(bs, s);
         const T4 pi = pos[s];
         const T4 di = dip[s];
-        const T rgi = (kStoreG03<T> && !GVDW) ? T(0) : rg[s];
+        const T rgi = (kStoreAll<T> && !GVDW) ? T(0) : rg[s];
         const T4 gvi = GVDW ? gva.gv[s] : di;
         const int start = candStart[s], cnt = nb[s];
         // FP32: the partner gathers through buffer resources (as in kPairFieldOtf); unused for FP64
@@ -643,21 +648,20 @@ __global__ void __launch_bounds__(kPairBlock) kPairFinal(int n, const typename V
         int k = lane;
         for (; k+(U-1)*L < cnt; k += U*L) {
             int v[U], j[U];
-            T2 ga[U], gb[U];
             T4 pjv[U], dj[U], gvj[U];
-            T rgj[U];
+            T2 ga[U], gb[U];   // FP64 only
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 v[u] = pj[start+k+u*L];
                 j[u] = entryAtom(v[u], bs.ext);
-                ga[u] = g12[start+k+u*L];
-                if (kStoreG03<T>)
+                if (kStoreAll<T>) {
+                    ga[u] = g12[start+k+u*L];
                     gb[u] = g03[start+k+u*L];
+                }
             }
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 gather(j[u], pjv[u], dj[u]);
-                rgj[u] = (kStoreG03<T> && !GVDW) ? T(0) : dj[u].w;
                 gvj[u] = GVDW ? gva.gv[j[u]] : dj[u];
             }
             // the U entries of a step summed in T (FP32: one FP64 addition per step instead of per entry), the
@@ -665,8 +669,8 @@ __global__ void __launch_bounds__(kPairBlock) kPairFinal(int n, const typename V
             T fu[3] = {-T(0), -T(0), -T(0)}, eu[3] = {-T(0), -T(0), -T(0)}, uu = -T(0);   // -0: folds away
 #pragma unroll
             for (int u = 0; u < U; u++)
-                finalTerm<T, STRAIN, GVDW>(pi, di, pjv[u], dj[u], ga[u], gb[u], rgi+rgj[u], beta, box, v[u], bs.ext,
-                                           acc, fu, eu, uu, gvi, gvj[u], gva, eg);
+                finalTerm<T, STRAIN, GVDW>(pi, di, pjv[u], dj[u], ga[u], gb[u], rgi+dj[u].w, beta, box, v[u], bs.ext, acc,
+                                           fu, eu, uu, gvi, gvj[u], gva, eg);
             acc[0] += (double) uu;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
@@ -676,14 +680,16 @@ __global__ void __launch_bounds__(kPairBlock) kPairFinal(int n, const typename V
         }
         for (; k < cnt; k += L) {
             const int v = pj[start+k], j = entryAtom(v, bs.ext);
-            T2 gb{};
-            if (kStoreG03<T>)
-                gb = g03[start+k];
             T4 pjr, dj;
+            T2 ga{}, gb{};
+            if (kStoreAll<T>) {
+                ga = g12[start+k];
+                gb = g03[start+k];
+            }
             gather(j, pjr, dj);
             const T4 gvj = GVDW ? gva.gv[j] : dj;
-            finalTerm<T, STRAIN, GVDW>(pi, di, pjr, dj, g12[start+k], gb, (kStoreG03<T> && !GVDW) ? T(0) : rgi+dj.w,
-                                       beta, box, v, bs.ext, acc, f, e, acc[0], gvi, gvj, gva, eg);
+            finalTerm<T, STRAIN, GVDW>(pi, di, pjr, dj, ga, gb, rgi+dj.w, beta, box, v, bs.ext, acc, f, e, acc[0], gvi,
+                                       gvj, gva, eg);
         }
 #pragma unroll
         for (int c = 0; c < 3; c++) {
@@ -764,7 +770,7 @@ __global__ void kGvdwSkip(int n, const int* __restrict__ order, const int* __res
 // with U_ij = q_i q_j G0 + (q_i d_j.x - q_j d_i.x + d_i.d_j) G1 - (d_i.x)(d_j.x) G2 and
 // dG_n/da = (2/sqrt(pi)) (2 a^2)^n exp(-a^2 r^2), the a-derivative of B_n[erf(a r)/r] (the beta part of G_n does
 // not depend on a; beyond the damping cut the a part is dropped, and its derivative with it).  The tangents use
-// dG_n = -(x . x') G_{n+1}, so G0..G3 stored by the setup pass cover phi' and E'.
+// dG_n = -(x . x') G_{n+1}, so G0..G3 cover phi' and E'.  dip.w is the partner's rg.
 template<class T, int L, bool TAN, bool BATCH>
 __global__ void __launch_bounds__(kPairBlock) kPairTangent(int n, const typename Vec4<T>::type* __restrict__ pos,
                                                            const T* __restrict__ rg, T beta,
@@ -797,20 +803,22 @@ __global__ void __launch_bounds__(kPairBlock) kPairTangent(int n, const typename
     double acc[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     for (int k = lane; k < cnt; k += L) {
         const int ent = pj[start+k], j = entryAtom(ent, bs.ext);
-        const T2 ga = g12[start+k];
-        const T G1 = ga.x, G2 = ga.y;
         const T4 pjv = pos[j];
         const T4 dj = dip[j];
         T x = pi.x-pjv.x, y = pi.y-pjv.y, z = pi.z-pjv.z;
         pairImage(x, y, z, box, ent, bs.ext);
-        T G0, G3;
-        if constexpr (kStoreG03<T>) {
-            const T2 gb = g03[start+k];
-            G0 = gb.x;
-            G3 = gb.y;
+        const T r2 = x*x+y*y+z*z, rgSum = rgi+dj.w;
+        T G[4];
+        if constexpr (kStoreAll<T>) {
+            const T2 ga = g12[start+k], gb = g03[start+k];
+            G[0] = gb.x;
+            G[1] = ga.x;
+            G[2] = ga.y;
+            G[3] = gb.y;
         }
         else
-            g03FromG12(G1, G2, x*x+y*y+z*z, rgi+rg[j], beta, G0, G3);
+            pairG<T, 4>(rgSum, beta, r2, G);
+        const T G0 = G[0], G1 = G[1], G2 = G[2], G3 = G[3];
         const T qj = pjv.w, qi = pi.w;
         const T djx = dj.x*x+dj.y*y+dj.z*z, dix = di.x*x+di.y*y+di.z*z, didj = di.x*dj.x+di.y*dj.y+di.z*dj.z;
         acc[0] += (double) (qj*G0+djx*G1);
@@ -818,15 +826,14 @@ __global__ void __launch_bounds__(kPairBlock) kPairTangent(int n, const typename
         acc[1] += (double) (c*x-dj.x*G1);
         acc[2] += (double) (c*y-dj.y*G1);
         acc[3] += (double) (c*z-dj.z*G1);
-        const T r2 = x*x+y*y+z*z;
-        const T a = rsqrtT(rgi+rg[j]);
+        const T a = rsqT(rgSum);
         const T a2 = a*a;
-        const bool damp = a*sqrt(r2) < PairPrec<T>::kDampCut;
+        const bool damp = a2*r2 < PairPrec<T>::kDampCut*PairPrec<T>::kDampCut;
         T e0 = 0, e1 = 0, e2 = 0;
         const T w = T(-2)*Ri*a*a2;
         const T mixed = qi*djx-qj*dix+didj;
         if (damp) {
-            e0 = T(kTwoOverSqrtPi)*expT(-a2*r2);
+            e0 = T(kTwoOverSqrtPi)*expNegT(a2*r2);
             e1 = T(2)*a2*e0;
             e2 = T(2)*a2*e1;
             acc[4] += (double) ((qi*qj*e0+mixed*e1-dix*djx*e2)*w);
@@ -882,11 +889,11 @@ template<class T, bool BATCH>
 __global__ void __launch_bounds__(kPairBlock) kShortList(int n, const typename Vec4<T>::type* __restrict__ pos,
                                                          const int* __restrict__ candStart,
                                                          const int* __restrict__ nb, const int* __restrict__ pj,
-                                                         const typename Vec2<T>::type* __restrict__ g12,
-                                                         BoxSel<T> bs, T rpre2, int* __restrict__ srCount,
-                                                         int* __restrict__ srJ,
+                                                         const T* __restrict__ rg, T beta, BoxSel<T> bs, T rpre2,
+                                                         int* __restrict__ srCount, int* __restrict__ srJ,
                                                          typename Vec2<T>::type* __restrict__ srG, int* over) {
     typedef typename Vec4<T>::type T4;
+    typedef typename Vec2<T>::type T2;
     const int gid = blockIdx.x*blockDim.x+threadIdx.x;
     const int s = gid/64, lane = gid%64;
     if (s >= n)   // uniform per wavefront (64 lanes per atom, blocks of whole wavefronts)
@@ -900,19 +907,26 @@ __global__ void __launch_bounds__(kPairBlock) kShortList(int n, const typename V
         const int k = k0+lane;
         bool in = false;
         int j = 0;
+        T r2 = 0;
         if (k < cnt) {
             j = pj[start+k];   // the raw entry, kept as is (the preconditioner decodes it)
             const T4 pjv = pos[entryAtom(j, bs.ext)];
             T x = pi.x-pjv.x, y = pi.y-pjv.y, z = pi.z-pjv.z;
             pairImage(x, y, z, box, j, bs.ext);
-            in = x*x+y*y+z*z < rpre2;
+            r2 = x*x+y*y+z*z;
+            in = r2 < rpre2;
         }
         const unsigned long long m = __ballot(in);
         if (in) {
             const int q = kept+__popcll(m & below);
             if (q < kPreCap) {
                 srJ[(size_t) s*kPreCap+q] = j;
-                srG[(size_t) s*kPreCap+q] = g12[start+k];
+                T G[3];
+                pairG<T, 3>(rg[s]+rg[entryAtom(j, bs.ext)], beta, r2, G);
+                T2 g;
+                g.x = G[1];
+                g.y = G[2];
+                srG[(size_t) s*kPreCap+q] = g;
             }
         }
         kept += __popcll(m);
@@ -956,7 +970,7 @@ template<class T>
 void launchPairCompact(hipStream_t st, int n, const typename Vec4<T>::type* pos, const int* candStart,
                        const int* cand, int* nb, int* pj, BoxSel<T> box, T rc2, int lanes) {
     dispatchLanes(lanes, box.table != nullptr, [&](auto L, auto B) {
-        kCompact<T, L(), B()><<<groupsBlocks(n, L()), kPairBlock, 0, st>>>(n, pos, candStart, cand, nb, pj, box, rc2);
+        kCompact<T, L(), 4, B()><<<groupsBlocks(n, L()), kPairBlock, 0, st>>>(n, pos, candStart, cand, nb, pj, box, rc2);
     });
 }
 
@@ -1072,20 +1086,20 @@ void launchPairTangent(hipStream_t st, int n, const typename Vec4<T>::type* pos,
 
 template<class T>
 void launchShortList(hipStream_t st, int n, const typename Vec4<T>::type* pos, const int* candStart, const int* nb,
-                     const int* pj, const typename Vec2<T>::type* g12, BoxSel<T> box, T rpre2, int* srCount, int* srJ,
+                     const int* pj, const T* rg, T beta, BoxSel<T> box, T rpre2, int* srCount, int* srJ,
                      typename Vec2<T>::type* srG, int* over) {
     const int blocks = groupsBlocks(n, 64);
     if (box.table != nullptr)
-        kShortList<T, true><<<blocks, kPairBlock, 0, st>>>(n, pos, candStart, nb, pj, g12, box, rpre2, srCount, srJ,
+        kShortList<T, true><<<blocks, kPairBlock, 0, st>>>(n, pos, candStart, nb, pj, rg, beta, box, rpre2, srCount, srJ,
                                                           srG, over);
     else
-        kShortList<T, false><<<blocks, kPairBlock, 0, st>>>(n, pos, candStart, nb, pj, g12, box, rpre2, srCount, srJ,
+        kShortList<T, false><<<blocks, kPairBlock, 0, st>>>(n, pos, candStart, nb, pj, rg, beta, box, rpre2, srCount, srJ,
                                                            srG, over);
 }
 
 #define PGM_INSTANTIATE_PAIRS(T)                                                                                      \
     template void launchShortList<T>(hipStream_t, int, const Vec4<T>::type*, const int*, const int*, const int*,     \
-                                     const Vec2<T>::type*, BoxSel<T>, T, int*, int*, Vec2<T>::type*, int*);          \
+                                     const T*, T, BoxSel<T>, T, int*, int*, Vec2<T>::type*, int*);                    \
     template void launchPairCompact<T>(hipStream_t, int, const Vec4<T>::type*, const int*, const int*, int*, int*,   \
                                        BoxSel<T>, T, int);                                                            \
     template void launchPairSetup<T>(hipStream_t, int, const Vec4<T>::type*, const T*, const Vec4<T>::type*,         \
