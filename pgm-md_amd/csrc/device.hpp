@@ -41,12 +41,14 @@ __device__ __forceinline__ void minImage(T& x, T& y, T& z, const BoxT<T>& b) {
 // over spatially sorted atoms gather their partners from one slab of the system per L2 instead of from all of
 // it.  A bijection of [0, gridDim.x) for any grid size.  reverse: each XCD walks its range from the end (the
 // part of the data that the pass before, walking forward, touched last comes first).
-__device__ __forceinline__ int xcdBlock(bool reverse = false) {
+__device__ __forceinline__ int xcdBlock(int b, int nb, bool reverse) {
     constexpr int kXcd = 8;
-    const int nb = (int) gridDim.x, b = (int) blockIdx.x;
     const int per = nb/kXcd, rem = nb%kXcd, x = b%kXcd, local = b/kXcd;
     const int l = reverse ? (x < rem ? per : per-1)-local : local;
     return x < rem ? x*(per+1)+l : rem*(per+1)+(x-rem)*per+l;
+}
+__device__ __forceinline__ int xcdBlock(bool reverse = false) {
+    return xcdBlock((int) blockIdx.x, (int) gridDim.x, reverse);
 }
 
 // Precision traits of the pair kernels: series length below a r = 1 and the damping cut beyond which the

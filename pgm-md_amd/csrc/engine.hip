@@ -1793,7 +1793,7 @@ private:
     // 512 planes or more (a batch) the chip is full: the 64-snapshot batch 17.6 -> 16.8 ms.  With fewer, as long as a
     // plane's atoms do not outweigh the launches saved: in mixed precision 1,536 atoms on 32^3 (288 atom rows per
     // plane) 712 -> 600 us, 24,000 on 70^3 (2,057) 730 -> 685, 96,000 on 72^3 (8,000) 2,020 -> 2,600; in FP64 30,000
-    // on 75 x 80 x 72 (2,400) 1,370 -> 1,398.
+    // on 75 x 80 x 72 (2,400) 1,250 -> 1,174 with the field pass beside the planes (pairBesidePlanes).
     bool planePath() const {
         size_t lds = 0;
         long long planes = 0;
@@ -1811,7 +1811,7 @@ private:
         }
         if (lds > kPlaneLds)
             return false;
-        const long long most = s_.precision == PGM_MIXED ? 2200 : 1500;   // atom rows per plane
+        const long long most = s_.precision == PGM_MIXED ? 2200 : 2600;   // atom rows per plane
         return planes >= kManyPlanes || (long long) n_*s_.order <= most*planes;
     }
     static constexpr int kManyPlanes = 512;
@@ -1941,7 +1941,7 @@ private:
         fftL_.plane = plane ? 1 : 0;
         fftL_.zyFused = (plane || (fftL_.blocks[3] >= 512 && fftL_.lds[3] <= 48*1024)) ? 1 : 0;
         // (few planes: as many wavefronts per plane as a workgroup holds; many: several workgroups per CU)
-        fftL_.planeThreads = plane && fftL_.blocks[3] < kManyPlanes ? 1024 : 256;
+        fftL_.planeThreads = plane && fftL_.blocks[3] < kManyPlanes ? kPlaneThreads : 256;
         upload(fftGroupsD_, fg.data(), fg.size()*sizeof(FftGroup));
         fftL_.groups = fftGroupsD_.as<FftGroup>();
         fftL_.ngroups = (int) fg.size();
@@ -2376,19 +2376,19 @@ private:
     }
     // The x-plane passes (fftL_.plane): the densities of the solves spread and transformed in z and y.
     template<class T>
-    void planeSpread(PlaneSolves<T>& solves, CgSkip skip, int it) {
+    void planeSpread(PlaneSolves<T>& solves, CgSkip skip, int it, const PairFieldArgs<T>* pair = nullptr) {
         typedef typename Vec2<T>::type T2;
         solves.cplxStride = (size_t) cplxTotal_;
         tb(kPhSpread, it);
         launchPlaneSpread<T>(pmeSt_, fftL_, pmeSel(), brickStartD_.as<int>(), pmeAtomD_.as<PmeAtom<T>>(),
-                             posT<T>(), solves, cplxD_.as<T2>(), twD_.as<T2>(), skip);
+                             posT<T>(), solves, cplxD_.as<T2>(), twD_.as<T2>(), skip, pair, lanes_);
         te();
     }
     // ... and whole solves: spread, convolution, the fields gathered.
     template<class T>
-    void planeSolve(PlaneSolves<T> solves, CgSkip skip, int it = -1) {
+    void planeSolve(PlaneSolves<T> solves, CgSkip skip, int it = -1, const PairFieldArgs<T>* pair = nullptr) {
         typedef typename Vec2<T>::type T2;
-        planeSpread<T>(solves, skip, it);
+        planeSpread<T>(solves, skip, it, pair);
         tb(kPhFft, it);
         convolve<T>(nullptr, 0, false, skip, nullptr, 0, solves.n);
         te();
@@ -2445,14 +2445,15 @@ private:
 
     template<class T>
     void pmeSolve(const typename Vec4<T>::type* dip, bool withQ, const typename Vec4<T>::type* posq, int energyMode,
-                  bool strain, double* field, double* force, CgSkip skip, int it = -1) {
+                  bool strain, double* field, double* force, CgSkip skip, int it = -1,
+                  const PairFieldArgs<T>* pair = nullptr) {
         if (fftL_.plane && !force) {
             PlaneSolves<T> one{};
             one.n = 1;
             one.dip[0] = dip;
             one.withQ[0] = withQ ? 1 : 0;
             one.out[0] = field;
-            planeSolve<T>(one, skip, it);
+            planeSolve<T>(one, skip, it, pair);
             return;
         }
         pmeGrids<T>(dip, withQ, posq, energyMode, strain, gridD_.as<T>(), skip, it);
@@ -2465,16 +2466,42 @@ private:
     template<class T>
     void matvec(const typename Vec4<T>::type* posT, const typename Vec4<T>::type* dipT, CgSkip skip,
                 int it = -1) {
+        const PairFieldArgs<T> pair = fieldArgs<T>(posT, dipT, fieldOtf_);
+        if (pairBesidePlanes()) {
+            pmeSolve<T>(dipT, false, posT, 0, false, trD_.as<double>(), nullptr, skip, it, &pair);
+            return;
+        }
         // the fork is recorded before the pair pass is enqueued (the PME stream waits for nothing later), and the
         // long pair pass is enqueued first, so the host's PME launches do not delay it
         fork();
         tb(kPhPairField, it);
-        launchPairField<T>(st_, n_, posT, dipT, candStartD_.as<int>(), nbD_.as<int>(), pjD_.as<int>(),
-                           g12D_.as<typename Vec2<T>::type>(), boxSel<T>(), tdD_.as<double>(), skip, lanes_, fieldOtf_,
-                           (T) s_.beta, nextListDirection());
+        launchPairField<T>(st_, pair, lanes_, skip);
         te();
         pmeSolve<T>(dipT, false, posT, 0, false, trD_.as<double>(), nullptr, skip, it);
         join();
+    }
+    template<class T>
+    PairFieldArgs<T> fieldArgs(const typename Vec4<T>::type* posT, const typename Vec4<T>::type* dipT, bool otf) {
+        PairFieldArgs<T> a{};
+        a.n = n_;
+        a.pos = posT;
+        a.dip = dipT;
+        a.candStart = candStartD_.as<int>();
+        a.nb = nbD_.as<int>();
+        a.pj = pjD_.as<int>();
+        a.g12 = g12D_.as<typename Vec2<T>::type>();
+        a.bs = boxSel<T>();
+        a.field = tdD_.as<double>();
+        a.otf = otf;
+        a.beta = (T) s_.beta;
+        a.reverse = nextListDirection();
+        return a;
+    }
+    // The field pass in the idle blocks of the x-plane spread: one system whose planes leave CUs free (1,024 threads per
+    // plane: fewer than 512 of them), the solve in line, no phases being timed (they bracket the two apart).  A CG product
+    // of 12,000 atoms takes 51 us so, 62 with the two in line, 89 on two streams.
+    bool pairBesidePlanes() const {
+        return fftL_.plane && fftL_.planeThreads == kPlaneThreads && !fftL_.wide && !batch_ && pmeSt_ == st_ && !timing_;
     }
 
     // How a solve ended, from its norm and residuals cg[0..1+stop] (CgSkip): the iterations it took, its last residual,
@@ -2954,9 +2981,7 @@ private:
         auto once = [&] {
             pairSetup<T>(lanes, fused, otf, pTD_.as<T4>());
             for (int k = 0; k <= iterations_; k++)
-                launchPairField<T>(st_, n, pos, dTD_.as<T4>(), candStartD_.as<int>(), nbD_.as<int>(), pjD_.as<int>(),
-                                   g12D_.as<T2>(), bt, tdD_.as<double>(), CgSkip{}, lanes, otf, (T) s_.beta,
-                                   nextListDirection());
+                launchPairField<T>(st_, fieldArgs<T>(pos, dTD_.as<T4>(), otf), lanes, CgSkip{});
             launchPairFinal<T>(st_, n, pos, dTD_.as<T4>(), rgT<T>(), (T) s_.beta, candStartD_.as<int>(),
                                nbD_.as<int>(), pjD_.as<int>(), g12D_.as<T2>(), g03D_.as<T2>(), bt,
                                fpairD_.as<double>(), edD_.as<double>(), perAtomD_.as<double>(), false,

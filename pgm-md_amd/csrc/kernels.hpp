@@ -191,10 +191,22 @@ void launchPairCompactSetup(hipStream_t st, int n, const typename Vec4<T>::type*
 // launchPairFinal): the atoms in the opposite block order (the same results; the engine alternates the
 // direction from one pass over the list to the next, so that a pass starts on what the one before touched last).
 template<class T>
-void launchPairField(hipStream_t st, int n, const typename Vec4<T>::type* pos, const typename Vec4<T>::type* dip,
-                     const int* candStart, const int* nb, const int* pj, const typename Vec2<T>::type* g12,
-                     BoxSel<T> box, double* field, CgSkip skip, int lanes, bool otf = false, T beta = T(0),
-                     bool reverse = false);
+struct PairFieldArgs {
+    int n;
+    const typename Vec4<T>::type* pos;
+    const typename Vec4<T>::type* dip;
+    const int* candStart;
+    const int* nb;
+    const int* pj;
+    const typename Vec2<T>::type* g12;
+    BoxSel<T> bs;
+    double* field;
+    bool otf;
+    T beta;
+    bool reverse;
+};
+template<class T>
+void launchPairField(hipStream_t st, const PairFieldArgs<T>& args, int lanes, CgSkip skip);
 // The CG preconditioner's short-range list: per atom, its compacted pairs within the radius (srJ partner, srG its
 // G1, G2; at most kPreCap, counted in srCount); *over set when an atom has more (cleared by the caller).
 template<class T>
@@ -404,6 +416,7 @@ struct FftGroup {
     FastDiv byK2, byKh, byZy, byZx;
     FftPlan plan[3];             // the transforms along x, y and z
 };
+constexpr int kPlaneThreads = 1024;   // most threads of a block of the x-plane passes
 struct FftLaunch {
     const FftGroup* groups;      // device table
     int ngroups;
@@ -413,7 +426,7 @@ struct FftLaunch {
     int wide;                    // the plans' radices (makePlan)
     int zyFused;                 // z and y in one pass per x-plane (many small grids), else apart
     int plane;                   // spread and gather in the x-plane passes too (kPlaneSpread, kPlaneGather)
-    int planeThreads;            // threads per block of the x-plane passes
+    int planeThreads;            // threads per block of the x-plane passes (kPlaneThreads, or fewer for many planes)
 };
 // The shape of group g's stages (lines per block) and its blocks per stage, as the transforms use them.
 template<class T>
@@ -445,10 +458,13 @@ struct PlaneSolves {
 };
 // The density of the solves spread into the x-planes and transformed in z and y into cplx; their potentials transformed
 // back and gathered (launchPmeConvolve with stages = 0 in between).
+// pair (may be null; one system, L.planeThreads = kPlaneThreads and not L.wide): the rows of launchPairField with that
+// many lanes in further blocks of the launch.
 template<class T>
 void launchPlaneSpread(hipStream_t st, const FftLaunch& L, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms,
                        const typename Vec4<T>::type* posq, const PlaneSolves<T>& solves,
-                       typename Vec2<T>::type* cplx, const typename Vec2<T>::type* tw, CgSkip skip);
+                       typename Vec2<T>::type* cplx, const typename Vec2<T>::type* tw, CgSkip skip,
+                       const PairFieldArgs<T>* pair = nullptr, int pairLanes = 0);
 template<class T>
 void launchPlaneGather(hipStream_t st, const FftLaunch& L, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms,
                        const PlaneSolves<T>& solves, typename Vec2<T>::type* cplx,

@@ -11,6 +11,7 @@
 // kernels, then the partners' positions and dipoles), then computes, so U independent gathers are in flight.
 // T = float: FP32 pair arithmetic with FP64 accumulation per lane; T = double: FP64 throughout.
 #include "kernels.hpp"
+#include "pairfield.hpp"
 
 #include <stdexcept>
 #include <type_traits>
@@ -24,7 +25,7 @@ constexpr int kPairBlock = 256;
 
 // At most 6 of the 8 wavefronts a SIMD holds, whatever the registers would allow: the PME kernels of the other stream
 // need the rest.  A pass whose every block fits beside its like leaves them no room until it drains.  The field pass
-// alone takes 83 us at 7 wavefronts per SIMD and 86 at 6 (98,000 atoms), its product with a PME solve beside it 197 us
+// alone takes 83 us at 7 wavefronts per SIMD and 84 at 6 (98,000 atoms), its product with a PME solve beside it 197 us
 // and 165 (in line: 187); per evaluation at 999,000 atoms 9.86 ms at 7, 8.62 at 6, 8.78 at 5, 9.07 at 4.
 #define PGM_PAIR_BOUNDS __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(1, 6)))
 
@@ -377,153 +378,18 @@ __global__ void PGM_PAIR_BOUNDS kPairSetup(int n, const typename Vec4<T>::type* 
     }
 }
 
-template<class T>
-__device__ __forceinline__ void fieldTerm(const typename Vec4<T>::type& pi, const typename Vec4<T>::type& pj,
-                                          const typename Vec4<T>::type& d, const typename Vec2<T>::type& g,
-                                          const BoxT<T>& box, int v, int ext, double& ex, double& ey,
-                                          double& ez) {
-    T x = pi.x-pj.x, y = pi.y-pj.y, z = pi.z-pj.z;
-    pairImage(x, y, z, box, v, ext);
-    const T c2 = (d.x*x+d.y*y+d.z*z)*g.y;
-    ex += (double) (c2*x-d.x*g.x);
-    ey += (double) (c2*y-d.y*g.x);
-    ez += (double) (c2*z-d.z*g.x);
-}
-
-template<class T, int L, int U, bool BATCH>
-__global__ void PGM_PAIR_BOUNDS kPairField(int n, const typename Vec4<T>::type* __restrict__ pos,
-                                                         const typename Vec4<T>::type* __restrict__ dip,
-                                                         const int* __restrict__ candStart,
-                                                         const int* __restrict__ nb, const int* __restrict__ pj,
-                                                         const typename Vec2<T>::type* __restrict__ g12, BoxSel<T> bs,
-                                                         double* __restrict__ field, CgSkip skip,
-                                                         bool reverse) {
-    typedef typename Vec4<T>::type T4;
-    typedef typename Vec2<T>::type T2;
+template<class T, int SH, int U, bool BATCH>
+__global__ void PGM_PAIR_BOUNDS kPairField(PairFieldArgs<T> a, CgSkip skip) {
     if (skip())
         return;
-    const int gid = xcdBlock(reverse)*blockDim.x+threadIdx.x;
-    const int s = gid/L, lane = gid%L;
-    if (s >= n)
-        return;
-    const BoxT<T> box = selectBox<BATCH>(bs, s);
-    const T4 pi = pos[s];
-    const int start = candStart[s], cnt = nb[s];
-    double ex = 0, ey = 0, ez = 0;
-    int k = lane;
-    for (; k+(U-1)*L < cnt; k += U*L) {
-        int v[U];
-        T2 g[U];
-        T4 pjv[U], d[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            v[u] = pj[start+k+u*L];
-            g[u] = g12[start+k+u*L];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int j = entryAtom(v[u], bs.ext);
-            pjv[u] = pos[j];
-            d[u] = dip[j];
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++)
-            fieldTerm<T>(pi, pjv[u], d[u], g[u], box, v[u], bs.ext, ex, ey, ez);
-    }
-    for (; k < cnt; k += L) {
-        const int v = pj[start+k], j = entryAtom(v, bs.ext);
-        fieldTerm<T>(pi, pos[j], dip[j], g12[start+k], box, v, bs.ext, ex, ey, ez);
-    }
-    ex = groupSum<L>(ex);
-    ey = groupSum<L>(ey);
-    ez = groupSum<L>(ez);
-    if (lane == 0) {
-        field[3*s] = ex;
-        field[3*s+1] = ey;
-        field[3*s+2] = ez;
-    }
+    pairFieldRow<T, U, BATCH>(xcdBlock(a.reverse)*blockDim.x+threadIdx.x, SH, a);
 }
 
-// A buffer resource over n float4 records (the gfx9 raw-buffer data word): a gather then addresses a record with
-// one 32-bit offset, the same for the position and the dipole of a partner, instead of two 64-bit addresses.  An
-// offset past the records reads zeros.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t float4Records(const float4* p, int n) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float4*>(p), (short) 0, n*(int) sizeof(float4), 0x00020000);
-}
-__device__ __forceinline__ float4 loadRecord(__amdgpu_buffer_rsrc_t r, int offset) {
-    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, offset, 0, 0));
-}
-
-// The FP32 field pass with the kernels evaluated on the fly (no stored kernels read): per entry the partner's
-// index, position and dipole (w = its radius parameter rg_j; rg_i rides in the atom's own dipole w), G1 and G2
-// from r^2 and rg_i + rg_j (pairKernelsF, as the setup pass evaluates them).
-template<int L, int U, bool BATCH>
-__global__ void PGM_PAIR_BOUNDS kPairFieldOtf(int n, const float4* __restrict__ pos,
-                                                            const float4* __restrict__ dip,
-                                                            const int* __restrict__ candStart,
-                                                            const int* __restrict__ nb, const int* __restrict__ pj,
-                                                            BoxSel<float> bs, float beta, double* __restrict__ field,
-                                                            CgSkip skip, bool reverse) {
+template<int SH, int U, bool BATCH>
+__global__ void PGM_PAIR_BOUNDS kPairFieldOtf(PairFieldArgs<float> a, CgSkip skip) {
     if (skip())
         return;
-    const int gid = xcdBlock(reverse)*blockDim.x+threadIdx.x;
-    const int s = gid/L, lane = gid%L;
-    if (s >= n)
-        return;
-    const BoxT<float> box = selectBox<BATCH>(bs, s);
-    const float4 pi = pos[s];
-    const float rgi = dip[s].w;
-    const __amdgpu_buffer_rsrc_t posR = float4Records(pos, n), dipR = float4Records(dip, n);
-    const int start = candStart[s], cnt = nb[s];
-    // the U entries of a step summed in FP32 (the matrix-vector product is FP32), the steps in FP64
-    double ex = 0, ey = 0, ez = 0;
-    auto term = [&](const float4& pjv, const float4& d, int v, float& fx, float& fy, float& fz) {
-        float x = pi.x-pjv.x, y = pi.y-pjv.y, z = pi.z-pjv.z;
-        pairImage(x, y, z, box, v, bs.ext);
-        float G[3];
-        pairKernelsF<3>(rgi+d.w, beta, x*x+y*y+z*z, G);
-        const float c2 = (d.x*x+d.y*y+d.z*z)*G[2];
-        fx = fmaf(c2, x, fmaf(-d.x, G[1], fx));
-        fy = fmaf(c2, y, fmaf(-d.y, G[1], fy));
-        fz = fmaf(c2, z, fmaf(-d.z, G[1], fz));
-    };
-    int k = lane;
-    for (; k+(U-1)*L < cnt; k += U*L) {
-        int v[U];
-        float4 pjv[U], d[U];
-#pragma unroll
-        for (int u = 0; u < U; u++)
-            v[u] = pj[start+k+u*L];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int o = entryAtom(v[u], bs.ext)*(int) sizeof(float4);
-            pjv[u] = loadRecord(posR, o);
-            d[u] = loadRecord(dipR, o);
-        }
-        float fx = -0.0f, fy = -0.0f, fz = -0.0f;   // -0: adding it is exact for every x, so it folds away
-#pragma unroll
-        for (int u = 0; u < U; u++)
-            term(pjv[u], d[u], v[u], fx, fy, fz);
-        ex += (double) fx;
-        ey += (double) fy;
-        ez += (double) fz;
-    }
-    for (; k < cnt; k += L) {
-        const int v = pj[start+k], o = entryAtom(v, bs.ext)*(int) sizeof(float4);
-        float fx = -0.0f, fy = -0.0f, fz = -0.0f;   // -0: adding it is exact for every x, so it folds away
-        term(loadRecord(posR, o), loadRecord(dipR, o), v, fx, fy, fz);
-        ex += (double) fx;
-        ey += (double) fy;
-        ez += (double) fz;
-    }
-    ex = groupSum<L>(ex);
-    ey = groupSum<L>(ey);
-    ez = groupSum<L>(ez);
-    if (lane == 0) {
-        field[3*s] = ex;
-        field[3*s+1] = ey;
-        field[3*s+2] = ez;
-    }
+    pairFieldRowOtf<U, BATCH>(xcdBlock(a.reverse)*blockDim.x+threadIdx.x, SH, a);
 }
 
 // The GVDW pair term of one visit of pair (i, j) (combination rule: A = a_i a_j, C6 = c_i c_j, B = (b_i + b_j)/2
@@ -1010,20 +876,16 @@ void launchPairCompactSetup(hipStream_t st, int n, const typename Vec4<T>::type*
 }
 
 template<class T>
-void launchPairField(hipStream_t st, int n, const typename Vec4<T>::type* pos, const typename Vec4<T>::type* dip,
-                     const int* candStart, const int* nb, const int* pj, const typename Vec2<T>::type* g12,
-                     BoxSel<T> box, double* field, CgSkip skip, int lanes, bool otf, T beta, bool reverse) {
-    dispatchLanes(lanes, box.table != nullptr, [&](auto L, auto B) {
+void launchPairField(hipStream_t st, const PairFieldArgs<T>& a, int lanes, CgSkip skip) {
+    dispatchLanes(lanes, a.bs.table != nullptr, [&](auto L, auto B) {
+        constexpr int SH = L() == 16 ? 4 : L() == 32 ? 5 : 6;
         if constexpr (sizeof(T) == sizeof(float)) {
-            if (otf) {
-                kPairFieldOtf<L(), 4, B()><<<groupsBlocks(n, L()), kPairBlock, 0, st>>>(n, pos, dip, candStart, nb,
-                                                                                       pj, box, beta, field, skip,
-                                                                                       reverse);
+            if (a.otf) {
+                kPairFieldOtf<SH, 4, B()><<<groupsBlocks(a.n, L()), kPairBlock, 0, st>>>(a, skip);
                 return;
             }
         }
-        kPairField<T, L(), 4, B()><<<groupsBlocks(n, L()), kPairBlock, 0, st>>>(n, pos, dip, candStart, nb, pj, g12,
-                                                                                box, field, skip, reverse);
+        kPairField<T, SH, 4, B()><<<groupsBlocks(a.n, L()), kPairBlock, 0, st>>>(a, skip);
     });
 }
 
@@ -1108,9 +970,7 @@ void launchShortList(hipStream_t st, int n, const typename Vec4<T>::type* pos, c
     template void launchPairCompactSetup<T>(hipStream_t, int, const Vec4<T>::type*, const T*, const Vec4<T>::type*,  \
                                             const Vec4<T>::type*, const int*, const int*, int*, int*, Vec2<T>::type*, \
                                             Vec2<T>::type*, BoxSel<T>, T, T, T, double*, double*, int);               \
-    template void launchPairField<T>(hipStream_t, int, const Vec4<T>::type*, const Vec4<T>::type*, const int*,       \
-                                     const int*, const int*, const Vec2<T>::type*, BoxSel<T>, double*, CgSkip,        \
-                                     int, bool, T, bool);                                                             \
+    template void launchPairField<T>(hipStream_t, const PairFieldArgs<T>&, int, CgSkip);                             \
     template void launchPairFinal<T>(hipStream_t, int, const Vec4<T>::type*, const Vec4<T>::type*, const T*, T,      \
                                      const int*, const int*, const int*, const Vec2<T>::type*, const Vec2<T>::type*,  \
                                      BoxSel<T>, double*, double*, double*, bool, const GvdwArgs<T>&, int, bool);      \

@@ -11,6 +11,7 @@
 //              reciprocal forces -[q grad phi + (grad grad phi) . d] (core/pgm_core.cpp:241-264, 453-487);
 //   x-planes   small and many grids: spread + z + y, and y + z + gather, one x-plane per workgroup in LDS.
 #include "kernels.hpp"
+#include "pairfield.hpp"
 
 #include <type_traits>
 
@@ -77,7 +78,6 @@ FftPlan makePlan(int K, bool wide) {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kPlaneThreads = 1024;   // most threads of a block of the x-plane passes
 constexpr int kPlaneList = 2048;      // atoms listed at a time by the x-plane spread and gather
 
 template<class T2>
@@ -1030,7 +1030,10 @@ __device__ __forceinline__ const PmeSys* planeSystem(const PmeSel& ps, const Fft
     return BATCH ? ps.table+ps.groupSys[grp.boxOff+grid] : nullptr;
 }
 
-template<class T, int P, bool BATCH, bool WIDE>
+// PAIR: the first planes blocks are that; the others run the rows of the CG field pass, which need nothing of it.  Few
+// planes leave most CUs idle, and the field pass of a small system takes less than a plane: a CG product of 8,600 atoms
+// 59 -> 49 us, of 12,000 62 -> 51, of 24,000 91 -> 78.
+template<class T, int P, bool BATCH, bool WIDE, bool PAIR>
 __global__ void __launch_bounds__(kPlaneThreads) kPlaneSpread(const FftGroup* __restrict__ groups,
                                                               const unsigned short* __restrict__ blockGroup, PmeSel ps,
                                                               const int* __restrict__ brickStart,
@@ -1039,7 +1042,8 @@ __global__ void __launch_bounds__(kPlaneThreads) kPlaneSpread(const FftGroup* __
                                                               PlaneSolves<T> solves,
                                                               typename Vec2<T>::type* __restrict__ cplxAll,
                                                               const typename Vec2<T>::type* __restrict__ twAll,
-                                                              CgSkip skip) {
+                                                              CgSkip skip, PairFieldArgs<T> pair, int planes,
+                                                              int pairSh) {
     typedef typename Vec4<T>::type T4;
     typedef typename Vec2<T>::type T2;
     constexpr int W = GridFixed<T>::words;
@@ -1047,6 +1051,19 @@ __global__ void __launch_bounds__(kPlaneThreads) kPlaneSpread(const FftGroup* __
     __shared__ __align__(16) int list[kPlaneList+4];   // and its counter: whole 16 bytes before the dynamic LDS
     if (skip())
         return;
+    if constexpr (PAIR) {
+        if ((int) blockIdx.x >= planes) {
+            const int gid = xcdBlock((int) blockIdx.x-planes, (int) gridDim.x-planes, pair.reverse)*blockDim.x+threadIdx.x;
+            if constexpr (sizeof(T) == sizeof(float)) {
+                if (pair.otf) {
+                    pairFieldRowOtf<4, BATCH>(gid, pairSh, pair);
+                    return;
+                }
+            }
+            pairFieldRow<T, 4, BATCH>(gid, pairSh, pair);
+            return;
+        }
+    }
     const FftGroup& grp = groupOf(groups, blockGroup);
     const PmeGrid& g = grp.g;
     const int K0 = g.K[0], K1 = g.K[1], K2 = g.K[2], Kh = g.K3h, KK = K1*K2;
@@ -1655,13 +1672,24 @@ void launchPmeConvolve(hipStream_t st, const FftLaunch& L, T* real, typename Vec
 template<class T>
 void launchPlaneSpread(hipStream_t st, const FftLaunch& L, PmeSel ps, const int* brickStart, const PmeAtom<T>* atoms,
                        const typename Vec4<T>::type* posq, const PlaneSolves<T>& solves,
-                       typename Vec2<T>::type* cplx, const typename Vec2<T>::type* tw, CgSkip skip) {
+                       typename Vec2<T>::type* cplx, const typename Vec2<T>::type* tw, CgSkip skip,
+                       const PairFieldArgs<T>* pair, int pairLanes) {
+    const int planes = L.blocks[3];
     dispatchOrder(ps.order, ps.table != nullptr, [&](auto P, auto B) {
-        auto go = [&](auto W) {
-            kPlaneSpread<T, P(), B(), W()><<<dim3(L.blocks[3], solves.n), L.planeThreads, L.lds[4], st>>>(
-                L.groups, L.blockGroup[3], ps, brickStart, atoms, posq, solves, cplx, tw, skip);
+        auto go = [&](auto W, auto F) {
+            const int sh = pairLanes == 16 ? 4 : pairLanes == 32 ? 5 : 6;
+            const int extra = F() ? (int) ((((long long) pair->n << sh)+L.planeThreads-1)/L.planeThreads) : 0;
+            kPlaneSpread<T, P(), B(), W(), F()><<<dim3(planes+extra, solves.n), L.planeThreads, L.lds[4], st>>>(
+                L.groups, L.blockGroup[3], ps, brickStart, atoms, posq, solves, cplx, tw, skip,
+                F() ? *pair : PairFieldArgs<T>{}, planes, sh);
         };
-        L.wide ? go(std::true_type{}) : go(std::false_type{});
+        if constexpr (!B()) {
+            if (pair) {
+                go(std::false_type{}, std::true_type{});
+                return;
+            }
+        }
+        L.wide ? go(std::true_type{}, std::false_type{}) : go(std::false_type{}, std::false_type{});
     });
 }
 
@@ -1752,7 +1780,7 @@ void launchZero(hipStream_t st, T* p, size_t count, CgSkip skip) {
                                        double*, CgSkip, long long*, size_t, int, int, size_t);                    \
     template void launchPlaneSpread<T>(hipStream_t, const FftLaunch&, PmeSel, const int*, const PmeAtom<T>*,           \
                                        const Vec4<T>::type*, const PlaneSolves<T>&, Vec2<T>::type*,         \
-                                       const Vec2<T>::type*, CgSkip);                                                 \
+                                       const Vec2<T>::type*, CgSkip, const PairFieldArgs<T>*, int);                   \
     template void launchPlaneGather<T>(hipStream_t, const FftLaunch&, PmeSel, const int*, const PmeAtom<T>*,           \
                                        const PlaneSolves<T>&, Vec2<T>::type*, const Vec2<T>::type*,         \
                                        CgSkip);                                                                        \
