@@ -212,23 +212,37 @@ __global__ void __launch_bounds__(kCgBlock) kCgAp(int n, int it, const double* a
     __shared__ double smem[kCgBlock/64][4];
     if (blockIdx.x == 0 && threadIdx.x == 0)
         cg[2+it] = 0.0;
-    if (skip())
-        return;
     double v[3] = {0, 0, 0};   // p.Ap, z.Ap, Ap.f Ap
-    for (int s = blockIdx.x*blockDim.x+threadIdx.x; s < n; s += gridDim.x*blockDim.x) {
+    auto row = [&](int s, double* q) {
         const double a = alpha[s], f = a/(1.0-a*pc.cj);
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const int k = 3*s+c;
             const double pk = p[k];
-            const double q = (a > 0 ? pk/a-(td[k]+recField(tr, s, c)+cself*pk) : 0.0);
-            ap[k] = q;
-            v[0] += pk*q;
+            q[c] = (a > 0 ? pk/a-(td[k]+recField(tr, s, c)+cself*pk) : 0.0);
+            v[0] += pk*q[c];
             if (!pc.pre) {
-                v[1] += f*r[k]*q;
-                v[2] += f*q*q;
+                v[1] += f*r[k]*q[c];
+                v[2] += f*q[c]*q[c];
             }
         }
+    };
+    // the first row before the residual is looked at: its loads and the residual's are then one round trip, not two (with
+    // kCgStep alike 1,536 atoms 434 -> 408 us per step of 4 iterations)
+    int s = blockIdx.x*blockDim.x+threadIdx.x;
+    double q[3] = {0, 0, 0};
+    if (s < n)
+        row(s, q);
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]));
+    if (skip())
+        return;
+    while (s < n) {
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            ap[3*s+c] = q[c];
+        s += gridDim.x*blockDim.x;
+        if (s < n)
+            row(s, q);
     }
     const int reg[3] = {kPpAp, kPzAp, kPfAA};
     writePartials<3>(v, reg, partials, smem, 0.0, nullptr);
@@ -242,6 +256,27 @@ __global__ void __launch_bounds__(kCgBlock) kCgStep(int n, int it, const double*
                                                     const T* rgw) {
     __shared__ double smem[kCgBlock/64][4];
     __shared__ double smem2[kCgBlock/64][2];
+    // the first row's operands before the residual and the partial sums are looked at (as kCgAp)
+    struct Row {
+        double a, x[3], r[3], p[3], ap[3];
+    } w{};
+    auto load = [&](int s) {
+        w.a = alpha[s];
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            w.x[c] = x[3*s+c];
+            w.r[c] = r[3*s+c];
+            w.p[c] = p[3*s+c];
+            w.ap[c] = ap[3*s+c];
+        }
+    };
+    int s = blockIdx.x*blockDim.x+threadIdx.x;
+    if (s < n)
+        load(s);
+    asm volatile("" : "+v"(w.a));
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+        asm volatile("" : "+v"(w.x[c]), "+v"(w.r[c]), "+v"(w.p[c]), "+v"(w.ap[c]));
     if (skip())
         return;
     const int reg[4] = {kPpAp, kPzAp, kPfAA, (it & 1) ? kPRz1 : kPRz0};
@@ -250,23 +285,25 @@ __global__ void __launch_bounds__(kCgBlock) kCgStep(int n, int it, const double*
     const double rz = sum[3], step = rz/fmax(sum[0], 1e-300);
     const double bc = -step*(sum[1]-step*sum[2])/fmax(rz, 1e-300);
     double v[1] = {0}, mx = 0;
-    for (int s = blockIdx.x*blockDim.x+threadIdx.x; s < n; s += gridDim.x*blockDim.x) {
-        const double a = alpha[s], f = a/(1.0-a*pc.cj);
+    while (s < n) {
+        const double f = w.a/(1.0-w.a*pc.cj);
         double d[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const int k = 3*s+c;
-            const double pk = p[k];
-            x[k] += step*pk;
-            const double rn = r[k]-step*ap[k];
+            x[k] = w.x[c]+step*w.p[c];
+            const double rn = w.r[c]-step*w.ap[c];
             const double zn = f*rn;
             r[k] = rn;
-            d[c] = zn+bc*pk;
+            d[c] = zn+bc*w.p[c];
             p[k] = d[c];
-            mx = fmax(mx, fabs(a*rn));
+            mx = fmax(mx, fabs(w.a*rn));
             v[0] += rn*zn;
         }
         pT[s] = pairVector<T>(d, rgw ? rgw[s] : T(0));
+        s += gridDim.x*blockDim.x;
+        if (s < n)
+            load(s);
     }
     const int out[1] = {(it & 1) ? kPRz0 : kPRz1};
     writePartials<1>(v, out, partials, smem2, mx, cg+2+it);
