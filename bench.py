@@ -42,7 +42,8 @@ TRAFFIC_FILE = os.path.join("profiles", "water96k_traffic.md")
 
 # Algorithmic HBM bytes per launch of the pair passes: per entry of the full list within the cutoff (E = 2P
 # entries) and per atom (N), s = 4 (mixed) or 8 (FP64) bytes per real.  Entry: the compacted index (4) and
-# the stored kernels (G1, G2: 2s; FP64 also G0, G3: 2s more) read or written once; compaction also reads the
+# the stored kernels (G1, G2: 2s, in FP32 by the setup and field passes alone and not where the field pass evaluates
+# its own; FP64 also G0, G3: 2s more) read or written once; compaction also reads the
 # candidate indices (4 per candidate).  Atom: its own and (once, as cache-resident partners) its neighbours'
 # position (4s), dipole (4s), radius parameter (s), list offsets and counts, and the FP64 outputs.
 PAIR_BYTES = {
@@ -50,7 +51,7 @@ PAIR_BYTES = {
     "pair_compact": {"mixed": (4, 28, 4), "double": (4, 44, 4)},
     "pair_setup": {"mixed": (12, 112, 0), "double": (36, 164, 0)},
     "pair_field": {"mixed": (12, 68, 0), "double": (20, 100, 0)},
-    "pair_final": {"mixed": (12, 176, 0), "double": (36, 212, 0)},
+    "pair_final": {"mixed": (4, 176, 0), "double": (36, 212, 0)},
 }
 # compaction fused into the setup pass: candidates in, compacted entries and kernels out, no index round trip
 PAIR_BYTES_FUSED_SETUP = {"mixed": (12, 112, 4), "double": (36, 164, 4)}
@@ -166,8 +167,10 @@ def roofline(dom, live, P, C, N, precision, lanes, fused, setup_lanes=None):
     E = 2 * P
     table = dict(PAIR_BYTES, pair_setup=PAIR_BYTES_FUSED_SETUP) if fused else PAIR_BYTES
     kernels = dict(KERNEL_OF_PHASE, pair_setup="kCompactSetup") if fused else KERNEL_OF_PHASE
-    per_launch = {ph: b[precision][0] * E + b[precision][1] * N + b[precision][2] * C for ph, b in table.items()}
-    stored = {ph: b[precision][0] * E + b[precision][2] * C for ph, b in table.items()}
+    on_the_fly = precision == "mixed" and VARIANTS["mixed"][2]
+    entry = {ph: b[precision][0] - (8 if on_the_fly and ph in ("pair_setup", "pair_field") else 0) for ph, b in table.items()}
+    per_launch = {ph: entry[ph] * E + b[precision][1] * N + b[precision][2] * C for ph, b in table.items()}
+    stored = {ph: entry[ph] * E + b[precision][2] * C for ph, b in table.items()}
     t = live["launch_avg_us"] * 1e-6
     flops = PAIR_FLOPS_PER_P[dom] * P
     achieved = flops / t / 1e12

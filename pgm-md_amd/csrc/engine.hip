@@ -1906,7 +1906,8 @@ private:
         if (groups_.size() > 65535)
             throw std::invalid_argument("pgm_hip: more than 65535 PME grid shapes");
         fftL_ = FftLaunch{};
-        // (the wide radices pay where a launch fills the chip: 216^3 1,660 -> 1,500 us per evaluation, 112^3 and 72^3 5% slower)
+        // (the wide radices pay where a launch fills the chip: 216^3 1,660 -> 1,500 us per evaluation, 112^3 and 72^3
+        // 5% slower)
         const bool wide = realTotal_ >= 4000000;
         fftL_.wide = wide ? 1 : 0;
         int boxOff = 0;

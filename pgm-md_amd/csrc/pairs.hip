@@ -30,9 +30,9 @@ constexpr int kPairBlock = 256;
 #define PGM_PAIR_BOUNDS __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(1, 6)))
 
 // FP64 stores all four kernels per pair: reading their 32 bytes takes the final pass less than evaluating them (770 us
-// and 1,206 over 88 million pairs; storing G0 and G3 too takes the setup from 980 to 1,300).  FP32 stores G1, G2 for the field
-// passes alone, and nothing where those evaluate their own: the final pass evaluates G0..G3 as fast as it reads 8 bytes
-// and rebuilds the rest (98,000 atoms 1,225 -> 1,140 us per step, 999,000 9.95 -> 9.2 ms).
+// and 1,206 over 88 million pairs; storing G0 and G3 too takes the setup from 980 to 1,300).  FP32 stores G1, G2 for
+// the field passes alone, and nothing where those evaluate their own: the final pass evaluates G0..G3 as fast as it
+// read 8 bytes and rebuilt the rest from them (98,000 atoms 1,225 -> 1,140 us per step, 999,000 9.95 -> 9.2 ms).
 template<class T>
 constexpr bool kStoreAll = sizeof(T) == sizeof(double);
 
@@ -54,9 +54,9 @@ __device__ __forceinline__ void streamStore(V* p, const V& v) {
     __builtin_nontemporal_store(v.y, &p->y);
 }
 
-// Compaction: every atom's candidates within rc, in place in its segment (pj), and the count (nb).  Bound by the latency
-// of index and position: U steps' loads are in flight at once (48 million candidates
-// 130 -> 107 us in FP32, 140 million 447 -> 427 in FP64).
+// Compaction: every atom's candidates within rc, in place in its segment (pj), and the count (nb).  Bound by the
+// latency of index and position: U steps' loads are in flight at once (48 million candidates 130 -> 107 us in FP32,
+// 140 million 447 -> 427 in FP64).
 template<class T, int L, int U, bool BATCH>
 __global__ void PGM_PAIR_BOUNDS kCompact(int n, const typename Vec4<T>::type* __restrict__ pos,
                                                        const int* __restrict__ candStart,
@@ -100,8 +100,8 @@ __global__ void PGM_PAIR_BOUNDS kCompact(int n, const typename Vec4<T>::type* __
         nb[s] = kept;
 }
 
-// The kernels G1, G2 (FP64: and G0, G3) of one compacted pair, the field of (q, dip) at i and, DUAL, of dual at i, from the displacement
-// x = r_i - r_j (the pair's image) and the partner's charge.
+// The kernels G1, G2 (FP64: and G0, G3) of one compacted pair, the field of (q, dip) at i and, DUAL, of dual at i, from
+// the displacement x = r_i - r_j (the pair's image) and the partner's charge.
 template<class T, bool DUAL>
 __device__ __forceinline__ void setupTermX(T x, T y, T z, T qj, T rgSum, const typename Vec4<T>::type& d,
                                            const typename Vec4<T>::type& u, T beta, typename Vec2<T>::type& ga,

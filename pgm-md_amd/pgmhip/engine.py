@@ -534,7 +534,7 @@ def eval_erfc_f32(x) -> np.ndarray:
 
 
 def eval_pair_kernels(precision: str, rg_sum, r2, beta: float) -> np.ndarray:
-    """(n, 6): G0..G3 of the device pair kernels, then G0, G3 as the FP32 passes rebuild them (pgm_eval_pair_kernels)."""
+    """(n, 6): G0..G3 of the device pair kernels, then G0, G3 as the final pass takes them (pgm_eval_pair_kernels)."""
     lib = load() if _lib is None else _lib
     rg_sum = np.ascontiguousarray(rg_sum, dtype=np.float64)
     r2 = np.ascontiguousarray(r2, dtype=np.float64)
