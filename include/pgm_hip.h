@@ -274,9 +274,13 @@ int pgm_set_timing_phases(pgm_engine* e, unsigned mask);
  * Numerical Recipes 2nd ed. 6.2, with v_rcp_f32 and exp).  pgm_eval_pair_kernels: out[i][0..3] = G0..G3 of a
  * pair at squared distance r2[i] with rg_i + rg_j = rg_sum[i] (a = rg_sum^-1/2) and Ewald beta, as the pair
  * passes of the given precision compute them; out[i][4..5] = G0, G3 as the final and tangent
- * passes take them (the same values).  Errors: pgm_last_error(NULL). */
+ * passes take them (the same values).  pgm_eval_grid_fixed: for an atom of atoms[i] = (charge, dipole[3] per grid
+ * unit, fractions[3] of a grid cell) whether the PME spread converts its contributions in the fast way, words[i][0],
+ * and the value v[i] converted in the general way, [1..2], and in the fast way, [3..4] (high and low word; PGM_MIXED:
+ * low words 0).  Errors: pgm_last_error(NULL). */
 int pgm_eval_erfc_f32(int n, const float* x, float* y);
 int pgm_eval_pair_kernels(int precision, int n, const double* rg_sum, const double* r2, double beta, double* out);
+int pgm_eval_grid_fixed(int precision, int n, const double* atoms, const double* v, long long* words);
 
 #ifdef __cplusplus
 }

@@ -1,5 +1,5 @@
-// Device math on host arrays, for tests: the FP32 erfc fit and the FP32 / FP64 pair kernels exactly as the
-// pair passes evaluate them, so they can be checked against the mathematics and against each other.
+// Device math on host arrays, for tests: the FP32 erfc fit, the FP32 / FP64 pair kernels and the PME grid's fixed-point
+// conversions exactly as the passes evaluate them, so they can be checked against the mathematics and each other.
 #include <string>
 
 #include "../../include/pgm_hip.h"
@@ -41,6 +41,21 @@ __global__ void kEvalPair(int n, int precision, const double* rgSum, const doubl
         o[4] = G[0];
         o[5] = G[3];
     }
+}
+
+// atoms[i] = (q, e[3], fr[3]); words[i] = the atom's fixedFits, v[i] by toFixed (hi, lo) and by toFixedFast (hi, lo).
+template<class T>
+__global__ void kEvalFixed(int n, const double* atoms, const double* v, long long* words) {
+    const int i = blockIdx.x*blockDim.x+threadIdx.x;
+    if (i >= n)
+        return;
+    T a[7];
+    for (int k = 0; k < 7; k++)
+        a[k] = (T) atoms[7*(size_t) i+k];
+    long long* o = words+5*(size_t) i;
+    o[0] = fixedFits<T>(a[0], a+1, a+4) ? 1 : 0;
+    toFixed<T>((T) v[i], o[1], o[2]);
+    toFixedFast<T>((T) v[i], o[3], o[4]);
 }
 
 // Copies in, one launch, copies out, on the current device; frees what it allocated on every path.
@@ -106,6 +121,23 @@ int pgm_eval_pair_kernels(int precision, int n, const double* rg_sum, const doub
     return pgmhip::onDevice(bytes, rg_sum, bytes, r2, 6*bytes, out, [&](void* dr, void* dq, void* dOut) {
         pgmhip::kEvalPair<<<(n+255)/256, 256>>>(n, precision, static_cast<const double*>(dr),
                                                  static_cast<const double*>(dq), beta, static_cast<double*>(dOut));
+    });
+}
+
+int pgm_eval_grid_fixed(int precision, int n, const double* atoms, const double* v, long long* words) {
+    if (n < 0 || (n > 0 && (!atoms || !v || !words)) || (precision != PGM_DOUBLE && precision != PGM_MIXED)) {
+        pgmhip::setGlobalError("pgm_hip: pgm_eval_grid_fixed needs a precision, n >= 0 and all arrays");
+        return -1;
+    }
+    if (n == 0)
+        return 0;
+    const size_t bytes = sizeof(double)*(size_t) n;
+    return pgmhip::onDevice(7*bytes, atoms, bytes, v, 5*bytes, words, [&](void* da, void* dv, void* dw) {
+        auto go = [&](auto kernel) {
+            kernel<<<(n+255)/256, 256>>>(n, static_cast<const double*>(da), static_cast<const double*>(dv),
+                                         static_cast<long long*>(dw));
+        };
+        precision == PGM_MIXED ? go(pgmhip::kEvalFixed<float>) : go(pgmhip::kEvalFixed<double>);
     });
 }
 

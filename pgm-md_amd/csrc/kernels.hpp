@@ -369,6 +369,13 @@ template<class T>
 __host__ __device__ constexpr T fixedLimit() {
     return sizeof(T) == sizeof(float) ? T(1 << 18) : T(1 << 26);
 }
+// Whether every contribution of an atom with charge q, dipole e (per grid unit) and grid fractions fr (0..1) may take
+// toFixedFast: the splines and their first derivatives are at most 1.  One sum over all they are made of, which anything
+// that is not finite fails.
+template<class T>
+__device__ __forceinline__ bool fixedFits(T q, const T* e, const T* fr) {
+    return fabs(q)+fabs(e[0])+fabs(e[1])+fabs(e[2])+(fr[0]+fr[1]+fr[2]) < fixedLimit<T>();
+}
 template<class T>
 __device__ __forceinline__ void toFixedFast(T v, long long& hi, long long& lo) {
     if constexpr (GridFixed<T>::words == 2) {

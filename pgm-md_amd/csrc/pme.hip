@@ -577,10 +577,9 @@ __global__ void __launch_bounds__(kBlock) kSpread(PmeSel ps, const int* __restri
         bsplines<T, P>(a.fr[0], t1s, u1s, v1s);
         bsplines<T, P>(a.fr[1], t2s, u2s, v2s);
         bsplines<T, P>(a.fr[2], t3, u3, v3);
-        // the splines and their first derivatives are at most 1, so one test, the same for the whole wavefront,
-        // admits every contribution to the conversion of a few instructions; anything beyond its range, or not
-        // finite, takes the general one
-        const bool fast = !TAN && __all(fabs(q)+fabs(e[0])+fabs(e[1])+fabs(e[2]) < fixedLimit<T>());
+        // one test, the same for the whole wavefront, admits every contribution to the conversion of a few
+        // instructions; anything beyond its range, or not finite, takes the general one
+        const bool fast = !TAN && __all(fixedFits<T>(q, e, a.fr));
         const int l1b = a.base[1]-lo1, l2b = a.base[2]-lo2;
         for (int j1 = lane; j1 < P; j1 += G) {
             const T t1 = pick<T, P>(t1s, j1), u1 = pick<T, P>(u1s, j1), v1 = TAN ? pick<T, P>(v1s, j1) : T(0);
@@ -1101,8 +1100,7 @@ __global__ void __launch_bounds__(kPlaneThreads) kPlaneSpread(const FftGroup* __
 #pragma unroll
         for (int c = 0; c < 3; c++)
             e[c] = d.x*rc[0][c]+d.y*rc[1][c]+d.z*rc[2][c];
-        // (the conversion of a few instructions: the splines and their first derivatives are at most 1; as kSpread)
-        const bool fast = __all(fabs(q)+fabs(e[0])+fabs(e[1])+fabs(e[2]) < fixedLimit<T>());
+        const bool fast = __all(fixedFits<T>(q, e, a.fr));   // (as kSpread)
 #pragma unroll
         for (int j2 = 0; j2 < P; j2++) {
             const T A = (q*t1+e[0]*u1)*t2[j2]+e[1]*t1*u2[j2];

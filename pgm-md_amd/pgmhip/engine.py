@@ -64,7 +64,7 @@ EXPORTS = [
     "pgm_freeze_history", "pgm_set_timing", "pgm_set_timing_phases", "pgm_get_timing", "pgm_num_pairs", "pgm_backward",
     "pgm_backward_device", "pgm_adjoint_iterations", "pgm_adjoint_residual", "pgm_set_batch", "pgm_num_systems",
     "pgm_compute_batch", "pgm_compute_batch_device", "pgm_backward_batch", "pgm_backward_batch_device",
-    "pgm_autotune", "pgm_set_lanes", "pgm_eval_erfc_f32", "pgm_eval_pair_kernels", "pgm_set_gvdw",
+    "pgm_autotune", "pgm_set_lanes", "pgm_eval_erfc_f32", "pgm_eval_pair_kernels", "pgm_eval_grid_fixed", "pgm_set_gvdw",
     "pgm_set_preconditioner", "pgm_set_candidates", "pgm_wait_device", "pgm_launch_pending", "pgm_set_field_otf",
     "pgm_field_otf", "pgm_field", "pgm_compute_device_f64_noalloc", "pgm_set_pme_overlap", "pgm_pme_overlap",
     "pgm_list_check_state",
@@ -154,6 +154,7 @@ def load(path: str = LIB_PATH) -> C.CDLL:
     lib.pgm_set_candidates.argtypes = [vp, C.c_int, vp, vp, vp, vp]
     lib.pgm_wait_device.argtypes = [vp, vp]
     lib.pgm_eval_pair_kernels.argtypes = [C.c_int, C.c_int, vp, vp, C.c_double, vp]
+    lib.pgm_eval_grid_fixed.argtypes = [C.c_int, C.c_int, vp, vp, vp]
     _ = dp
     _lib = lib
     return lib
@@ -543,6 +544,19 @@ def eval_pair_kernels(precision: str, rg_sum, r2, beta: float) -> np.ndarray:
     if lib.pgm_eval_pair_kernels(prec, len(r2), _ptr(rg_sum), _ptr(r2), float(beta), _ptr(out)) != 0:
         raise PgmError(lib.pgm_last_error(None).decode())
     return out
+
+
+def eval_grid_fixed(precision: str, atoms, v) -> np.ndarray:
+    """(n, 5): whether the PME spread converts the contributions of atoms (n, 7: charge, dipole, fractions) in the fast
+    way, then v by the general and by the fast conversion, high and low words (pgm_eval_grid_fixed)."""
+    lib = load() if _lib is None else _lib
+    atoms = np.ascontiguousarray(atoms, dtype=np.float64)
+    v = np.ascontiguousarray(v, dtype=np.float64)
+    words = np.empty((len(v), 5), dtype=np.int64)
+    prec = {"double": 0, "mixed": 1}[precision]
+    if lib.pgm_eval_grid_fixed(prec, len(v), _ptr(atoms), _ptr(v), _ptr(words)) != 0:
+        raise PgmError(lib.pgm_last_error(None).decode())
+    return words
 
 
 def total_energy(terms: dict) -> float:
