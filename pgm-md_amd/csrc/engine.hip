@@ -869,7 +869,7 @@ public:
             out.fixedScale = fixedScale;
             posPrevD_.reserve(3*sizeof(double)*n_);   // kept for the next launch's check, after this one's
             out.posKeep = posPrevD_.as<double>();
-            prevValid_ = !extList_;
+            prevValid_ = false;   // until the last kernel, which writes them, is enqueued
             const bool mixed = s_.precision == PGM_MIXED;
             mixed ? prep<float>() : prep<double>();
             asyncEval_ = true;
@@ -884,6 +884,7 @@ public:
                 asyncEval_ = asyncCg_ = false;
                 throw;
             }
+            prevValid_ = !extList_;
             const bool cgAhead = asyncCg_;
             asyncEval_ = asyncCg_ = false;
             if (!cgAhead)
