@@ -253,6 +253,11 @@ int pgm_field_otf(const pgm_engine* e);
 int pgm_set_pme_overlap(pgm_engine* e, int on);
 int pgm_pme_overlap(const pgm_engine* e);
 int pgm_pme_overlap_times(pgm_engine* e, double* ms);
+/* No counterpart in the reference: how the PME solves run for the grids and atoms of the last evaluation, a sum of
+ * PGM_PME_PLANES (spread, transforms and gather of whole x-planes in LDS; else bricks and a transform per dimension),
+ * PGM_PME_WIDE (transforms with radices up to 10) and PGM_PME_BESIDE (on a stream of their own). */
+enum { PGM_PME_PLANES = 1, PGM_PME_WIDE = 2, PGM_PME_BESIDE = 4 };
+int pgm_pme_path(const pgm_engine* e);
 
 /* No counterpart in the reference (whose engine prints host wall clocks under PGM_CUDA_TIMING,
  * core/cuda/pgm_cuda.cu:1814-1817): HIP-event timing of the kernel groups of every evaluation, for

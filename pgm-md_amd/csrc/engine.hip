@@ -1275,6 +1275,10 @@ public:
         overlapChosen_ = true;
     }
     const double* overlapTimes() const { return overlapMs_; }
+    int pmePath() const {
+        return (fftL_.plane ? PGM_PME_PLANES : 0) | (fftL_.wide ? PGM_PME_WIDE : 0) |
+               (overlapPme() ? PGM_PME_BESIDE : 0);
+    }
     bool fieldOtf() const { return fieldOtf_; }
     void setFieldOtf(bool on) {
         if (on && s_.precision != PGM_MIXED)
@@ -3467,6 +3471,7 @@ int pgm_set_pme_overlap(pgm_engine* e, int on) {
     return guarded(e, [&](DeviceEngine& g) { g.setPmeOverlap(on != 0); });
 }
 int pgm_pme_overlap(const pgm_engine* e) { return (e && e->eng) ? (e->eng->pmeOverlap() ? 1 : 0) : -1; }
+int pgm_pme_path(const pgm_engine* e) { return (e && e->eng) ? e->eng->pmePath() : -1; }
 int pgm_pme_overlap_times(pgm_engine* e, double* ms) {
     return guarded(e, [&](DeviceEngine& g) {
         if (!ms)

@@ -68,7 +68,7 @@ EXPORTS = [
     "pgm_set_preconditioner", "pgm_set_candidates", "pgm_wait_device", "pgm_launch_pending", "pgm_set_field_otf",
     "pgm_field_otf", "pgm_field", "pgm_compute_device_f64_noalloc", "pgm_set_pme_overlap", "pgm_pme_overlap",
     "pgm_list_check_state",
-    "pgm_pme_overlap_times", "pgm_setup_lanes", "pgm_set_setup_lanes",
+    "pgm_pme_overlap_times", "pgm_pme_path", "pgm_setup_lanes", "pgm_set_setup_lanes",
 ]  # fmt: skip
 PHASES = ["list", "prep", "pair_compact", "pair_setup", "pair_field", "pme_spread", "pme_fft", "pme_gather", "cg",
           "pair_final", "final"]  # fmt: skip
@@ -127,6 +127,7 @@ def load(path: str = LIB_PATH) -> C.CDLL:
     lib.pgm_set_setup_lanes.argtypes = [vp, C.c_int]
     lib.pgm_set_pme_overlap.argtypes = [vp, C.c_int]
     lib.pgm_pme_overlap.argtypes = [vp]
+    lib.pgm_pme_path.argtypes = [vp]
     lib.pgm_pme_overlap_times.argtypes = [vp, vp]
     lib.pgm_set_history.argtypes = [vp, C.c_int, vp]
     lib.pgm_freeze_history.argtypes = [vp, C.c_int]
@@ -460,6 +461,11 @@ class Engine:
 
     def pme_overlap(self) -> bool:
         return self.lib.pgm_pme_overlap(self.h) == 1
+
+    def pme_path(self) -> set:
+        """How the PME solves run since the last evaluation: a subset of {"planes", "wide", "beside"} (pgm_pme_path)."""
+        bits = self.lib.pgm_pme_path(self.h)
+        return {name for k, name in enumerate(("planes", "wide", "beside")) if bits >> k & 1}
 
     def pme_overlap_times(self) -> tuple:
         """The autotuner's ms per CG product: (PME after the field pass, PME beside it)."""
