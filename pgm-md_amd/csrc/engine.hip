@@ -1794,11 +1794,16 @@ private:
     }
 
     // Whether the PME solves run as x-plane passes (kPlaneSpread, kFftXConv, kPlaneGather): three launches a solve in
-    // place of seven, no fixed-point grid and no potentials in memory, but only as many workgroups as x-planes.  With
-    // 512 planes or more (a batch) the chip is full: the 64-snapshot batch 17.6 -> 16.8 ms.  With fewer, as long as a
-    // plane's atoms do not outweigh the launches saved: in mixed precision 1,536 atoms on 32^3 (288 atom rows per
-    // plane) 712 -> 600 us, 24,000 on 70^3 (2,057) 730 -> 685, 96,000 on 72^3 (8,000) 2,020 -> 2,600; in FP64 30,000
-    // on 75 x 80 x 72 (2,400) 1,250 -> 1,174 with the field pass beside the planes (pairBesidePlanes).
+    // place of seven, no fixed-point grid and no potentials in memory, but only as many workgroups as x-planes.  The
+    // line is the mean of a plane's atom rows (atoms x order).  Fewer than 512 planes, bricks -> planes per step (the
+    // field pass beside the planes, pairBesidePlanes; both autotuned): in mixed precision 718 -> 630 us at 2,057 rows
+    // (24,000 atoms on 70^3), 799 -> 756 at 2,400 (32,000 on 80^3), 826 -> 853 at 3,000 (40,000 on 80^3), 959 -> 931 at
+    // 3,429 (48,000 on 84^3), 1,009 -> 1,124 at 4,267 (64,000 on 90^3); in FP64 1,119 -> 1,032 at 2,400 (30,000 on 75^3),
+    // 1,223 -> 1,143 at 2,700, 1,399 -> 1,333 at 3,111, 1,898 -> 2,212 at 3,938 (42,000 on 64^3).  512 planes or more (a
+    // batch) fill the chip with bricks too, so planes of many atoms lose the launches' gain earlier in mixed precision:
+    // a fit's step 2.94 -> 2.63 ms at 307 rows (20 boxes of 1,536 atoms), 3.54 -> 3.37 at 500, 5.07 -> 5.05 at 750,
+    // 4.81 -> 4.88 at 1,069 (11 of 8,553), 12.7 -> 14.5 at 3,000 (8 of 40,000); in FP64 16.4 -> 15.4 at 2,057, 20.9 ->
+    // 19.7 at 2,880 (7 of 36,000), 48.8 -> 48.9 at 3,938.
     bool planePath() const {
         size_t lds = 0;
         long long planes = 0;
@@ -1816,8 +1821,8 @@ private:
         }
         if (lds > kPlaneLds)
             return false;
-        const long long most = s_.precision == PGM_MIXED ? 2200 : 2600;   // atom rows per plane
-        return planes >= kManyPlanes || (long long) n_*s_.order <= most*planes;
+        const long long most = s_.precision == PGM_DOUBLE ? 2600 : planes >= kManyPlanes ? 900 : 2200;
+        return (long long) n_*s_.order <= most*planes;
     }
     static constexpr int kManyPlanes = 512;
     // The brick edge with the fewest tile points (each a global addition in the spread and a load in the gather) that

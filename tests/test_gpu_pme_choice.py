@@ -3,7 +3,8 @@
 Brick passes with more atom rows per plane (atoms x order / planes) than the x-plane passes take in either precision, with
 a margin of 20%, on grids whose first dimension is at most 1.5 bricks; bricks of more than 8 points on a grid whose planes
 do not fit the LDS; x-planes of more than 64 KiB of LDS, of a grid with 512 planes (256 threads per plane), of a batch with
-more than 512, and of a batch of four million points (wide radices); stored and on-the-fly field passes mixed between an
+more than 512, and of a batch of four million points (wide radices); a batch whose 512 planes have too many atoms for
+them; stored and on-the-fly field passes mixed between an
 evaluation and its backward.  Against the FP64 oracle with the bounds of test_gpu_edge.
 """
 
@@ -89,6 +90,21 @@ def test_batch_of_four_million_points(precision):
     ]
     assert sum(np.prod(sy.settings["grid"]) for sy in systems) >= 4000000
     _batch_against_oracle(systems, precision, {"planes", "wide"})
+
+
+def test_batch_of_full_planes():
+    """512 planes of 960 atom rows: each system alone takes the x-planes, the batch of the two the bricks."""
+    st = S.base_settings(grid=(256, 20, 20), tol=1e-6, predictor=0, peek=0.0)
+    systems = [S.water_box(13660, 7.43, 24, k, 0.02, f"w{k}", dict(st)) for k in (1, 2)]
+    eng, off, pos, boxes = _batch(systems, "mixed")
+    terms, f = eng.compute_batch(pos, boxes)
+    assert "planes" not in eng.pme_path()
+    for k, sy in enumerate(systems):
+        single = E.Engine.for_system(sy, precision="mixed")
+        t, fk, _ = single.compute(sy.pos, sy.box)
+        assert "planes" in single.pme_path()
+        assert abs(E.total_energy(terms[k]) / E.total_energy(t) - 1) < 1e-6, k
+        assert rel_rms(f[off[k] : off[k + 1]], fk) < 5e-5, k
 
 
 @pytest.mark.parametrize("first", [False, True])
