@@ -246,7 +246,7 @@ int pgm_set_field_otf(pgm_engine* e, int on);
 int pgm_field_otf(const pgm_engine* e);
 /* No counterpart in the reference (whose PME solves run in line): the PME solves of an evaluation on a second
  * stream, with a hardware queue of its own, beside the pair pass they are independent of (1, the default; until
- * it is set or autotuned, engines of fewer than 16,384 atoms take 0 all the same, which is faster there), or
+ * it is set or autotuned, small systems take 0 all the same, where that is faster: pgm_pme_path says which), or
  * after it on the engine stream (0).  Results are the same bit for bit either way.  pgm_autotune times one CG
  * product (field pass + PME solve) both ways and keeps the faster; pgm_pme_overlap_times gives those two
  * timings, ms[0] after, ms[1] beside (ms per product; zeros before an autotune). */

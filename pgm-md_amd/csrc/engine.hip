@@ -46,8 +46,11 @@ constexpr size_t kBrickLds = 80*1024;         // LDS of a spread's tile: two wor
 constexpr size_t kPlaneLds = 150*1024;        // dynamic LDS an x-plane block may take (160 KiB less its static arrays)
 // The PME solves run beside the pair passes only from this size on, unless the autotuner or the caller says so: below
 // it a solve is a chain of launches of a few us each, and the two streams' waits for each other cost more than the
-// overlap gains (1,536 atoms 700 us per step beside, 590 in line; 24,000 atoms 712 and 725; 98,000 1,335 and 1,545).
-constexpr int kOverlapAtoms = 16384;
+// overlap gains.  Per step beside and in line, brick passes, mixed: 12,000 atoms 645 and 588 us, 24,000 718 and 667,
+// 40,000 861 and 854, 48,000 936 and 955; FP64: 18,000 917 and 910, 24,000 1,014 and 999, 32,000 1,186 and 1,205, 40,000
+// 1,354 and 1,435.  Where the field pass rides in the x-plane spread's launch (fieldInPlanes) in line is faster at every
+// size it has: mixed 18,000 atoms 650 and 574, 30,000 790 and 738; FP64 18,000 931 and 877, 30,000 1,266 and 1,211.
+constexpr int kOverlapAtomsMixed = 44000, kOverlapAtomsDouble = 28000;
 
 void hipCheck(hipError_t e, const char* what) {
     if (e != hipSuccess)
@@ -1439,7 +1442,7 @@ private:
     // the device's PME stream, shared by its engines (acquirePmeStream)
     hipStream_t st2_ = nullptr, pmeSt_ = nullptr;
     bool pmeOverlap_ = true;              // PME on st2_ beside the pair passes (the autotuner measures it)
-    bool overlapChosen_ = false;          // ... as the caller or the autotuner chose, else only from kOverlapAtoms on
+    bool overlapChosen_ = false;          // ... as the caller or the autotuner chose, else by size (overlapPme)
     double overlapMs_[2] = {0.0, 0.0};    // the autotuner's CG product: PME after, beside the field pass
     hipEvent_t evFork_ = nullptr, evJoin_ = nullptr;
     int n_ = 0, nGlobal_ = 0, covN_ = -1, covBuiltN_ = -1;   // covBuiltN_: the atom count of the covalent CSR
@@ -2354,7 +2357,11 @@ private:
     // PME beside the pair passes unless PME phases are being timed (their brackets are on the engine stream).
     bool overlapPme() const {
         constexpr unsigned pmeMask = (1u << kPhSpread) | (1u << kPhFft) | (1u << kPhGather);
-        return pmeOverlap_ && (overlapChosen_ || n_ >= kOverlapAtoms) && !(timing_ && (phaseMask_ & pmeMask));
+        if (timing_ && (phaseMask_ & pmeMask))
+            return false;
+        if (overlapChosen_)
+            return pmeOverlap_;
+        return !fieldInPlanes() && n_ >= (s_.precision == PGM_MIXED ? kOverlapAtomsMixed : kOverlapAtomsDouble);
     }
     // The PME stream of one evaluation, back to the engine stream when the scope ends (also on an error).
     struct PmeStreamScope {
@@ -2511,9 +2518,10 @@ private:
     // The field pass in the idle blocks of the x-plane spread: one system whose planes leave CUs free (1,024 threads per
     // plane: fewer than 512 of them), the solve in line, no phases being timed (they bracket the two apart).  A CG product
     // of 12,000 atoms takes 51 us so, 62 with the two in line, 89 on two streams.
-    bool pairBesidePlanes() const {
-        return fftL_.plane && fftL_.planeThreads == kPlaneThreads && !fftL_.wide && !batch_ && pmeSt_ == st_ && !timing_;
+    bool fieldInPlanes() const {
+        return fftL_.plane && fftL_.planeThreads == kPlaneThreads && !fftL_.wide && !batch_;
     }
+    bool pairBesidePlanes() const { return fieldInPlanes() && pmeSt_ == st_ && !timing_; }
 
     // How a solve ended, from its norm and residuals cg[0..1+stop] (CgSkip): the iterations it took, its last residual,
     // and whether it converged.

@@ -113,3 +113,17 @@ def test_launch_stale_list_and_short_solve(torch, precision, beside):
     step(jump, True)   # more iterations than the solves before
     _is(eng, beside)
     _is(ref, not beside)
+
+
+def test_default_is_in_line_where_the_field_pass_rides_in_the_planes():
+    """Until it is set or tuned: in line on the x-planes of one system, also with many atoms, and on small bricks;
+    beside for large systems on bricks."""
+    for nmol, edge, grid, planes, beside in (
+        (6000, 5.64, (72, 72, 72), True, False),
+        (6000, 5.64, (24, 72, 72), False, False),
+        (15200, 7.69, (24, 72, 72), False, True),
+    ):
+        sy = S.water_box(nmol, edge, 25, 3, 0.02, "w", S.base_settings(grid=grid, tol=1e-4))
+        eng = E.Engine.for_system(sy, precision="mixed")
+        eng.compute(sy.pos, sy.box, forces=False)
+        _is(eng, beside, planes)
