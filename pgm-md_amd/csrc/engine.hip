@@ -1915,9 +1915,7 @@ private:
         }
         // the merged transform launches: every group's share of each stage
         std::vector<FftGroup> fg;
-        std::vector<unsigned short> blockGroup[4];
-        if (groups_.size() > 65535)
-            throw std::invalid_argument("pgm_hip: more than 65535 PME grid shapes");
+        std::vector<int> blockGroup[4];
         fftL_ = FftLaunch{};
         // (the wide radices pay where a launch fills the chip: 216^3 1,660 -> 1,500 us per evaluation, 112^3 and 72^3
         // 5% slower)
@@ -1942,7 +1940,7 @@ private:
             for (int k = 0; k < 4; k++) {
                 f.blk0[k] = fftL_.blocks[k];
                 fftL_.blocks[k] += b[k];
-                blockGroup[k].insert(blockGroup[k].end(), b[k], (unsigned short) fg.size());
+                blockGroup[k].insert(blockGroup[k].end(), b[k], (int) fg.size());
             }
             for (int k = 0; k < 5; k++)
                 fftL_.lds[k] = std::max(fftL_.lds[k], l[k]);
@@ -1961,8 +1959,8 @@ private:
         fftL_.ngroups = (int) fg.size();
         if (fg.size() > 1)
             for (int k = 0; k < 4; k++) {
-                upload(blockGroupD_[k], blockGroup[k].data(), blockGroup[k].size()*sizeof(unsigned short));
-                fftL_.blockGroup[k] = blockGroupD_[k].as<unsigned short>();
+                upload(blockGroupD_[k], blockGroup[k].data(), blockGroup[k].size()*sizeof(int));
+                fftL_.blockGroup[k] = blockGroupD_[k].as<int>();
             }
         brickTotal_ = 0;
         for (Sys& y : sys_) {

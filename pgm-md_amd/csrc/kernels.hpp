@@ -427,7 +427,7 @@ constexpr int kPlaneThreads = 1024;   // most threads of a block of the x-plane 
 struct FftLaunch {
     const FftGroup* groups;      // device table
     int ngroups;
-    const unsigned short* blockGroup[4];   // the group of every block of the four launches (nullptr: one group)
+    const int* blockGroup[4];   // the group of every block of the four launches (nullptr: one group)
     int blocks[4];               // z, y, x and fused z+y launch sizes
     size_t lds[5];               // dynamic LDS of those stages and the x-plane spread (the largest shape's)
     int wide;                    // the plans' radices (makePlan)

@@ -649,7 +649,7 @@ __device__ __forceinline__ void loadTransform(typename Vec2<T>::type* tw, FftPla
 }
 
 // The group (grid shape) of this block.
-__device__ __forceinline__ const FftGroup& groupOf(const FftGroup* groups, const unsigned short* blockGroup) {
+__device__ __forceinline__ const FftGroup& groupOf(const FftGroup* groups, const int* blockGroup) {
     return groups[blockGroup ? blockGroup[blockIdx.x] : 0];
 }
 
@@ -658,7 +658,7 @@ __device__ __forceinline__ const FftGroup& groupOf(const FftGroup* groups, const
 // the next spread), else from the real grid.
 template<class T, bool INVERSE, bool WIDE>
 __global__ void __launch_bounds__(kBlock) kFftZ(const FftGroup* __restrict__ groups,
-                                                const unsigned short* __restrict__ blockGroup,
+                                                const int* __restrict__ blockGroup,
                                                 T* __restrict__ realAll, typename Vec2<T>::type* __restrict__ cplxAll,
                                                 const typename Vec2<T>::type* __restrict__ twAll, CgSkip skip,
                                                 long long* __restrict__ fixedAll, size_t fixedStride) {
@@ -771,7 +771,7 @@ __global__ void __launch_bounds__(kBlock) kFftZ(const FftGroup* __restrict__ gro
 // y: lines of K2 for fixed (x, z), a tile of consecutive z per block.
 template<class T, bool INVERSE, bool WIDE>
 __global__ void __launch_bounds__(kBlock) kFftY(const FftGroup* __restrict__ groups,
-                                                const unsigned short* __restrict__ blockGroup,
+                                                const int* __restrict__ blockGroup,
                                                 typename Vec2<T>::type* __restrict__ cplxAll,
                                                 const typename Vec2<T>::type* __restrict__ twAll, CgSkip skip) {
     typedef typename Vec2<T>::type T2;
@@ -910,7 +910,7 @@ __device__ __forceinline__ typename Vec2<T>::type* planeInverse(const PmeGrid& g
 // the other way round.  The plane goes through global memory once each way instead of twice.
 template<class T, bool INVERSE, bool WIDE>
 __global__ void __launch_bounds__(kPlaneThreads) kFftZY(const FftGroup* __restrict__ groups,
-                                                        const unsigned short* __restrict__ blockGroup,
+                                                        const int* __restrict__ blockGroup,
                                                         T* __restrict__ realAll,
                                                         typename Vec2<T>::type* __restrict__ cplxAll,
                                                         const typename Vec2<T>::type* __restrict__ twAll,
@@ -1034,7 +1034,7 @@ __device__ __forceinline__ const PmeSys* planeSystem(const PmeSel& ps, const Fft
 // 59 -> 49 us, of 12,000 62 -> 51, of 24,000 91 -> 78.
 template<class T, int P, bool BATCH, bool WIDE, bool PAIR>
 __global__ void __launch_bounds__(kPlaneThreads) kPlaneSpread(const FftGroup* __restrict__ groups,
-                                                              const unsigned short* __restrict__ blockGroup, PmeSel ps,
+                                                              const int* __restrict__ blockGroup, PmeSel ps,
                                                               const int* __restrict__ brickStart,
                                                               const PmeAtom<T>* __restrict__ atoms,
                                                               const typename Vec4<T>::type* __restrict__ posq,
@@ -1127,7 +1127,7 @@ __global__ void __launch_bounds__(kPlaneThreads) kPlaneSpread(const FftGroup* __
 // The plane's share of E = -grad phi at the atoms that reach it: out[(s P + j1) 3 + c], s the sorted atom.
 template<class T, int P, bool BATCH, bool WIDE>
 __global__ void __launch_bounds__(kPlaneThreads) kPlaneGather(const FftGroup* __restrict__ groups,
-                                                              const unsigned short* __restrict__ blockGroup, PmeSel ps,
+                                                              const int* __restrict__ blockGroup, PmeSel ps,
                                                               const int* __restrict__ brickStart,
                                                               const PmeAtom<T>* __restrict__ atoms, PlaneSolves<T> solves,
                                                               typename Vec2<T>::type* __restrict__ cplxAll,
@@ -1195,7 +1195,7 @@ __global__ void __launch_bounds__(kPlaneThreads) kPlaneGather(const FftGroup* __
 // x: forward, influence function (energy, strain), back; a tile of consecutive z for fixed y per block.
 template<class T, bool WIDE>
 __global__ void __launch_bounds__(kBlock) kFftXConv(const FftGroup* __restrict__ groups,
-                                                    const unsigned short* __restrict__ blockGroup,
+                                                    const int* __restrict__ blockGroup,
                                                     typename Vec2<T>::type* __restrict__ cplxAll,
                                                     const T* __restrict__ inflAll,
                                                     const typename Vec2<T>::type* __restrict__ twAll,
