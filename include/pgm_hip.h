@@ -85,7 +85,7 @@ int pgm_set_candidates(pgm_engine* e, int nseg, const int* seg_i, const int* seg
 /* The CG preconditioner, the reference CUDA engine's PGM_CUDA_PRECOND and PGM_CUDA_JACOBI_SELF options
  * (core/cuda/pgm_cuda.cu:1753-1760, precondK :1526-1588): radius > 0 [nm, at most the cutoff] applies the
  * short-range M = D + D T_s D, D = diag(alpha), T_s the direct-space dipole tensor of the pairs within radius
- * (from the stored pair kernels; Jacobi everywhere when an atom has more than 48 of them); radius 0 is Jacobi,
+ * (Jacobi everywhere when an atom has more than 48 of them); radius 0 is Jacobi,
  * with jacobi_self != 0 alpha/(1 - alpha c_self).  The tolerance stays on max |alpha r|; the solution is the same,
  * the iteration count changes.  Unlike the reference, which uses it only when the predicted guess rides on the
  * pair setup, it applies to every solve, the adjoint's included.  Kept across pgm_set_atoms; default Jacobi. */
@@ -275,11 +275,11 @@ int pgm_set_timing_phases(pgm_engine* e, unsigned mask);
 
 /* No counterpart in the reference: test hooks that evaluate the device's own math on host arrays (they
  * allocate, copy and synchronize on the current device; for tests, not for production loops).
- * pgm_eval_erfc_f32: y[i] = erfc(x[i]) as the FP32 pair kernels compute it (the Chebyshev fit of Press et al.,
- * Numerical Recipes 2nd ed. 6.2, with v_rcp_f32 and exp).  pgm_eval_pair_kernels: out[i][0..3] = G0..G3 of a
+ * pgm_eval_erfc_f32: y[i] = erfc(x[i]) as the FP32 pair kernels compute it (a degree-8 fit of exp(x^2) erfc(x) in
+ * 1/(1 + x/2), times exp(-x^2); 0 <= x <= 4.5).  pgm_eval_pair_kernels: out[i][0..3] = G0..G3 of a
  * pair at squared distance r2[i] with rg_i + rg_j = rg_sum[i] (a = rg_sum^-1/2) and Ewald beta, as the pair
- * passes of the given precision compute them; out[i][4..5] = G0, G3 as the final and tangent
- * passes take them (the same values).  pgm_eval_grid_fixed: for an atom of atoms[i] = (charge, dipole[3] per grid
+ * passes of the given precision compute them; out[i][4..5] = G0, G3 again, as the final and tangent passes take
+ * them.  pgm_eval_grid_fixed: for an atom of atoms[i] = (charge, dipole[3] per grid
  * unit, fractions[3] of a grid cell) whether the PME spread converts its contributions in the fast way, words[i][0],
  * and the value v[i] converted in the general way, [1..2], and in the fast way, [3..4] (high and low word; PGM_MIXED:
  * low words 0).  Errors: pgm_last_error(NULL). */

@@ -748,7 +748,7 @@ public:
             // Once the engine has solved before, the CG is enqueued ahead as a launch's is (the most iterations
             // the last 16 solves needed, one more if they varied, each skipped on the device once converged): no
             // host wait between the solve and the final stage.  The forces are added only if those iterations
-            // sufficed (the solve's device flag); a solve that needed more is evaluated again, from the same guess
+            // sufficed (by the residual words, CgSkip); a solve that needed more is evaluated again, from the same guess
             // (the history is advanced only by a complete solve), with its convergence checked on the host.
             bool ahead = polarizable_ && s_.polarizable && numRecent_ > 0;
             FinalOut out{};
@@ -833,7 +833,7 @@ public:
     // host wait.  The pair list is checked on the device and read by the completion; before the launch the host
     // predicts from the last step's displacement and largest move whether the list will hold and rebuilds it if
     // not (core/cuda/pgm_cuda.cu:1912-1928).  The CG iterations enqueued are the most that the last 16 solves
-    // needed (one more if their counts varied), each behind its device flag; the first launch of an engine (no
+    // needed (one more if their counts varied), each behind the residual before it; the first launch of an engine (no
     // such count yet), and a repeat after a solve that needed more, wait on the host between chunks of iterations
     // instead.  The forces are added to
     // the fixed-point buffer in any case; the completion says whether they are valid.

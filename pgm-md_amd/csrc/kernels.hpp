@@ -307,7 +307,7 @@ struct PmeSel {
     int order;
     int brick;
     FastDiv byTile;         // (the gather's) division by its tile's edge
-    int atomLanes;          // lanes per atom of the spread and the gather over bricks: 2 (full bricks) or 8
+    int atomLanes;          // lanes per atom of the spread and the gather over bricks: 2 (full bricks) or 4
     size_t fixedStride;     // FP64 fixed-point grids: the second words' offset (the stacked real grids' size)
 };
 

@@ -1313,7 +1313,7 @@ enum { kGatherField = 0, kGatherForce = 1, kGatherPot = 2, kGatherTan = 3 };
 // One workgroup per brick: the brick's potential with its halo is loaded into LDS in whole rows, and G lanes per atom
 // gather from there, lane g the rows j1 = g, g + G, ... of P x P points.  Gathered from memory, an atom's 36 rows of
 // 6 points touch some 40 lines, 2.4 cycles each of the CU's address path; the tile's rows are read once for all of
-// the brick's atoms.  Sums in FP64, the G lanes' in a fixed order.  Per solve, FP32: 999,000 atoms on 216^3 250 -> 96 us,
+// the brick's atoms.  Sums in FP64, the G lanes' in a fixed order.  Per solve, alone, FP32: 999,000 atoms on 216^3 250 -> 96 us,
 // 96,000 on 72^3 24 -> 16 us, 98,000 on 112^3 26 -> 19 us.
 // Field and force per sorted atom; potential and tangents as out: phi[n], E[3n] at offsets 0 and n, phi'[n], E'[3n] at
 // offsets 5n and 6n.

@@ -2,8 +2,9 @@
 //   guess       mu4 / mu3 / last-solution predictor from the history (global order) or alpha b
 //               (core/pgm_core.cpp:307-328; initialGuess, core/cuda/pgm_cuda.cu:1318-1335);
 //   CG          Jacobi-preconditioned CG with the flexible Polak-Ribiere beta, err = max|alpha r| / mean|alpha b|
-//               (core/pgm_core.cpp:330-385).  Every reduction is written as per-block partials and reduced
-//               again, identically, by every block of the consuming kernel: deterministic, no atomics;
+//               (core/pgm_core.cpp:330-385).  Every sum is written as per-block partials and added up again,
+//               identically, by every block of the consuming kernel, and the residual goes through an atomic maximum:
+//               deterministic;
 //   post        peek, history push, total dipoles (core/pgm_core.cpp:386-397, 413-416);
 //   final       total field, self/polarization sums, covalent chain rule, forces out
 //               (core/pgm_core.cpp:488-534).
