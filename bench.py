@@ -179,6 +179,9 @@ def roofline(dom, live, P, C, N, precision, lanes, fused, setup_lanes=None):
     if dom in ("pair_setup", "pair_compact") and setup_lanes:
         lanes = setup_lanes
     prefix = f"{kernels[dom]}<{real}, {lanes},"
+    if dom == "pair_field":   # named by the logarithm of its lanes, and apart where it evaluates its own kernels
+        sh = lanes.bit_length() - 1
+        prefix = f"kPairFieldOtf<{sh}," if on_the_fly else f"kPairField<{real}, {sh},"
     traffic = next((v for k, v in traffic_table().items() if k.startswith(prefix)), None)
     return {
         "bound": "valu", "kernel": f"{kernels[dom]}<{real}, {lanes}>", "phase": dom,
